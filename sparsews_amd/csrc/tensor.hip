@@ -12,15 +12,15 @@
 //                           owners and k_mttkrp_keys instead.
 //     2. radix sort         stable on the i bits only: the buckets are the
 //                           output rows, CSF (j,k) order kept inside each.
-//     3. k_mttkrp_accum     each half-wavefront (32 lanes = 32 ranks) walks a
-//                           segment of the bucketed nonzeros, loading factor
-//                           rows Bf(j,:), Cf(k,:) as coalesced 256-byte rows
+//     3. k_mttkrp_accum     each group of 16 or 32 lanes (a rank per lane)
+//                           walks a segment of the bucketed nonzeros, loading
+//                           factor rows Bf(j,:), Cf(k,:) as coalesced rows
 //                           (Bf(j,:) only when j changes: within a row the
 //                           nonzeros come in (j, k) order) and accumulating
-//                           the rank-R fiber in registers;
-//                           a fiber is added into M when its row changes (only
-//                           segment-boundary rows are shared, so the atomics
-//                           are few and uncontended).
+//                           the rank-R fiber in registers; a row inside one
+//                           segment is stored, rows over several segments of
+//                           a workgroup meet in LDS, and only rows that reach
+//                           other workgroups are added with atomics.
 //     4. k_rows_present + scan + k_rows_compact: the sorted list of rows that
 //                           hold a nonzero (the reference's COO output rows).
 //   The product is (X * Bf) * Cf, the reference's B_vals * C_vals * D_vals
@@ -200,19 +200,33 @@ __global__ __launch_bounds__(256) void k_mttkrp_keys(int64_t nnz, const int32_t*
   }
 }
 
-// Each half-wavefront owns `seg` consecutive bucketed nonzeros.  Lanes cover
-// ranks r = lane32, lane32 + 32, ... (R <= 64 supported with two slices).
-// The half-wavefront loads 32 keys and values at once (coalesced), then
-// walks them kAccU at a time: the factor rows of kAccU nonzeros are loaded
-// before any is used, so their latencies overlap; the sums still run in
-// bucket order.
+// The bucketed nonzeros in tiles of one workgroup, `seg` consecutive ones per
+// group of G lanes; the lanes cover ranks lane, lane + G, ... (S slices).
+// A group loads G keys and values at once (coalesced, the next G in flight
+// while these are used), stages them in LDS, and walks them kAccU at a time,
+// each nonzero's record one 16-byte broadcast read; the factor rows of kAccU
+// nonzeros are loaded before any is used, so their latencies overlap.  The
+// sums run in bucket order.
+//
+// A row that starts and ends inside a group's segment is stored at once: no
+// other group holds a part of it.  The segments' first and last rows meet in
+// LDS after the walk; only the tile's own first and last rows are added into
+// M with atomics, one per tile.  With one per segment of 128 the atomics of
+// the skewed rows bounded the kernel: a row of 2M nonzeros was 15,600 adds to
+// the same two lines, about 50 ns each across the XCDs.  50k x 40k x 30k,
+// 20M nonzeros, R = 32: 1,204 us with an atomic per segment and row, 518 us
+// with one per tile, 470 us with the factors' byte offsets made once per
+// nonzero by the lane that loads it (64 VGPRs, 8 wavefronts per SIMD); now
+// the gathered factor rows (about 8 GB from the L2) bound it.
 constexpr int kAccBlock = 256;
 constexpr int kAccU = 4;
+constexpr int kAccSegMax = 256;  // nonzeros per group at most
+constexpr int kAccSegMin = 32;
 
 // kMask: per row, the OR of its nonzeros' shared stored factor columns
 // (mB[j] & mC[k]) is or-ed into rmask[i], the row's stored output columns.
-template <bool kTwo, bool kMask>
-__global__ __launch_bounds__(kAccBlock) void k_mttkrp_accum(int64_t nnz, int64_t seg, const uint64_t* __restrict__ keys,
+template <int G, int S, bool kMask, bool kOff32>
+__global__ __launch_bounds__(kAccBlock, S == 1 && !kMask ? 8 : 4) void k_mttkrp_accum(int64_t nnz, int seg, const uint64_t* __restrict__ keys,
                                                             const double* __restrict__ vals, int bj, int bk, int R,
                                                             const double* __restrict__ Bf,
                                                             const double* __restrict__ Cf, double* __restrict__ M,
@@ -220,88 +234,168 @@ __global__ __launch_bounds__(kAccBlock) void k_mttkrp_accum(int64_t nnz, int64_t
                                                             const uint64_t* __restrict__ mB,
                                                             const uint64_t* __restrict__ mC,
                                                             unsigned long long* __restrict__ rmask) {
-  const int half = threadIdx.x >> 5;
-  const int r0 = threadIdx.x & 31;
-  const int64_t hid = (int64_t)blockIdx.x * (kAccBlock / 32) + half;
-  const int64_t e0 = hid * seg;
-  if (e0 >= nnz) return;  // uniform per half-wavefront
+  constexpr int NG = kAccBlock / G;
+  // a nonzero as the walk reads it: its factor rows' byte offsets (kOff32:
+  // both factors below 4 GiB) or its j and k, its value, and its row with
+  // the top bit set where j differs from the previous nonzero's
+  struct alignas(16) Rec {
+    uint32_t j, k;
+    double val;
+  };
+  __shared__ Rec recs[kAccBlock];
+  __shared__ uint32_t rows[kAccBlock];
+  // per group: its segment's first row (slot 2g) and, if another, its last
+  // (slot 2g + 1): row (-1: none) and sums
+  __shared__ int32_t brow[2 * NG];
+  __shared__ double bsum[2 * NG][S * G];
+  __shared__ uint64_t bmask[kMask ? 2 * NG : 1];
+  const int g = threadIdx.x / G;
+  const int r0 = threadIdx.x % G;
+  const int64_t e0 = ((int64_t)blockIdx.x * NG + g) * seg;
   const int64_t e1 = e0 + seg < nnz ? e0 + seg : nnz;
   const uint64_t jm = (1ull << bj) - 1, km = (1ull << bk) - 1;
-  constexpr bool two = kTwo;  // R > 32: a second slice of ranks per lane
-  const int r1 = r0 + 32;
-  const int rr0 = r0 < R ? r0 : 0, rr1 = r1 < R ? r1 : 0;  // in-range rank for the loads
-  int64_t cur = -1;
-  double acc0 = 0.0, acc1 = 0.0;
+  uint32_t rr[S];  // in-range ranks for the loads
+#pragma unroll
+  for (int q = 0; q < S; ++q) rr[q] = r0 + q * G < R ? r0 + q * G : 0;
+  const auto factor = [&](const double* __restrict__ f, uint32_t x, int q) -> double {
+    if (kOff32) return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(f) + (x + rr[q] * 8u));
+    return f[(int64_t)x * R + rr[q]];
+  };
+  int32_t cur = -1;
+  bool first = true;  // cur is the segment's first row
+  double acc[S];
+#pragma unroll
+  for (int q = 0; q < S; ++q) acc[q] = 0.0;
   uint64_t rowm = 0;
   // Bf(j,:) of the last nonzero: within a row the nonzeros come in (j, k)
   // order, so runs of equal j reuse it instead of gathering it again
-  int64_t jprev = -1;
-  double bp0 = 0.0, bp1 = 0.0;
-  for (int64_t base = e0; base < e1; base += 32) {
-    const int cnt = (int)(e1 - base < 32 ? e1 - base : 32);
-    const int64_t me = base + (r0 < cnt ? r0 : cnt - 1);
-    const uint64_t mykey = keys[me];
-    const double myval = vals[me];
+  double bp[S];
+#pragma unroll
+  for (int q = 0; q < S; ++q) bp[q] = 0.0;
+  const auto to_slot = [&](int slot) {
+#pragma unroll
+    for (int q = 0; q < S; ++q) bsum[slot][r0 + q * G] = acc[q];
+    if (r0 == 0) brow[slot] = cur;
+    if (kMask && r0 == 0) bmask[slot] = rowm;
+  };
+  const uint32_t unit = kOff32 ? (uint32_t)R * 8u : 1u;
+  uint64_t nkey = 0;
+  double nval = 0.0;
+  if (e0 + r0 < e1) {
+    nkey = keys[e0 + r0];
+    nval = vals[e0 + r0];
+  }
+  uint32_t jlast = ~0u;  // j of the last nonzero of the previous G
+  Rec* const mine = recs + g * G;
+  uint32_t* const mrow = rows + g * G;
+  for (int64_t base = e0; base < e1; base += G) {  // uniform per group
+    const int cnt = (int)(e1 - base < G ? e1 - base : G);
+    {
+      const uint32_t j = (uint32_t)((nkey >> bk) & jm);
+      const uint32_t jb = (uint32_t)__shfl_up((int)j, 1, G);
+      mine[r0].j = j * unit;
+      mine[r0].k = (uint32_t)(nkey & km) * unit;
+      mine[r0].val = nval;
+      mrow[r0] = (uint32_t)(nkey >> (bj + bk)) | (j != (r0 ? jb : jlast) ? 0x80000000u : 0u);
+      jlast = (uint32_t)__shfl((int)j, G - 1, G);
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (base + G + r0 < e1) {
+      nkey = keys[base + G + r0];
+      nval = vals[base + G + r0];
+    }
     for (int t = 0; t < cnt; t += kAccU) {
-      uint64_t kk[kAccU];
-      double xv[kAccU], b0[kAccU], c0[kAccU], b1[kAccU], c1[kAccU];
+      uint32_t rw[kAccU];
+      double xv[kAccU], bv[kAccU][S], cv[kAccU][S];
+      uint64_t mk[kAccU];
 #pragma unroll
       for (int u = 0; u < kAccU; ++u) {
-        const int src = t + u < cnt ? t + u : cnt - 1;
-        kk[u] = __shfl(mykey, src, 32);
-        xv[u] = __shfl(myval, src, 32);
-      }
-      bool nb[kAccU];  // Bf(j,:) differs from the previous nonzero's (uniform per half-wavefront)
+        const int p = t + u < cnt ? t + u : cnt - 1;
+        const Rec rec = mine[p];
+        rw[u] = mrow[p];
+        xv[u] = rec.val;
+        if ((int32_t)rw[u] < 0) {  // uniform per group
 #pragma unroll
-      for (int u = 0; u < kAccU; ++u) {
-        const int64_t j = (int64_t)((kk[u] >> bk) & jm);
-        const int64_t k = (int64_t)(kk[u] & km);
-        const int64_t jbefore = u == 0 ? jprev : (int64_t)((kk[u - 1] >> bk) & jm);
-        nb[u] = j != jbefore;
-        b0[u] = b1[u] = 0.0;
-        if (nb[u]) {
-          b0[u] = Bf[j * R + rr0];
-          if (two) b1[u] = Bf[j * R + rr1];
+          for (int q = 0; q < S; ++q) bv[u][q] = factor(Bf, rec.j, q);
         }
-        c0[u] = Cf[k * R + rr0];
-        if (two) c1[u] = Cf[k * R + rr1];
+#pragma unroll
+        for (int q = 0; q < S; ++q) cv[u][q] = factor(Cf, rec.k, q);
+        if (kMask) mk[u] = mB[rec.j / unit] & mC[rec.k / unit];
       }
-      jprev = (int64_t)((kk[kAccU - 1] >> bk) & jm);
 #pragma unroll
       for (int u = 0; u < kAccU; ++u) {
-        if (nb[u]) {
-          bp0 = b0[u];
-          if (two) bp1 = b1[u];
+        if (t + u >= cnt) break;  // uniform per group
+        const int32_t i = (int32_t)(rw[u] & 0x7FFFFFFFu);
+        if ((int32_t)rw[u] < 0) {
+#pragma unroll
+          for (int q = 0; q < S; ++q) bp[q] = bv[u][q];
         }
-        b0[u] = bp0;
-        if (two) b1[u] = bp1;
-      }
-#pragma unroll
-      for (int u = 0; u < kAccU; ++u) {
-        if (t + u >= cnt) break;  // uniform per half-wavefront
-        const int64_t i = (int64_t)(kk[u] >> (bj + bk));
         if (i != cur) {
           if (cur >= 0) {
-            if (r0 < R) atomicAdd(&M[cur * R + r0], acc0);
-            if (two && r1 < R) atomicAdd(&M[cur * R + r1], acc1);
-            if (r0 == 0) present[cur] = 1;
-            if (kMask && r0 == 0) atomicOr(&rmask[cur], (unsigned long long)rowm);
+            if (first) {
+              to_slot(2 * g);
+            } else {
+#pragma unroll
+              for (int q = 0; q < S; ++q)
+                if (r0 + q * G < R) M[(int64_t)cur * R + r0 + q * G] = acc[q];
+              if (r0 == 0) present[cur] = 1;
+              if (kMask && r0 == 0) rmask[cur] = rowm;
+            }
+            first = false;
           }
           cur = i;
-          acc0 = acc1 = 0.0;
+#pragma unroll
+          for (int q = 0; q < S; ++q) acc[q] = 0.0;
           rowm = 0;
         }
-        if (kMask) rowm |= mB[(kk[u] >> bk) & jm] & mC[kk[u] & km];
-        acc0 += (xv[u] * b0[u]) * c0[u];
-        if (two) acc1 += (xv[u] * b1[u]) * c1[u];
+        if (kMask) rowm |= mk[u];
+#pragma unroll
+        for (int q = 0; q < S; ++q) acc[q] += (xv[u] * bp[q]) * cv[u][q];
       }
     }
   }
-  if (cur >= 0) {
-    if (r0 < R) atomicAdd(&M[cur * R + r0], acc0);
-    if (two && r1 < R) atomicAdd(&M[cur * R + r1], acc1);
-    if (r0 == 0) present[cur] = 1;
-    if (kMask && r0 == 0) atomicOr(&rmask[cur], (unsigned long long)rowm);
+  // the segment's last row, and the slots that hold none
+  if (cur < 0 || first) {
+    if (r0 == 0) brow[2 * g + 1] = -1;
+    if (cur < 0 && r0 == 0) brow[2 * g] = -1;
+  }
+  if (cur >= 0) to_slot(first ? 2 * g : 2 * g + 1);
+  __syncthreads();
+  // runs of equal rows over the slots: the group owning a run's first slot
+  // sums it
+  int lo = 0, hi = 2 * NG - 1;  // the tile's first and last slots that hold a row
+  while (lo < 2 * NG && brow[lo] < 0) ++lo;
+  while (hi >= 0 && brow[hi] < 0) --hi;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int s0 = 2 * g + h;
+    const int32_t row = brow[s0];
+    if (row < 0) continue;
+    int before = s0 - 1;
+    while (before >= lo && brow[before] < 0) --before;
+    if (before >= lo && brow[before] == row) continue;
+    double sum[S];
+#pragma unroll
+    for (int q = 0; q < S; ++q) sum[q] = 0.0;
+    uint64_t msum = 0;
+    for (int s = s0; s <= hi; ++s) {
+      if (brow[s] < 0) continue;
+      if (brow[s] != row) break;
+#pragma unroll
+      for (int q = 0; q < S; ++q) sum[q] += bsum[s][r0 + q * G];
+      if (kMask) msum |= bmask[s];
+    }
+    const bool shared = row == brow[lo] || row == brow[hi];  // other tiles may hold parts of it
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+      const int r = r0 + q * G;
+      if (r < R) {
+        if (shared) atomicAdd(&M[(int64_t)row * R + r], sum[q]);
+        else M[(int64_t)row * R + r] = sum[q];
+      }
+    }
+    if (r0 == 0) present[row] = 1;
+    if (kMask && r0 == 0) atomicOr(&rmask[row], (unsigned long long)msum);
   }
 }
 
@@ -799,25 +893,35 @@ static int mttkrp_run(spws_ctx* ctx, const Csf3& x, int32_t I, int32_t J, int32_
       SPWS_HIP(hipStreamSynchronize(s));
       kept = x.nnz - *hd;
     }
-    // segments of 128 nonzeros per half-wavefront
-    const int64_t seg = 128;
-    const int64_t halves = div_up(kept, seg);
-    const unsigned ga = (unsigned)std::max<int64_t>(1, div_up(halves, kAccBlock / 32));
+    // 16 lanes per group up to rank 16; segments long enough for few atomics,
+    // short enough for 8 workgroups per CU (the 32-lane kernel's occupancy)
+    const int lanes = R <= 16 ? 16 : 32;
+    const int groups = kAccBlock / lanes;
+    int cus = 0;
+    SPWS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    const int64_t fill = kept / ((int64_t)std::max(cus, 1) * 8 * groups) / 32 * 32;
+    const int seg = (int)std::min<int64_t>(kAccSegMax, std::max<int64_t>(kAccSegMin, fill));
+    const unsigned ga = (unsigned)div_up(kept, (int64_t)seg * groups);
+    // both factors addressed with 32-bit byte offsets while they are below 4 GiB
+    const bool off32 = std::max<int64_t>(J, K) * R * 8 <= (int64_t)UINT32_MAX;
+#define SPWS_MTTKRP_ACCUM(G, S, MASK)                                                                               \
+  do {                                                                                                              \
+    if (off32)                                                                                                      \
+      SPWS_LAUNCH(ctx, "mttkrp_accum", (k_mttkrp_accum<G, S, MASK, true>), dim3(ga), dim3(kAccBlock), 0, kept, seg, \
+                  keys, vals, bj, bk, R, Bf, Cf, M, present, mB, mC, rmask);                                        \
+    else                                                                                                            \
+      SPWS_LAUNCH(ctx, "mttkrp_accum", (k_mttkrp_accum<G, S, MASK, false>), dim3(ga), dim3(kAccBlock), 0, kept,     \
+                  seg, keys, vals, bj, bk, R, Bf, Cf, M, present, mB, mC, rmask);                                   \
+  } while (0)
     if (kept > 0) {
-      if (R > 32 && masked) {
-        SPWS_LAUNCH(ctx, "mttkrp_accum", (k_mttkrp_accum<true, true>), dim3(ga), dim3(kAccBlock), 0, kept, seg, keys,
-                    vals, bj, bk, R, Bf, Cf, M, present, mB, mC, rmask);
-      } else if (R > 32) {
-        SPWS_LAUNCH(ctx, "mttkrp_accum", (k_mttkrp_accum<true, false>), dim3(ga), dim3(kAccBlock), 0, kept, seg, keys,
-                    vals, bj, bk, R, Bf, Cf, M, present, mB, mC, rmask);
-      } else if (masked) {
-        SPWS_LAUNCH(ctx, "mttkrp_accum", (k_mttkrp_accum<false, true>), dim3(ga), dim3(kAccBlock), 0, kept, seg, keys,
-                    vals, bj, bk, R, Bf, Cf, M, present, mB, mC, rmask);
-      } else {
-        SPWS_LAUNCH(ctx, "mttkrp_accum", (k_mttkrp_accum<false, false>), dim3(ga), dim3(kAccBlock), 0, kept, seg,
-                    keys, vals, bj, bk, R, Bf, Cf, M, present, mB, mC, rmask);
-      }
+      if (R <= 16 && masked) SPWS_MTTKRP_ACCUM(16, 1, true);
+      else if (R <= 16) SPWS_MTTKRP_ACCUM(16, 1, false);
+      else if (R <= 32 && masked) SPWS_MTTKRP_ACCUM(32, 1, true);
+      else if (R <= 32) SPWS_MTTKRP_ACCUM(32, 1, false);
+      else if (masked) SPWS_MTTKRP_ACCUM(32, 2, true);
+      else SPWS_MTTKRP_ACCUM(32, 2, false);
     }
+#undef SPWS_MTTKRP_ACCUM
     ctx->stats.products = kept * (int64_t)R;
   }
   if ((rc = exclusive_scan<int32_t, int32_t>(ctx, present, poff, I))) return rc;

@@ -58,6 +58,61 @@ def test_mttkrp_small(ctx, R):
     assert np.all(M[empty] == 0)
 
 
+def check_mttkrp(ctx, dims, idx, Bf, Cf, seed):
+    """MTTKRP of the coordinates idx (distinct) against extended-precision
+    sums."""
+    rng = np.random.default_rng(seed)
+    idx = np.asarray(idx, dtype=np.int32)
+    idx = idx[np.lexsort((idx[:, 2], idx[:, 1], idx[:, 0]))]
+    X = gen.COO3(dims, idx, rng.uniform(-1.0, 1.0, len(idx)))
+    rows, M = run_mttkrp(ctx, X, Bf, Cf)
+    np.testing.assert_array_equal(rows, np.unique(idx[:, 0]))
+    exact = np.zeros((dims[0], Bf.shape[1]), dtype=np.longdouble)
+    absum = np.zeros((dims[0], Bf.shape[1]))
+    for at in range(0, len(idx), 1 << 18):
+        i, j, k = idx[at:at + (1 << 18)].T
+        t = (X.vals[at:at + (1 << 18), None] * Bf[j]) * Cf[k]
+        u, start = np.unique(i, return_index=True)
+        exact[u] += np.add.reduceat(t.astype(np.longdouble), start, axis=0)
+        absum[u] += np.add.reduceat(np.abs(t), start, axis=0)
+    assert oracle.max_value_error(M.ravel(), exact.astype(np.float64).ravel(), absum.ravel()) <= TOL
+
+
+# ranks at the edges of a group's lanes and slices; rows of one nonzero, rows
+# that end on a segment or a tile, one row over many tiles
+@pytest.mark.parametrize("R", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("shape", ["one", "singles", "segments", "hot"])
+def test_mttkrp_segment_edges(ctx, R, shape):
+    print(f"case: mttkrp segments {shape} R={R}", flush=True)
+    dims = (3000, 200, 150)
+    if shape == "one":
+        idx = [(5, 7, 9)]
+    elif shape == "singles":  # every nonzero its own row
+        idx = [(i, i % 200, i % 150) for i in range(2049)]
+    elif shape == "segments":  # rows of 31, 32, 33, 255, 256, 257, 511, 513 nonzeros
+        idx = [(3 * q, e % 200, e // 200) for q, c in enumerate((31, 32, 33, 255, 256, 257, 511, 513, 1, 1))
+               for e in range(c)]
+    else:  # one row of every (j, k), rows of one nonzero on both sides
+        dims = (3000, 2000, 600) if R == 32 else dims
+        j, k = np.meshgrid(np.arange(dims[1]), np.arange(dims[2]), indexing="ij")
+        idx = np.stack([np.full(j.size, 1500), j.ravel(), k.ravel()], axis=1)
+        idx = np.concatenate([idx, [(i, i % 200, i % 150) for i in range(1400, 1600) if i != 1500]])
+    rng = np.random.default_rng(R)
+    check_mttkrp(ctx, dims, idx, rng.uniform(-1, 1, (dims[1], R)), rng.uniform(-1, 1, (dims[2], R)), 5)
+
+
+def test_mttkrp_factor_over_4_gib(ctx):
+    """A factor of more than 2^32 bytes (64-bit addresses)."""
+    print("case: mttkrp wide factor", flush=True)
+    dims, R = (40, 30, 8_400_000), 64
+    rng = np.random.default_rng(6)
+    k = np.concatenate([rng.integers(0, dims[2], 300), [0, dims[2] - 1]])
+    Cf = np.zeros((dims[2], R))
+    Cf[k] = rng.uniform(-1, 1, (len(k), R))
+    idx = np.unique(np.stack([rng.integers(0, 40, len(k)), rng.integers(0, 30, len(k)), k], axis=1), axis=0)
+    check_mttkrp(ctx, dims, idx, rng.uniform(-1, 1, (dims[1], R)), Cf, 7)
+
+
 def test_mttkrp_taco_entry():
     print("case: mttkrp taco entry", flush=True)
     X = gen.zipf_coo3((120, 90, 70), 3000, (1.5, 1.5, 1.5), 12, 5, 0.0, 1.0)
