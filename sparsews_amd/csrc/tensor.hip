@@ -40,19 +40,18 @@
 //     2. radix sort         stable, on the (i, j) bits only: each fiber's
 //                           nonzeros end up together and keep the CSF order,
 //                           increasing k -- the order hash_il sums them.
-//     3. k_ttm_fiber_count + scan of the tile counts + k_ttm_fiber_starts:
-//                           fiber heads ranked within their tile, fiber
-//                           offsets and the output coordinates (i, j).
-//     4. k_ttm_accum        one 16-lane group per work item (at most 128
-//                           nonzeros of one fiber) sums X * U(k,:) in order;
-//                           a fiber of one item writes its vector, longer
-//                           fibers write partial sums that k_ttm_combine adds
-//                           in item order (no atomics; deterministic).
+//     3. k_ttm_seg_starts + scan: fiber starts per segment of 32 to 128
+//                           nonzeros, so each segment knows its first fiber.
+//     4. k_ttm_accum        one 16-lane group per segment sums X * U(k,:) in
+//                           order and writes each fiber that starts there,
+//                           with its coordinates; segments inside a longer
+//                           fiber write partial sums that k_ttm_fixup adds in
+//                           order (no atomics; deterministic).
 //   When i, j and k need more than 64 bits together, the fibers are found
 //   through an open-addressing table in HBM (k_ttm_insert, 64-bit keys
 //   (i << bj) | j, atomicCAS), collected and sorted (k_ttm_occupied,
 //   k_ttm_collect, radix sort, k_ttm_rank), and the nonzeros are then
-//   sorted by fiber rank (k_ttm_keys, k_ttm_heads) before step 5.
+//   sorted by fiber rank (k_ttm_keys) before steps 3 and 4.
 //   Output: semi-sparse -- the sorted fiber list (i,j) with a dense length-R
 //   vector each.
 #include <algorithm>
@@ -497,172 +496,236 @@ __global__ __launch_bounds__(256) void k_ttm_keys(int64_t nnz, const int32_t* __
   }
 }
 
-// foff[q] = first sorted position of fiber q (every fiber has a nonzero).
-__global__ __launch_bounds__(256) void k_ttm_heads(int64_t nnz, const uint64_t* __restrict__ keys, int bk, int64_t F,
-                                                   int32_t* __restrict__ foff) {
-  for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < nnz; p += (int64_t)gridDim.x * blockDim.x) {
-    const uint64_t q = keys[p] >> bk;
-    if (p == 0 || (keys[p - 1] >> bk) != q) foff[q] = (int32_t)p;
-    if (p == 0) foff[F] = (int32_t)nnz;
-  }
-}
+// Per-fiber sums over the nonzeros grouped by fiber (the keys' high bits are
+// the fiber, the low bk bits k; within a fiber k increases), in segments of
+// consecutive nonzeros, one segment per group of 16 lanes (a DPP row; a rank
+// per lane, S slices of 16 ranks, further ranks on blockIdx.y).
+//
+// A fiber belongs to the group in whose segment it starts, which follows it
+// for kTtmReach nonzeros beyond the segment, so a fiber of at most kTtmReach
+// nonzeros is summed by one group from 0.0 in order and stored at once.  A
+// longer fiber may fill whole segments beyond that: their groups write
+// partial sums, which k_ttm_fixup adds in order (no atomics: the result does
+// not depend on timing).  seg_off = exclusive prefix of the fiber starts per
+// segment gives each group its first fiber's index, so no list of fibers or
+// work items is built.
+//
+// A group reads 16 keys and values at once (the next 16 in flight while these
+// are used) and stages them in LDS with the byte offset of each U row; the U
+// rows of 8 / S nonzeros are in flight together (68 VGPRs, 7 wavefronts per
+// SIMD: 205 us; 16 in flight at 5 per SIMD 246 us, 4 at 8 per SIMD 211 us, on
+// 10M nonzeros in 1.16M fibers, R = 16).  It is bound by the issue of the
+// gathers from L2.  One work item per fiber padded to 16 nonzeros took 373 us,
+// and its item lists and their combination 130 us more
+// where the starts and the fixup now take 35 us.
+constexpr int kTtmLanes = 16;
+constexpr int kTtmBlock = 256;
+constexpr int kTtmGroups = kTtmBlock / kTtmLanes;
+constexpr int kTtmReach = 128;
+// log2 of the segment: 128 nonzeros, or down to 32 where that leaves fewer
+// groups than the chip holds (a group walks its segment one batch after
+// another: 200k nonzeros, R = 24, 46 us in segments of 128 and 29 in 32)
+constexpr int kTtmSegLogMin = 5, kTtmSegLogMax = 7;
+constexpr int kTtmWgPerCu = 7;
+constexpr int kTtmInFlight = 8;  // U values per lane in flight
+constexpr int kTtmStartRounds = 16;  // strides of 64 nonzeros per wavefront of k_ttm_seg_starts
 
-// Work items of at most kTtmChunk sorted nonzeros: a fiber of n nonzeros
-// has ceil(n / kTtmChunk) items (fibers reach 2,000 nonzeros, one per k).
-constexpr int kTtmChunk = 128;
-constexpr int kTtmLanes = 16;  // one DPP row per group (broadcasts by row_newbcast)
-constexpr int kTtmU = 16;
-constexpr int kTtmBlocksPerCu = 5;  // workgroups per CU in the accumulation grid (5 waves per SIMD: 96 VGPRs)
-
-__global__ __launch_bounds__(256) void k_ttm_chunks(int64_t F, const int32_t* __restrict__ foff,
-                                                    int32_t* __restrict__ nchunk) {
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < F; q += (int64_t)gridDim.x * blockDim.x)
-    nchunk[q] = (foff[q + 1] - foff[q] + kTtmChunk - 1) / kTtmChunk;
-}
-
-// Work item records {first nonzero, end, destination}: the destination is
-// the fiber q for a fiber of one item (its vector goes to Y), else ~c for
-// item c (its partial sum goes to the partial-sum rows).
-__global__ __launch_bounds__(256) void k_ttm_itemmap(int64_t F, const int32_t* __restrict__ foff,
-                                                     const int32_t* __restrict__ coff, int4* __restrict__ items) {
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < F; q += (int64_t)gridDim.x * blockDim.x) {
-    const int32_t c0 = coff[q], c1 = coff[q + 1], f1 = foff[q + 1];
-    for (int32_t c = c0; c < c1; ++c) {
-      const int32_t p0 = foff[q] + (c - c0) * kTtmChunk;
-      items[c] = make_int4(p0, min(p0 + kTtmChunk, f1), c1 - c0 == 1 ? (int32_t)q : ~c, 0);
-    }
-  }
-}
-
-// acc + the in-order sum over nonzeros [base, p1) of an item, loaded
-// kTtmLanes at a time (only items of more than kTtmLanes nonzeros take it).
-template <bool kOff32>
-__device__ __forceinline__ double ttm_load_u(const double* __restrict__ U, uint32_t k, int R, int rr) {
-  // with kOff32 (K * R * 8 < 2^32) the byte offset is a 32-bit value: the
-  // load takes U's address from scalar registers and a one-register offset
-  if (kOff32)
-    return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(U) +
-                                            (k * (uint32_t)R + (uint32_t)rr) * 8u);
-  return U[(int64_t)k * R + rr];
-}
-
-template <bool kOff32>
-__device__ __forceinline__ double ttm_item_tail(double acc, int32_t base, int32_t p1, int l, int rr, int R, uint64_t km,
-                                             const uint64_t* __restrict__ keys, const double* __restrict__ vals,
-                                             const double* __restrict__ U) {
-  for (; base < p1; base += kTtmLanes) {
-    const int cnt2 = p1 - base < kTtmLanes ? p1 - base : kTtmLanes;
-    const int32_t m2 = base + (l < cnt2 ? l : cnt2 - 1);
-    const uint32_t k2 = (uint32_t)(keys[m2] & km);
-    const double v2 = vals[m2];
-    double uv[kTtmU];
+// Fiber starts per segment of 2^segl nonzeros (nonzero p starts a fiber when
+// its key's high bits differ from p - 1's).
+__global__ __launch_bounds__(256) void k_ttm_seg_starts(int64_t nnz, int segl, int64_t nseg,
+                                                        const uint64_t* __restrict__ keys, int bk,
+                                                        int32_t* __restrict__ cnt) {
+  const int lane = lane_id();
+  const int64_t p0 = ((int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave) * (kTtmStartRounds * kWave);
+  // the nonzero before each row of 16 lanes, loaded by its first lane; the
+  // others take theirs from the lane before
+  uint64_t key[kTtmStartRounds], edge[kTtmStartRounds];
 #pragma unroll
-    for (int u = 0; u < kTtmU; ++u) {
-      const uint32_t k = row_lane(k2, u);  // lanes past cnt2 hold the last entry
-      uv[u] = ttm_load_u<kOff32>(U, k, R, rr);
-    }
-#pragma unroll
-    for (int u = 0; u < kTtmU; ++u) {
-      const double x = row_lane(v2, u);
-      if (u < cnt2) acc += x * uv[u];
-    }
+  for (int u = 0; u < kTtmStartRounds; ++u) {
+    const int64_t p = p0 + u * kWave + lane;
+    key[u] = p < nnz ? keys[p] : 0;
+    edge[u] = (lane & 15) == 0 && p > 0 && p < nnz ? keys[p - 1] : 0;
   }
-  return acc;
+  uint64_t starts[kTtmStartRounds];  // uniform
+#pragma unroll
+  for (int u = 0; u < kTtmStartRounds; ++u) {
+    const int64_t p = p0 + u * kWave + lane;
+    const uint64_t left = dpp_move<0x111, 0xF>(key[u], edge[u]);  // row_shr:1
+    starts[u] = __ballot(p < nnz && (p == 0 || (key[u] >> bk) != (left >> bk)));
+  }
+  // 32-nonzero counts of the wavefront's rounds, a lane each, then the sums
+  // of 2^(segl - 5) neighbours
+  static_assert(2 * kTtmStartRounds <= kWave, "a lane per 32 nonzeros");
+  int32_t c = 0;
+#pragma unroll
+  for (int u = 0; u < kTtmStartRounds; ++u) {
+    if (lane == 2 * u) c = __popc((uint32_t)starts[u]);
+    if (lane == 2 * u + 1) c = __popc((uint32_t)(starts[u] >> 32));
+  }
+  for (int d = 1; d < 1 << (segl - 5); d <<= 1) c += __shfl_down(c, d, kWave);
+  const int64_t seg = (p0 + (int64_t)lane * 32) >> segl;
+  if (lane < 2 * kTtmStartRounds && (lane & ((1 << (segl - 5)) - 1)) == 0 && seg < nseg) cnt[seg] = c;
 }
 
-// One group of kTtmLanes lanes per work item (ranks r = lane, lane +
-// kTtmLanes, ...), each group walking items c, c + G, ... of a grid of G
-// groups.  The group holds its item's first kTtmLanes sorted keys/values (a
-// lane each), gathers the rows U(k,:) of all of them, then sums in order;
-// longer items load their further nonzeros kTtmLanes at a time.  While an
-// item's rows of U are in flight, the next item's keys/values and the record
-// after it load too, so each item costs about one memory latency instead of
-// three dependent ones.  A single-item fiber writes its vector; the items of
-// a longer fiber write partial sums, which k_ttm_combine adds in item order
-// (so the result does not depend on timing).
-template <bool kOff32>
-__global__ __launch_bounds__(256) void k_ttm_accum(const int32_t* __restrict__ nitems_p, int R,
-                                                   const int4* __restrict__ items,
-                                                   const uint64_t* __restrict__ keys, const double* __restrict__ vals,
-                                                   int bk, const double* __restrict__ U, double* __restrict__ Y,
-                                                   double* __restrict__ part) {
-  const int groups = 256 / kTtmLanes;
-  const int l = threadIdx.x % kTtmLanes;
-  const uint64_t km = (1ull << bk) - 1;
-  const uint32_t km32 = (uint32_t)km;  // k < 2^31: the key's low word holds it
-  const uint32_t* __restrict__ keys_lo = reinterpret_cast<const uint32_t*>(keys);  // little-endian low words
-  const int64_t nitems = *nitems_p;  // the items' count, on the device (the grid is sized for at most that many)
-  const int64_t stride = (int64_t)gridDim.x * groups;
-  int64_t c = (int64_t)blockIdx.x * groups + threadIdx.x / kTtmLanes;
-  if (c >= nitems) return;  // uniform per group
-  // current item: record and first keys/values; next item: record
-  int4 cur = items[c];
-  int4 nxt = make_int4(0, 1, 0, 0);
-  if (c + stride < nitems) nxt = items[c + stride];
-  int32_t me = cur.x + min(l, cur.y - cur.x - 1);
-  uint32_t kraw = keys_lo[2 * (int64_t)me];
-  double myval = vals[me];
-  for (;;) {
-    const int64_t cn = c + stride;
-    const bool has_next = cn < nitems;  // uniform per group
-    // prefetches, left unused until the next iteration (no wait here)
-    uint32_t nkraw = 0;
-    double nval = 0.0;
-    int4 nn = nxt;
-    if (has_next) {
-      const int32_t nme = nxt.x + min(l, nxt.y - nxt.x - 1);
-      nkraw = keys_lo[2 * (int64_t)nme];
-      nval = vals[nme];
-      if (cn + stride < nitems) nn = items[cn + stride];
-    }
-    const uint32_t myk = kraw & km32;
-    const int32_t p0 = cur.x, p1 = cur.y;
-    const int cnt = min(p1 - p0, kTtmLanes);
-    for (int r0 = 0; r0 < R; r0 += kTtmLanes) {
-      const int r = r0 + l;
-      const int rr = r < R ? r : R - 1;
-      double acc = 0.0;
-      {
-        double uv[kTtmU];
-#pragma unroll
-        for (int u = 0; u < kTtmU; ++u) {
-          const uint32_t k = row_lane(myk, u);  // lanes past cnt hold the last entry
-          uv[u] = ttm_load_u<kOff32>(U, k, R, rr);
-        }
-#pragma unroll
-        for (int u = 0; u < kTtmU; ++u) {
-          const double x = row_lane(myval, u);
-          if (u < cnt) acc += x * uv[u];
-        }
-      }
-      // the item's further nonzeros (items of more than kTtmLanes)
-      if (p1 - p0 > kTtmLanes) acc = ttm_item_tail<kOff32>(acc, p0 + kTtmLanes, p1, l, rr, R, km, keys, vals, U);
-      if (r < R) {
-        if (cur.z >= 0) Y[(int64_t)cur.z * R + r] = acc;
-        else part[(int64_t)(~cur.z) * R + r] = acc;
-      }
-    }
-    if (!has_next) break;
-    c = cn;
-    cur = nxt;
-    nxt = nn;
-    kraw = nkraw;
-    myval = nval;
-  }
-}
-
-// Fibers of several items: Y(q,:) = sum of their partial sums in item order.
-__global__ __launch_bounds__(256) void k_ttm_combine(int64_t F, int R, const int32_t* __restrict__ coff,
-                                                     const double* __restrict__ part, double* __restrict__ Y) {
-  const int groups = 256 / kTtmLanes;
+// kMask: every fiber's fmask is or-ed with the U row masks of its nonzeros.
+template <int S, bool kOff32, bool kMask>
+__global__ __launch_bounds__(kTtmBlock, kMask ? 4 : 7) void k_ttm_accum(int64_t nnz, int segl, int64_t nseg, int R,
+                                                         const uint64_t* __restrict__ keys,
+                                                         const double* __restrict__ vals, int bj, int bk,
+                                                         const int32_t* __restrict__ seg_off,
+                                                         const double* __restrict__ U, double* __restrict__ Y,
+                                                         double* __restrict__ part, int32_t* __restrict__ out_i,
+                                                         int32_t* __restrict__ out_j,
+                                                         const uint64_t* __restrict__ umask,
+                                                         unsigned long long* __restrict__ fmask) {
+  constexpr int kU = kTtmInFlight / S;  // nonzeros whose U rows are in flight together
+  // a nonzero as the sums read it: its U row's byte offset (kOff32: U below
+  // 4 GiB) or its k, and its value; one pad record per group keeps the four
+  // groups of a wavefront in different LDS banks
+  struct alignas(16) Rec {
+    uint32_t k, pad;
+    double val;
+  };
+  __shared__ Rec recs[kTtmGroups][kTtmLanes + 1];
   const int g = threadIdx.x / kTtmLanes;
   const int l = threadIdx.x % kTtmLanes;
-  for (int64_t q = (int64_t)blockIdx.x * groups + g; q < F; q += (int64_t)gridDim.x * groups) {
-    const int32_t c0 = coff[q], c1 = coff[q + 1];
-    if (c1 - c0 <= 1) continue;
+  const int64_t s = (int64_t)blockIdx.x * kTtmGroups + g;
+  if (s >= nseg) return;  // uniform per group; no barrier follows
+  const int r0 = blockIdx.y * (S * kTtmLanes) + l;
+  const bool lead_block = blockIdx.y == 0;
+  const uint32_t km = (uint32_t)((1ull << bk) - 1);  // k < 2^31
+  const uint64_t jm = (1ull << bj) - 1;
+  const uint32_t unit = kOff32 ? (uint32_t)R * 8u : 1u;
+  uint32_t rr[S];  // in-range ranks for the loads
+#pragma unroll
+  for (int q = 0; q < S; ++q) rr[q] = (uint32_t)min(r0 + q * kTtmLanes, R - 1);
+  const int64_t e0 = s << segl;
+  const int64_t e1 = min(e0 + (1 << segl), nnz);
+  const int64_t lim = min(e1 + kTtmReach, nnz);
+  const int32_t q0 = seg_off[s] - 1;  // the fiber running into this segment
+  // that fiber is this group's to sum (as a partial sum) when the segments
+  // within reach before this one have no start: its own group ends there
+  const int back = kTtmReach >> segl;
+  const bool filled = s >= back && seg_off[s - back] == q0 + 1;
+  uint64_t fprev = e0 > 0 ? keys[e0 - 1] >> bk : ~0ull;
+  uint64_t key = 0;
+  double val = 0.0;
+  if (e0 + l < lim) {
+    key = keys[e0 + l];
+    val = vals[e0 + l];
+  }
+  constexpr int32_t kDrop = -1, kPart = -2;
+  int32_t dest = filled ? kPart : kDrop;
+  int32_t q = q0;
+  double acc[S];
+#pragma unroll
+  for (int x = 0; x < S; ++x) acc[x] = 0.0;
+  uint64_t rowm = 0;
+  const auto flush = [&]() {
+    if (dest == kDrop) return;
+    double* const to = dest >= 0 ? Y + (int64_t)dest * R : part + s * R;
+#pragma unroll
+    for (int x = 0; x < S; ++x)
+      if (r0 + x * kTtmLanes < R) to[r0 + x * kTtmLanes] = acc[x];
+    if (kMask && l == 0 && lead_block) atomicOr(&fmask[dest >= 0 ? dest : q0], (unsigned long long)rowm);
+  };
+  Rec* const mine = recs[g];
+  for (int64_t base = e0; base < lim; base += kTtmLanes) {  // uniform per group
+    const bool beyond = base >= e1;  // following the last fiber out of the segment
+    if (beyond && dest < 0) break;
+    const uint64_t f = base + l < lim ? key >> bk : fprev;
+    const uint64_t left = dpp_move<0x111, 0xF>(f, fprev);  // row_shr:1; lane 0: the nonzero before
+    const bool start = base + l < lim && (f != left || base + l == 0);
+    const uint32_t hm = (uint32_t)(__ballot(start) >> (threadIdx.x & (kWave - kTtmLanes))) & 0xFFFFu;
+    int cnt = (int)min((int64_t)kTtmLanes, lim - base);
+    if (beyond && hm) cnt = __builtin_ctz(hm);  // the fiber ends here
+    mine[l].k = ((uint32_t)key & km) * unit;
+    mine[l].val = val;
+    if (!beyond && lead_block && out_i && start) {
+      const int32_t at = q + __popc(hm & ((2u << l) - 1u));
+      out_i[at] = (int32_t)(f >> bj);
+      out_j[at] = (int32_t)(f & jm);
+    }
+    fprev = row_lane(f, kTtmLanes - 1);
+    __builtin_amdgcn_wave_barrier();
+    if (base + kTtmLanes + l < lim) {
+      key = keys[base + kTtmLanes + l];
+      val = vals[base + kTtmLanes + l];
+    }
+    for (int t = 0; t < cnt; t += kU) {
+      double xv[kU], uv[kU][S];
+      uint64_t mk[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const Rec rec = mine[t + u < cnt ? t + u : cnt - 1];
+        xv[u] = rec.val;
+#pragma unroll
+        for (int x = 0; x < S; ++x) {
+          if (kOff32)
+            uv[u][x] = *reinterpret_cast<const double*>(reinterpret_cast<const char*>(U) + (rec.k + rr[x] * 8u));
+          else
+            uv[u][x] = U[(int64_t)rec.k * R + rr[x]];
+        }
+        if (kMask) mk[u] = umask[rec.k / unit];
+      }
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        if (t + u >= cnt) break;  // uniform per group
+        if ((hm >> (t + u)) & 1u) {
+          flush();
+          dest = ++q;
+#pragma unroll
+          for (int x = 0; x < S; ++x) acc[x] = 0.0;
+          rowm = 0;
+        }
+#pragma unroll
+        for (int x = 0; x < S; ++x) acc[x] += xv[u] * uv[u][x];
+        if (kMask) rowm |= mk[u];
+      }
+    }
+    if (beyond && hm) break;
+  }
+  flush();
+}
+
+// Fibers longer than their group's reach: Y(q,:) += the partial sums of the
+// segments beyond it, in order.  A lane looks at each segment; the first such
+// segments of the fibers are listed in LDS and taken by groups of 16 lanes.
+__global__ __launch_bounds__(kTtmBlock) void k_ttm_fixup(int segl, int64_t nseg, int R,
+                                                         const uint64_t* __restrict__ keys, int bk,
+                                                         const int32_t* __restrict__ seg_off,
+                                                         const double* __restrict__ part, double* __restrict__ Y) {
+  __shared__ int32_t list[kTtmBlock];
+  __shared__ int32_t count;
+  if (threadIdx.x == 0) count = 0;
+  __syncthreads();
+  const int back = kTtmReach >> segl;
+  const int64_t s0 = back + 1 + (int64_t)blockIdx.x * kTtmBlock;
+  // a segment whose leading nonzeros were summed into part: no fiber starts
+  // in the segments within reach before it and the fiber goes on
+  const auto runs_on = [&](int64_t t) {
+    return t < nseg && seg_off[t] == seg_off[t - back] &&
+           (keys[t << segl] >> bk) == (keys[(t << segl) - 1] >> bk);
+  };
+  const int64_t mine = s0 + threadIdx.x;
+  if (mine < nseg && seg_off[mine - back] != seg_off[mine - back - 1] && runs_on(mine))
+    list[atomicAdd(&count, 1)] = threadIdx.x;
+  __syncthreads();
+  const int l = threadIdx.x % kTtmLanes;
+  for (int c = threadIdx.x / kTtmLanes; c < count; c += kTtmGroups) {  // uniform per group
+    const int64_t s = s0 + list[c];
+    const int64_t q = seg_off[s] - 1;
+    int64_t end = s + 1;
+    for (;;) {  // 16 segments looked at together
+      const uint32_t stop =
+          (uint32_t)(__ballot(!runs_on(end + l)) >> (threadIdx.x & (kWave - kTtmLanes))) & 0xFFFFu;
+      end += stop ? __builtin_ctz(stop) : kTtmLanes;
+      if (stop) break;
+    }
     for (int r = l; r < R; r += kTtmLanes) {
-      double acc = part[(int64_t)c0 * R + r];
-      for (int32_t c = c0 + 1; c < c1; ++c) acc += part[(int64_t)c * R + r];
+      double acc = Y[q * R + r];
+#pragma unroll 4
+      for (int64_t t = s; t < end; ++t) acc += part[t * R + r];
       Y[q * R + r] = acc;
     }
   }
@@ -704,97 +767,6 @@ __global__ __launch_bounds__(256) void k_ttm_direct_keys(int64_t nnz, const int3
     nd = wave_sum(nd);
     if (lane_id() == 0 && nd) atomicAdd(dropped, nd);
   }
-}
-
-// per fiber: the OR of its nonzeros' U row masks (its stored output columns)
-__global__ __launch_bounds__(256) void k_ttm_fiber_mask(int64_t F, const int32_t* __restrict__ foff,
-                                                        const uint64_t* __restrict__ keys, int bk,
-                                                        const uint64_t* __restrict__ umask, uint64_t* __restrict__ fmask) {
-  const uint64_t km = (1ull << bk) - 1;
-  for (int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; f < F; f += (int64_t)gridDim.x * blockDim.x) {
-    uint64_t m = 0;
-    for (int32_t p = foff[f]; p < foff[f + 1]; ++p) m |= umask[keys[p] & km];
-    fmask[f] = m;
-  }
-}
-
-// Fiber starts of the sorted nonzeros (p starts a fiber when its (i, j)
-// differs from p - 1's), in tiles of kFibTile: a count per tile, then (with
-// the counts' prefix) each tile's starts ranked in order, with no flag or
-// rank array per nonzero.  A tile is walked in kFibItems coalesced rounds of
-// kFibBlock nonzeros; ballots give the ranks within a round's wavefronts.
-constexpr int kFibBlock = 256;
-constexpr int kFibItems = 16;
-constexpr int kFibTile = kFibBlock * kFibItems;
-constexpr int kFibWaves = kFibBlock / kWave;
-
-// Whether nonzero p starts a fiber (false past the end).
-__device__ __forceinline__ bool ttm_fiber_start(int64_t nnz, const uint64_t* __restrict__ keys, int bk, int64_t p) {
-  if (p >= nnz) return false;
-  return p == 0 || (keys[p - 1] >> bk) != (keys[p] >> bk);
-}
-
-__global__ __launch_bounds__(kFibBlock) void k_ttm_fiber_count(int64_t nnz, const uint64_t* __restrict__ keys, int bk,
-                                                                int32_t* __restrict__ tile_cnt) {
-  __shared__ int32_t wsum[kFibWaves];
-  const int64_t base = (int64_t)blockIdx.x * kFibTile + threadIdx.x;
-  int32_t c = 0;
-#pragma unroll
-  for (int it = 0; it < kFibItems; ++it) c += __popcll(__ballot(ttm_fiber_start(nnz, keys, bk, base + it * kFibBlock)));
-  if (lane_id() == 0) wsum[threadIdx.x / kWave] = c;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int32_t t = 0;
-#pragma unroll
-    for (int w = 0; w < kFibWaves; ++w) t += wsum[w];
-    tile_cnt[blockIdx.x] = t;
-  }
-}
-
-// tile_off = exclusive prefix of the tile counts (tile_off[ntiles] = F):
-// fiber q starts at foff[q]; its coordinates come from the key.
-__global__ __launch_bounds__(kFibBlock) void k_ttm_fiber_starts(int64_t nnz, const uint64_t* __restrict__ keys, int bj,
-                                                                int bk, const int32_t* __restrict__ tile_off,
-                                                                int64_t ntiles, int32_t* __restrict__ foff,
-                                                                int32_t* __restrict__ out_i,
-                                                                int32_t* __restrict__ out_j) {
-  // starts per (round, wavefront), then their exclusive prefix in that order
-  __shared__ int32_t cnt[kFibItems * kFibWaves];
-  static_assert(kFibItems * kFibWaves == kWave, "one wavefront scans the per-round counts");
-  const uint64_t jm = (1ull << bj) - 1;
-  const int lane = lane_id();
-  const int w = threadIdx.x / kWave;
-  const int64_t base = (int64_t)blockIdx.x * kFibTile + threadIdx.x;
-  const uint64_t below = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
-  uint32_t mine = 0;  // bit it: this thread's nonzero of round it starts a fiber
-  int32_t before[kFibItems];  // starts of this wavefront's lanes below this one, per round
-#pragma unroll
-  for (int it = 0; it < kFibItems; ++it) {
-    const bool st = ttm_fiber_start(nnz, keys, bk, base + it * kFibBlock);
-    const uint64_t m = __ballot(st);
-    mine |= (st ? 1u : 0u) << it;
-    before[it] = __popcll(m & below);
-    if (lane == 0) cnt[it * kFibWaves + w] = __popcll(m);
-  }
-  __syncthreads();
-  if (w == 0) {
-    const int32_t v = cnt[lane];
-    cnt[lane] = wave_incl_scan(v) - v;
-  }
-  __syncthreads();
-  const int32_t t0 = tile_off[blockIdx.x];
-#pragma unroll
-  for (int it = 0; it < kFibItems; ++it) {
-    if ((mine >> it) & 1u) {
-      const int64_t p = base + it * kFibBlock;
-      const int32_t q = t0 + cnt[it * kFibWaves + w] + before[it];
-      const uint64_t key = keys[p];
-      foff[q] = (int32_t)p;
-      out_i[q] = (int32_t)(key >> (bj + bk));
-      out_j[q] = (int32_t)((key >> bk) & jm);
-    }
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) foff[tile_off[ntiles]] = (int32_t)nnz;
 }
 
 static int csf_owners(spws_ctx* ctx, const Csf3& x, int32_t** leaf_fiber, int32_t** fiber_root) {
@@ -937,41 +909,59 @@ static int mttkrp_run(spws_ctx* ctx, const Csf3& x, int32_t I, int32_t J, int32_
   return SPWS_OK;
 }
 
-// Per-fiber sums over nonzeros grouped by fiber (foff[F + 1], keys' low bk
-// bits = k): work items of at most kTtmChunk nonzeros, in-order sums, then
-// the partial sums of long fibers combined in item order.
-static int ttm_accumulate(spws_ctx* ctx, int64_t nnz, int64_t F, int32_t R, int bk, const uint64_t* nkeys,
-                          const double* nvals, const int32_t* foff, const double* U, double* Y) {
-  int rc;
-  // coff = prefix of items per fiber
-  if ((rc = ctx->obuf[2].ensure(((size_t)F + 1) * 4 * 2))) return rc;
-  int32_t* nchunk = ctx->obuf[2].as<int32_t>();
-  int32_t* coff = nchunk + (F + 1);
-  const unsigned gf2 = (unsigned)std::min<int64_t>(div_up(F, 256), 65536);
-  SPWS_LAUNCH(ctx, "ttm_chunks", k_ttm_chunks, dim3(gf2), dim3(256), 0, F, foff, nchunk);
-  if ((rc = exclusive_scan<int32_t, int32_t>(ctx, nchunk, coff, F))) return rc;
-  // items <= F + nnz / kTtmChunk
-  const int64_t max_items = F + nnz / kTtmChunk + 1;
-  if ((rc = ctx->obuf[3].ensure((size_t)max_items * R * 8)) || (rc = ctx->obuf[4].ensure((size_t)max_items * 16)))
-    return rc;
-  // the item count stays on the device (coff[F]): no wait for it here
-  const int32_t* nitems_dev = coff + F;
-  int4* items = ctx->obuf[4].as<int4>();
-  SPWS_LAUNCH(ctx, "ttm_itemmap", k_ttm_itemmap, dim3(gf2), dim3(256), 0, F, foff, coff, items);
-  // one workgroup per slot of a few per CU: each group walks many items
-  int cus = 0;
+// Fiber starts per segment (2^*segl nonzeros) of the grouped nonzeros into
+// obuf[2] and their prefix into obuf[5], whose last entry is the number of
+// fibers.
+static int ttm_seg_offsets(spws_ctx* ctx, int64_t nnz, const uint64_t* nkeys, int bk, int* segl) {
+  int rc, cus = 0;
   SPWS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-  const unsigned ga = (unsigned)std::max<int64_t>(1, std::min<int64_t>(div_up(max_items, 256 / kTtmLanes),
-                                                                        (int64_t)std::max(cus, 1) * kTtmBlocksPerCu));
+  int l = kTtmSegLogMin;
+  while (l < kTtmSegLogMax && (nnz >> (l + 1)) >= (int64_t)cus * kTtmWgPerCu * kTtmGroups) ++l;
+  *segl = l;
+  const int64_t nseg = div_up(nnz, (int64_t)1 << l);
+  if ((rc = ctx->obuf[2].ensure((size_t)nseg * 4 + 4)) || (rc = ctx->obuf[5].ensure(((size_t)nseg + 1) * 4))) return rc;
+  int32_t* cnt = ctx->obuf[2].as<int32_t>();
+  if (nseg > 0)
+    SPWS_LAUNCH(ctx, "ttm_starts", k_ttm_seg_starts, dim3((unsigned)div_up(nnz, 256 * kTtmStartRounds)), dim3(256), 0,
+                nnz, l, nseg, nkeys, bk, cnt);
+  return exclusive_scan<int32_t, int32_t>(ctx, cnt, ctx->obuf[5].as<int32_t>(), nseg);
+}
+
+// Per-fiber sums over the grouped nonzeros (after ttm_seg_offsets) into Y,
+// and, with out_i, the fibers' coordinates.  umask and fmask: both or neither
+// (fmask zero on entry).
+static int ttm_accumulate(spws_ctx* ctx, int64_t nnz, int segl, int32_t R, int bj, int bk, const uint64_t* nkeys,
+                          const double* nvals, const double* U, double* Y, int32_t* out_i, int32_t* out_j,
+                          const uint64_t* umask, unsigned long long* fmask) {
+  int rc;
+  const int64_t nseg = div_up(nnz, (int64_t)1 << segl);
+  if ((rc = ctx->obuf[3].ensure((size_t)nseg * R * 8))) return rc;
+  double* part = ctx->obuf[3].as<double>();
+  const int32_t* seg_off = ctx->obuf[5].as<int32_t>();
   const bool off32 = ((int64_t)1 << bk) * R * 8 <= (int64_t)UINT32_MAX;  // every U offset fits in 32 bits
-  if (off32)
-    SPWS_LAUNCH(ctx, "ttm_accum", k_ttm_accum<true>, dim3(ga), dim3(256), 0, nitems_dev, R, items, nkeys, nvals, bk,
-                U, Y, ctx->obuf[3].as<double>());
-  else
-    SPWS_LAUNCH(ctx, "ttm_accum", k_ttm_accum<false>, dim3(ga), dim3(256), 0, nitems_dev, R, items, nkeys, nvals, bk,
-                U, Y, ctx->obuf[3].as<double>());
-  const unsigned gc = (unsigned)std::min<int64_t>(div_up(F, 256 / kTtmLanes), 65536);
-  SPWS_LAUNCH(ctx, "ttm_combine", k_ttm_combine, dim3(gc), dim3(256), 0, F, R, coff, ctx->obuf[3].as<double>(), Y);
+  const int slices = R <= 16 ? 1 : R <= 32 ? 2 : 4;
+  const dim3 grid((unsigned)div_up(nseg, kTtmGroups), (unsigned)div_up(R, slices * kTtmLanes));
+#define SPWS_TTM_ACCUM(S, OFF32, MASK)                                                                            \
+  SPWS_LAUNCH(ctx, "ttm_accum", (k_ttm_accum<S, OFF32, MASK>), grid, dim3(kTtmBlock), 0, nnz, segl, nseg, R, nkeys, \
+              nvals, bj, bk, seg_off, U, Y, part, out_i, out_j, umask, fmask)
+#define SPWS_TTM_ACCUM_S(S)                       \
+  do {                                            \
+    if (umask && off32) SPWS_TTM_ACCUM(S, true, true);        \
+    else if (umask) SPWS_TTM_ACCUM(S, false, true); \
+    else if (off32) SPWS_TTM_ACCUM(S, true, false); \
+    else SPWS_TTM_ACCUM(S, false, false);         \
+  } while (0)
+  switch (slices) {
+    case 1: SPWS_TTM_ACCUM_S(1); break;
+    case 2: SPWS_TTM_ACCUM_S(2); break;
+    default: SPWS_TTM_ACCUM_S(4); break;
+  }
+#undef SPWS_TTM_ACCUM_S
+#undef SPWS_TTM_ACCUM
+  const int64_t late = nseg - (kTtmReach >> segl) - 1;  // segments beyond the first group's reach
+  if (late > 0)
+    SPWS_LAUNCH(ctx, "ttm_fixup", k_ttm_fixup, dim3((unsigned)div_up(late, kTtmBlock)), dim3(kTtmBlock), 0, segl,
+                nseg, R, nkeys, bk, seg_off, (const double*)part, Y);
   return SPWS_OK;
 }
 
@@ -1010,11 +1000,13 @@ static int ttm_run(spws_ctx* ctx, const Csf3& x, int32_t I, int32_t J, int32_t K
   // hash path: a table of 2 * nnz (power of two) slots
   uint64_t T = 1024;
   while (!direct && T < 2 * (uint64_t)nz) T <<= 1;
-  const size_t nflag = direct ? nz + 1 : T + 1;
-  if ((rc = ctx->row_nnz.ensure(nflag * 4 * 2)) || (rc = ctx->keys[0].ensure(nz * 8)) ||
-      (rc = ctx->keys[1].ensure(nz * 8)) || (rc = ctx->vals[0].ensure(nz * 8)) || (rc = ctx->vals[1].ensure(nz * 8)))
+  const size_t nflag = T + 1;
+  if ((rc = ctx->keys[0].ensure(nz * 8)) || (rc = ctx->keys[1].ensure(nz * 8)) || (rc = ctx->vals[0].ensure(nz * 8)) ||
+      (rc = ctx->vals[1].ensure(nz * 8)))
     return rc;
-  if (!direct && ((rc = ctx->wide_tab.ensure(T * 8)) || (rc = ctx->slot_crd.ensure(nz * 4)))) return rc;
+  if (!direct && ((rc = ctx->row_nnz.ensure(nflag * 4 * 2)) || (rc = ctx->wide_tab.ensure(T * 8)) ||
+                  (rc = ctx->slot_crd.ensure(nz * 4))))
+    return rc;
   unsigned long long* table = ctx->wide_tab.as<unsigned long long>();
   int32_t* leaf_slot = ctx->slot_crd.as<int32_t>();
   int32_t* flag = ctx->row_nnz.as<int32_t>();
@@ -1057,34 +1049,25 @@ static int ttm_run(spws_ctx* ctx, const Csf3& x, int32_t I, int32_t J, int32_t K
       SPWS_HIP(hipStreamSynchronize(s));
       kept = x.nnz - *hd;
     }
-    // fiber starts counted per tile and the counts' prefix (flag / off hold
-    // nnz + 1 entries here, more than the tiles)
-    const int64_t ftiles = div_up(kept, kFibTile);
-    if (kept > 0)
-      SPWS_LAUNCH(ctx, "ttm_fibcount", k_ttm_fiber_count, dim3((unsigned)ftiles), dim3(kFibBlock), 0, kept, nkeys, bk,
-                  flag);
-    if ((rc = exclusive_scan<int32_t, int32_t>(ctx, flag, off, ftiles))) return rc;
-    SPWS_HIP(hipMemcpyAsync(hm, off + ftiles, 4, hipMemcpyDeviceToHost, s));
+    int segl;
+    if ((rc = ttm_seg_offsets(ctx, kept, nkeys, bk, &segl))) return rc;
+    SPWS_HIP(hipMemcpyAsync(hm, ctx->obuf[5].as<int32_t>() + div_up(kept, (int64_t)1 << segl), 4,
+                            hipMemcpyDeviceToHost, s));
     SPWS_HIP(hipStreamSynchronize(s));
     F = *hm;
     if ((rc = ctx->out_crd.ensure((size_t)(F > 0 ? F : 1) * 4 * 2)) ||
-        (rc = ctx->out_val.ensure((size_t)(F > 0 ? F : 1) * R * 8)) ||
-        (rc = ctx->obuf[5].ensure(((size_t)F + 1) * 4)))
+        (rc = ctx->out_val.ensure((size_t)(F > 0 ? F : 1) * R * 8)))
       return rc;
     int32_t* out_i = ctx->out_crd.as<int32_t>();
-    int32_t* out_j = out_i + F;
-    int32_t* foff = ctx->obuf[5].as<int32_t>();
-    if (kept > 0) {
-      SPWS_LAUNCH(ctx, "ttm_starts", k_ttm_fiber_starts, dim3((unsigned)ftiles), dim3(kFibBlock), 0, kept, nkeys, bj,
-                  bk, off, ftiles, foff, out_i, out_j);
-      if ((rc = ttm_accumulate(ctx, kept, F, R, bk, nkeys, nvals, foff, U, ctx->out_val.as<double>()))) return rc;
-    }
-    if (masked && F > 0) {
+    unsigned long long* fmask = nullptr;
+    if (masked) {
       if ((rc = ctx->obuf[6].ensure(256 + (size_t)F * 8))) return rc;
-      const unsigned gfm = (unsigned)std::min<int64_t>(div_up(F, 256), 65536);
-      SPWS_LAUNCH(ctx, "ttm_fiber_mask", k_ttm_fiber_mask, dim3(gfm), dim3(256), 0, F, foff, nkeys, bk, umask,
-                  reinterpret_cast<uint64_t*>(ctx->obuf[6].as<char>() + 256));
+      fmask = reinterpret_cast<unsigned long long*>(ctx->obuf[6].as<char>() + 256);
+      if (F > 0) SPWS_HIP(hipMemsetAsync(fmask, 0, (size_t)F * 8, s));
     }
+    if (kept > 0 && (rc = ttm_accumulate(ctx, kept, segl, R, bj, bk, nkeys, nvals, U, ctx->out_val.as<double>(), out_i,
+                                         out_i + F, umask, fmask)))
+      return rc;
     ctx->stats.products = kept * (int64_t)R;
   } else if (x.nnz > 0) {
     int32_t *leaf_fiber, *fiber_root;
@@ -1137,10 +1120,10 @@ static int ttm_run(spws_ctx* ctx, const Csf3& x, int32_t I, int32_t J, int32_t K
       nkeys = ctx->keys[1].as<uint64_t>();
       nvals = ctx->vals[1].as<double>();
     }
-    // fiber offsets reuse the flag array past rank_of_slot's T entries
-    int32_t* foff = off;
-    SPWS_LAUNCH(ctx, "ttm_heads", k_ttm_heads, dim3(g), dim3(256), 0, x.nnz, nkeys, bk, F, foff);
-    if ((rc = ttm_accumulate(ctx, x.nnz, F, R, bk, nkeys, nvals, foff, U, Y))) return rc;
+    int segl;
+    if ((rc = ttm_seg_offsets(ctx, x.nnz, nkeys, bk, &segl)) ||
+        (rc = ttm_accumulate(ctx, x.nnz, segl, R, bj, bk, nkeys, nvals, U, Y, nullptr, nullptr, nullptr, nullptr)))
+      return rc;
     ctx->stats.products = x.nnz * (int64_t)R;
   } else {
     if ((rc = ctx->out_crd.ensure(8)) || (rc = ctx->out_val.ensure(8))) return rc;

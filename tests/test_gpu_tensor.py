@@ -201,6 +201,58 @@ def test_ttm_roots_declines_wide_output_mode(ctx):
     np.testing.assert_array_equal(np.repeat(fj, 16), oj)
 
 
+# fibers at the edges of a segment (32 to 128 nonzeros) and of a group's reach
+# beyond it (128), alone, after short ones and over many segments; ranks at the
+# edges of a group's lanes and slices
+@pytest.mark.parametrize("R", [1, 16, 17, 33, 64, 65, 256])
+@pytest.mark.parametrize("lengths", [
+    (1,), (128,), (129,), (1200,),
+    tuple([1] * 515),
+    (31, 33, 32, 127, 129, 128, 1, 161, 160, 159, 257, 1, 1, 255, 383, 1000, 3, 1200, 1200, 2),
+    (7, 1200, 64, 64, 64, 96, 32, 1199, 1, 17, 500, 300),
+])
+def test_ttm_segment_edges(ctx, R, lengths):
+    """Fibers of at most 128 nonzeros bit for bit the sum in increasing k;
+    longer ones within the tolerance and the same again on a second call."""
+    print(f"case: ttm segments R={R} lengths={lengths[:8]}", flush=True)
+    K, J = 1200, 90
+    rng = np.random.default_rng(R)
+    idx = [(q // J, q % J, k) for q, c in enumerate(lengths) for k in sorted(rng.permutation(K)[:c])]
+    idx = np.asarray(idx, dtype=np.int32)
+    X = gen.COO3((len(lengths) // J + 1, J, K), idx, rng.uniform(-1, 1, len(idx)))
+    U = rng.uniform(-1, 1, (K, R))
+    fi, fj, Y = run_ttm(ctx, X, U, method=1)
+    q = np.arange(len(lengths))
+    np.testing.assert_array_equal(fi, q // J)
+    np.testing.assert_array_equal(fj, q % J)
+    at = 0
+    for f, c in enumerate(lengths):
+        t = X.vals[at:at + c, None] * U[idx[at:at + c, 2]]
+        at += c
+        seq = np.add.accumulate(np.concatenate([np.zeros((1, R)), t]), axis=0)[-1]
+        if c <= 128:
+            np.testing.assert_array_equal(Y[f], seq)
+        assert oracle.max_value_error(Y[f], seq, np.abs(t).sum(axis=0)) <= TOL
+    np.testing.assert_array_equal(run_ttm(ctx, X, U, method=1)[2], Y)
+
+
+def test_ttm_segments_of_64(ctx):
+    """A nonzero count whose segments hold 64: every fiber of 300."""
+    print("case: ttm segments of 64", flush=True)
+    dims, R = (20, 400, 300), 16
+    i, j, k = np.meshgrid(*(np.arange(d) for d in dims), indexing="ij")
+    idx = np.stack([i.ravel(), j.ravel(), k.ravel()], axis=1).astype(np.int32)
+    rng = np.random.default_rng(3)
+    X = gen.COO3(dims, idx, rng.uniform(-1, 1, len(idx)))
+    U = rng.uniform(-1, 1, (dims[2], R))
+    fi, fj, Y = run_ttm(ctx, X, U, method=1)
+    np.testing.assert_array_equal(fi, np.repeat(np.arange(20), 400))
+    np.testing.assert_array_equal(fj, np.tile(np.arange(400), 20))
+    V = X.vals.reshape(-1, 300)
+    exact = (V.astype(np.longdouble) @ U.astype(np.longdouble)).astype(np.float64)
+    assert oracle.max_value_error(Y.ravel(), exact.ravel(), (np.abs(V) @ np.abs(U)).ravel()) <= TOL
+
+
 @pytest.mark.parametrize("R", [16, 40])
 def test_ttm_long_fibers(ctx, R):
     """Fibers of 139-200 nonzeros: two 128-nonzero work items per fiber
@@ -352,6 +404,26 @@ def test_ttm_taco_hypersparse_factor(col_density):
     np.testing.assert_array_equal(gl, ol)
     Uz, _ = formats.dcsr_dense_and_mask(Ud)
     absY = np.einsum("ijk,kr->ijr", np.abs(dense(X)), np.abs(Uz))
+    assert oracle.max_value_error(gv, ov, absY[ok, oj, ol]) <= TOL
+
+
+@pytest.mark.parametrize("R", [16, 40])
+def test_ttm_masked_long_fibers(R):
+    """Stored columns of fibers over several segments: each is stored by one
+    of its parts only (U row k stores column k mod R, half the rows none)."""
+    print(f"case: ttm masked long fibers R={R}", flush=True)
+    X = gen.zipf_coo3((5, 6, 900), 20_000, (None, None, None), 18, 5, -1.0, 1.0)
+    k = np.arange(0, 900, 2)
+    Ud = formats.DCSR(900, R, k.astype(np.int32), np.arange(len(k) + 1, dtype=np.int32), (k % R).astype(np.int32),
+                      np.random.default_rng(18).uniform(-1, 1, len(k)))
+    At = taco.init_taco_tensor_COO([5, 6, R])
+    taco.ttm_compute(At, taco.csf_to_taco_tensor(formats.csf3_from_coo(X, (0, 2, 1))),
+                     taco.CC_to_taco_tensor(Ud, 900, R), 1)
+    gk, gj, gl, gv = taco.taco_coo(At)
+    ok, oj, ol, ov = oracle.ttm_hash_il(formats.csf3_from_coo(X, (0, 2, 1)), Ud, 5, 6, R)
+    for got, want in ((gk, ok), (gj, oj), (gl, ol)):
+        np.testing.assert_array_equal(got, want)
+    absY = np.einsum("ijk,kr->ijr", np.abs(dense(X)), np.abs(formats.dcsr_dense_and_mask(Ud)[0]))
     assert oracle.max_value_error(gv, ov, absY[ok, oj, ol]) <= TOL
 
 
