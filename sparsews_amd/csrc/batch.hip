@@ -16,14 +16,15 @@
 //   k_batch_gather     operands -> engine pools, indices rebased
 //   k_meta_clear, k_rowstat, device-sized scan, k_bin_offsets, k_binscatter
 //   numeric kernels of the wave / wave2 / block / block2 / wide paths
-//   (persistent grids; each reads its row count from the bin metadata; the
-//   block bins use the LDS bitmap kernel over each row's own column range
-//   when the engine bounds the request width by max_cols)
+//   (persistent grids; each reads its row count from the bin metadata; when
+//   the engine bounds the request width by max_cols the block bins use the
+//   LDS bitmap kernel over each row's own column range, and only count here)
 //   device-sized scan -> C_pos
 //   k_batch_req_meta   each request's nnz (and whether its output buffer holds it)
 //   k_batch_compact    rows into their request's output buffer when it has
 //                      one, into the engine's pools otherwise (columns
 //                      shifted back per row)
+//   k_row_bits         the counted rows, computed straight into that place
 //   k_batch_total, D2H of the batch nnz and of each request's nnz
 // No memset is recorded into the graph: clears are kernels.  The dense path
 // is not used in batches: the stacked column space is the sum of the
@@ -90,6 +91,7 @@ struct spws_batch {
   int64_t wide_slots = 0;
   int32_t wide_groups = 0;
   spws::PathParams pp{};
+  int cus = 0;
 };
 
 namespace spws {
@@ -273,6 +275,28 @@ __global__ __launch_bounds__(256) void k_batch_req_meta(const spws_batch_req* __
   }
 }
 
+// Where a batch row's entries go: its request's output buffer when it has one
+// that holds the request, else the engine's output pools; columns from the
+// request's own first column.
+struct BatchDst {
+  const int32_t* C_pos;
+  const int32_t* row_coloff;
+  const int32_t* row_req;
+  const spws_batch_req* reqs;
+  const int64_t* req_nnz;
+  int32_t* C_crd;
+  double* C_val;
+  __device__ RowOut operator()(int32_t i) const {
+    const int32_t dst = C_pos[i], shift = row_coloff[i], r = row_req[i];
+    const spws_batch_req& q = reqs[r];
+    if (q.out_pos && req_nnz[r] >= 0) {
+      const int32_t at = dst - C_pos[q.row0];
+      return {q.out_crd + at, q.out_val + at, shift};
+    }
+    return {C_crd + dst, C_val + dst, shift};
+  }
+};
+
 // Slot regions -> contiguous rows, a wavefront per row (k_compact's loop),
 // with each row written straight into its request's output buffer when it
 // has one that holds the request (row pointers rebased to the request's
@@ -287,7 +311,8 @@ __global__ __launch_bounds__(256) void k_batch_compact(const spws_batch_desc* __
                                                        const int32_t* __restrict__ row_req,
                                                        const spws_batch_req* __restrict__ reqs,
                                                        const int64_t* __restrict__ req_nnz,
-                                                       int32_t* __restrict__ C_crd, double* __restrict__ C_val) {
+                                                       int32_t* __restrict__ C_crd, double* __restrict__ C_val,
+                                                       DirectRows direct) {
   const int32_t m = desc->rows;
   const int lane = lane_id();
   const int32_t waves = gridDim.x * (blockDim.x / kWave);
@@ -309,6 +334,7 @@ __global__ __launch_bounds__(256) void k_batch_compact(const spws_batch_desc* __
         if (i == q.row0 + q.m - 1) q.out_pos[q.m] = dst + n - start;
       }
     }
+    if (direct(row_off[i + 1] - src)) continue;
     for (int32_t e0 = 0; e0 < n; e0 += kWave * kCompactUnroll) {
       int32_t c[kCompactUnroll];
       double v[kCompactUnroll];
@@ -384,30 +410,30 @@ static void enqueue_batch(spws_batch* b) {
   hipLaunchKernelGGL(k_binscatter, dim3(grows), dim3(256), 0, s, 0, m_dev, 1, row_ub, bmeta, bin_rows, row_nnz, b->pp);
   const unsigned gwave = (unsigned)std::min<int64_t>(c.max_rows, 8192);
   const unsigned gblk = (unsigned)std::min<int64_t>(c.max_rows, 1024);
-  // the block bins' row-per-workgroup kernel: a wider grid keeps more rows in flight
-  const unsigned gbin = (unsigned)std::min<int64_t>(c.max_rows, 8192);
   hipLaunchKernelGGL((k_row_wave<128, 1, true, kWaveRowsK>), dim3(gwave), dim3(64), 0, s, bin_rows, bmeta, (int)P_WAVE,
                      Ap, Ai, Ax, Bp, Bi, Bx, row_off, scrd, sval, row_nnz);
   hipLaunchKernelGGL((k_row_wave<512, 4, true>), dim3(gwave), dim3(64), 0, s, bin_rows, bmeta, (int)P_WAVE2, Ap, Ai,
                      Ax, Bp, Bi, Bx, row_off, scrd, sval, row_nnz);
-  if (c.max_cols > 0 && c.max_cols <= kBitmapCols) {
-    // every request is at most max_cols wide: LDS bitmap over each row's own column range
-    const int64_t v1 = std::min<int64_t>(b->pp.block_ub, c.max_cols), v2 = std::min<int64_t>(b->pp.block2_ub, c.max_cols);
-    hipLaunchKernelGGL((k_row_bitmap_rows<kBitmapRowsK, kBitmapItems1>), dim3(gbin), dim3(kBitmapBlock),
-                       bitmap_lds_bytes(c.max_cols, v1, true, kBitmapBlock), s,
-                       bin_rows, bmeta, (int)P_BLOCK, c.max_cols, Ap, Ai, Ax, Bp, Bi, Bx, row_off, scrd, sval, row_nnz,
-                       coloff, row_ncols);
-    hipLaunchKernelGGL((k_row_bitmap_rows<kBitmapRowsK, kBitmapItems2>), dim3(gbin), dim3(kBitmapBlock),
-                       bitmap_lds_bytes(c.max_cols, v2, true, kBitmapBlock), s,
-                       bin_rows, bmeta, (int)P_BLOCK2, c.max_cols, Ap, Ai, Ax, Bp, Bi, Bx, row_off, scrd, sval,
-                       row_nnz, coloff, row_ncols);
+  const bool bits = c.max_cols > 0 && c.max_cols <= kBitmapCols;
+  if (bits) {
+    // every request is at most max_cols wide: LDS bitmap over each row's own
+    // column range; the rows are counted here and computed in place below
+    const size_t lds = rowbits_lds_bytes(c.max_cols, 0, false);
+    hipLaunchKernelGGL((k_row_bits<kBits1Block, kBits1Items, false, true, NoDst>),
+                       dim3(rowbits_grid(b->cus, kBits1Block, lds, c.max_rows)), dim3(kBits1Block), lds, s, bin_rows,
+                       bmeta, (int)P_BLOCK, c.max_cols, 0, Ap, Ai, Ax, Bp, Bi, Bx, NoDst{}, row_nnz, coloff,
+                       row_ncols);
+    hipLaunchKernelGGL((k_row_bits<kBits2Block, kBits2Items, false, true, NoDst>),
+                       dim3(rowbits_grid(b->cus, kBits2Block, lds, c.max_rows)), dim3(kBits2Block), lds, s, bin_rows,
+                       bmeta, (int)P_BLOCK2, c.max_cols, 0, Ap, Ai, Ax, Bp, Bi, Bx, NoDst{}, row_nnz, coloff,
+                       row_ncols);
   } else {
     hipLaunchKernelGGL((k_row_block<2048, 1024, 256, true>), dim3(gblk), dim3(256), 0, s, bin_rows, bmeta,
                        (int)P_BLOCK, Ap, Ai, Ax, Bp, Bi, Bx, row_off, scrd, sval, row_nnz);
     hipLaunchKernelGGL((k_row_block<8192, 4096, 512, true>), dim3(gblk), dim3(512), 0, s, bin_rows, bmeta,
                        (int)P_BLOCK2, Ap, Ai, Ax, Bp, Bi, Bx, row_off, scrd, sval, row_nnz);
   }
-  if (c.max_cols > 0 && c.max_cols <= kBitmapCols) {
+  if (bits) {
     // products staged in the output pools, which the compaction fills later;
     // rows of at most acc_cap entries accumulate in LDS
     const size_t bm_bytes = bitmap_lds_bytes(c.max_cols, 0, false, kBitmapLongBlock);
@@ -427,7 +453,26 @@ static void enqueue_batch(spws_batch* b) {
                      Cp, req_nnz);
   hipLaunchKernelGGL(k_batch_compact, dim3((unsigned)std::min<int64_t>(div_up(c.max_rows, 4), 16384)), dim3(256), 0,
                      s, d_desc, row_off, Cp, scrd, sval, coloff, coloff + 2 * (size_t)c.max_rows, d_req, req_nnz, Ci,
-                     Cx);
+                     Cx, bits ? DirectRows{b->pp.wave2_ub, b->pp.block2_ub} : DirectRows{0, 0});
+  if (bits) {
+    // the block bins' rows at their place (the long rows staged their
+    // products in the pools: before this point only)
+    const BatchDst dst{Cp, coloff, coloff + 2 * (size_t)c.max_rows, d_req, req_nnz, Ci, Cx};
+    const int32_t v1 = std::min<int32_t>(b->pp.block_ub, c.max_cols);
+    const int32_t v2 = std::min<int32_t>(b->pp.block2_ub, c.max_cols);
+    const bool narrow = c.max_cols <= kBitsNarrow;
+    const size_t l1 = rowbits_lds_bytes(c.max_cols, v1, true), l2 = rowbits_lds_bytes(c.max_cols, v2, true);
+    hipLaunchKernelGGL((narrow ? k_row_bits<kBits1Block, kBits1Items, true, true, BatchDst>
+                               : k_row_bits<kBits1Block, kBits1Items, true, false, BatchDst>),
+                       dim3(rowbits_grid(b->cus, kBits1Block, l1, c.max_rows)),
+                       dim3(kBits1Block), l1, s, bin_rows, bmeta, (int)P_BLOCK, c.max_cols, v1, Ap, Ai, Ax, Bp, Bi,
+                       Bx, dst, row_nnz, coloff, row_ncols);
+    hipLaunchKernelGGL((narrow ? k_row_bits<kBits2Block, kBits2Items, true, true, BatchDst>
+                               : k_row_bits<kBits2Block, kBits2Items, true, false, BatchDst>),
+                       dim3(rowbits_grid(b->cus, kBits2Block, l2, c.max_rows)),
+                       dim3(kBits2Block), l2, s, bin_rows, bmeta, (int)P_BLOCK2, c.max_cols, v2, Ap, Ai, Ax, Bp, Bi,
+                       Bx, dst, row_nnz, coloff, row_ncols);
+  }
   hipLaunchKernelGGL(k_batch_total, dim3(1), dim3(64), 0, s, Cp, d_desc, (int64_t*)P(BP_TOTAL));
   (void)hipMemcpyAsync(b->h_total, P(BP_TOTAL), 8, hipMemcpyDeviceToHost, s);
   (void)hipMemcpyAsync(b->h_req_nnz, req_nnz, 8 * (size_t)c.max_requests, hipMemcpyDeviceToHost, s);
@@ -446,6 +491,7 @@ static void batch_release(spws_batch* b) {
 }
 
 static int batch_build(spws_batch* b) {
+  SPWS_HIP(hipDeviceGetAttribute(&b->cus, hipDeviceAttributeMultiprocessorCount, b->ctx->device));
   const spws_batch_caps& c = b->caps;
   const size_t rows = (size_t)c.max_rows, brows = (size_t)c.max_brows;
   const size_t annz = (size_t)c.max_annz, bnnz = (size_t)c.max_bnnz, ub = (size_t)c.max_products;

@@ -2,7 +2,9 @@
 // (spgemm_rowwise.hip) and the batched engine (batch.hip).  See
 // spgemm_rowwise.hip for the pipeline and the reference it follows.
 #pragma once
+#include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -202,14 +204,13 @@ __global__ __launch_bounds__(kRsBlock) void k_binscatter(int32_t m_host, const i
 // use all wavefronts.  Longer rows: each wavefront takes whole chunks.  Loop
 // bounds are wave-uniform, so the shuffles see every lane.
 
-template <bool kValues, class F>
+template <bool kValues, int kU = 4, class F>
 __device__ __forceinline__ void expand_products(int32_t a_beg, int32_t a_end, int32_t widx, int32_t nwaves,
                                                 const int32_t* __restrict__ Ai, const double* __restrict__ Ax,
                                                 const int32_t* __restrict__ Bp, const int32_t* __restrict__ Bi,
                                                 const double* __restrict__ Bx, F&& insert) {
   // kU strides of products are located and loaded before any is inserted,
   // so their B loads are in flight together
-  constexpr int kU = 4;
   const int lane = lane_id();
   // rows of at least two chunks per wavefront: each wavefront takes whole
   // chunks of its own (chunk widx, widx + nwaves, ...), so the chunks' load
@@ -274,15 +275,12 @@ __device__ __forceinline__ void expand_products(int32_t a_beg, int32_t a_end, in
 
 // The products of K rows gathered into registers: product g of row k (in
 // the order of expand_products) belongs to thread g % BLOCK as item
-// g / BLOCK.  A row's A entries are taken 64 at a time (kMultiChunk false:
-// the caller guarantees at most 64); with K > 1 each level of the first
-// chunk (A entries, B row bounds, B entries) is loaded for all K rows
-// together, so their load chains overlap.  Rows with take[k] false are
-// skipped (workgroup-uniform), and the caller guarantees that a taken row
-// has at most BLOCK * ITEMS products.  Unused items hold col = -1.  The
-// chunk loop costs registers: the block-bin kernel, whose occupancy
-// depends on them, takes single-chunk rows only.
-template <int BLOCK, int K, int ITEMS, bool kMultiChunk>
+// g / BLOCK.  A row's A entries are taken 64 at a time; with K > 1 each
+// level of the first chunk (A entries, B row bounds, B entries) is loaded for
+// all K rows together, so their load chains overlap.  Rows with take[k] false
+// are skipped (workgroup-uniform), and the caller guarantees that a taken row
+// has at most BLOCK * ITEMS products.  Unused items hold col = -1.
+template <int BLOCK, int K, int ITEMS>
 __device__ __forceinline__ void gather_rows_products(const bool (&take)[K], const int32_t (&a_beg)[K],
                                                      const int32_t (&a_end)[K], const int32_t* __restrict__ Ai,
                                                      const double* __restrict__ Ax, const int32_t* __restrict__ Bp,
@@ -320,8 +318,7 @@ __device__ __forceinline__ void gather_rows_products(const bool (&take)[K], cons
     }
     if (!take[k]) continue;
     int32_t base = 0;  // products of the row's earlier chunks
-    const int32_t c_end = kMultiChunk ? a_end[k] : min(a_end[k], a_beg[k] + kWave);
-    for (int32_t c = a_beg[k]; c < c_end; c += kWave) {
+    for (int32_t c = a_beg[k]; c < a_end[k]; c += kWave) {
       if (c != a_beg[k]) {  // later chunks: their A entries and B row bounds
         const int32_t p = c + lane;
         j[k] = -1;
@@ -494,7 +491,7 @@ __global__ __launch_bounds__(64) void k_row_wave(const int32_t* __restrict__ bin
     }
     int32_t pc[K][R];
     double pv[K][R];
-    gather_rows_products<kWave, K, R, true>(take, a_beg, a_end, Ai, Ax, Bp, Bi, Bx, pc, pv);
+    gather_rows_products<kWave, K, R>(take, a_beg, a_end, Ai, Ax, Bp, Bi, Bx, pc, pv);
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -1085,7 +1082,6 @@ __global__ __launch_bounds__(BLOCK) void k_row_block(const int32_t* __restrict__
 // row's columns lie in [row_colbase[i], row_colbase[i] + row_ncols[i]) (its
 // request's width), and the passes over the bitmap cover that range only.
 
-constexpr int kBitmapBlock = 256;
 constexpr size_t kLdsBudget = 156 * 1024;  // dynamic LDS a workgroup may take (of 160 KiB)
 constexpr int kBitmapLongBlock = 1024;  // rows beyond the block bins: 16 wavefronts per row
 constexpr int32_t kBitmapCols = 1 << 17;
@@ -1209,19 +1205,13 @@ __device__ __forceinline__ void bitmap_row(int32_t i, int32_t cb, int32_t w0, in
   __syncthreads();
 }
 
-template <bool kValues, bool kGlobal = false, int BLOCK = kBitmapBlock>
+// Symbolic rows beyond the block bins: the distinct columns counted.
+template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_row_bitmap(const int32_t* __restrict__ bin_rows,
                                                       const int32_t* __restrict__ bmeta, int path, int32_t ncols,
                                                       const int32_t* __restrict__ Ap, const int32_t* __restrict__ Ai,
-                                                      const double* __restrict__ Ax, const int32_t* __restrict__ Bp,
-                                                      const int32_t* __restrict__ Bi, const double* __restrict__ Bx,
-                                                      const int64_t* __restrict__ row_off,
-                                                      int32_t* __restrict__ slot_crd, double* __restrict__ slot_val,
-                                                      int32_t* __restrict__ row_nnz,
-                                                      const int32_t* __restrict__ row_colbase,
-                                                      const int32_t* __restrict__ row_ncols) {
-  // declared as double so the dynamic region (which follows the static
-  // arrays) starts 8-byte aligned: acc is updated with 64-bit LDS atomics
+                                                      const int32_t* __restrict__ Bp, const int32_t* __restrict__ Bi,
+                                                      int32_t* __restrict__ row_nnz) {
   extern __shared__ double bml_d[];
   __shared__ int32_t sh[BLOCK / kWave + 1];
   BitmapLds L;
@@ -1229,17 +1219,18 @@ __global__ __launch_bounds__(BLOCK) void k_row_bitmap(const int32_t* __restrict_
   const int wave = threadIdx.x / kWave;
   const int32_t count = bmeta[kMetaCount + path];
   const int32_t* rows = bin_rows + bmeta[kMetaOff + path];
+  int32_t w0, w1;
+  L.row_words<BLOCK>(ncols, &w0, &w1);
   for (int32_t r = blockIdx.x; r < count; r += gridDim.x) {
     const int32_t i = rows[r];
-    const int32_t cb = row_colbase ? row_colbase[i] : 0;
-    int32_t w0, w1;
-    L.row_words<BLOCK>(row_ncols ? row_ncols[i] : ncols, &w0, &w1);
     const int32_t a_beg = Ap[i], a_end = Ap[i + 1];
-    const int64_t off = kValues ? row_off[i] : 0;
-    bitmap_row<BLOCK, kValues, kGlobal>(
-        i, cb, w0, w1, off, 0, L, sh, slot_crd, slot_val, row_nnz,
-        [&](auto&& f) { expand_products<false>(a_beg, a_end, wave, BLOCK / kWave, Ai, Ax, Bp, Bi, Bx, f); },
-        [&](auto&& f) { expand_products<true>(a_beg, a_end, wave, BLOCK / kWave, Ai, Ax, Bp, Bi, Bx, f); });
+    bitmap_row<BLOCK, false, false>(
+        i, 0, w0, w1, 0, 0, L, sh, nullptr, nullptr, row_nnz,
+        [&](auto&& f) {
+          expand_products<false>(a_beg, a_end, wave, BLOCK / kWave, Ai, (const double*)nullptr, Bp, Bi,
+                                 (const double*)nullptr, f);
+        },
+        [](auto&&) {});
   }
 }
 
@@ -1321,88 +1312,347 @@ __global__ __launch_bounds__(BLOCK) void k_row_bitmap_staged(
   }
 }
 
-// register capacity of the two block bins (products per thread), rows per
-// step, and the largest grid of the numeric block-bin kernel.  The second
-// bin holds rows of up to kBlock2UbMax products but keeps 2048 of them in
-// registers, which keeps occupancy at the LDS limit.  One row per step:
-// two rows per step overlap their load chains but cost more occupancy
-// than they gain.
-constexpr int kBitmapItems1 = kBlockUbMax / kBitmapBlock;
-constexpr int kBitmapItems2 = 8;
-constexpr int kBitmapRowsK = 1;
-constexpr int kBitmapRowsGrid = 1 << 16;
+// ------------------------------------------------------------------ block-bin rows
+//
+// Rows of the block bins (at most kBitmapCols columns): a workgroup per row,
+// the grid's workgroups staying for many rows.  Products go through registers:
+// product p of a row belongs to thread p % 256 as item p / 256.
+//
+// While a row is worked on, the loads of the next ones are in flight, each
+// level of the chain row list -> row pointers -> A entries -> B row bounds ->
+// B entries one row further ahead, so a row costs its own work and not five
+// memory latencies.  A row of more than kBitsEntries A entries or
+// BLOCK * ITEMS products takes the plain expansion instead, one product per
+// lane at a time (more in flight there would cost every row its registers).
+//
+// A wavefront finds the A entry of each of its products with a max-scan over
+// marks at the entries' first products (12 instructions per 64 products; a
+// binary search over the lanes takes 42 and six dependent LDS round trips).
+// Every product writes its own column at its rank, so no pass walks the bits
+// of the bitmap.  65,536 rows of 2..64 entries squared (58,900 block rows,
+// 71M products): 640 us with one row per workgroup, searches and bit walks
+// (4,400 VALU instructions per row of 1,500 products), 465 us now (2,000; 4
+// wavefronts per SIMD by registers and LDS, LDS pipe about half busy).  Blocks
+// of 512 and 1,024 threads were slower (the A entries are scanned by every
+// wavefront), as were registers bounded below 120 (spills, each waited for).
+constexpr int kBits1Block = 256, kBits1Items = 4;  // threads and products per thread of the two bins
+constexpr int kBits2Block = 256, kBits2Items = 8;
+constexpr int kBitsEntries = 256;
+constexpr int32_t kBitsNarrow = 1 << 16;  // row widths whose columns are staged in 16 bits
 
-// Numeric block-bin rows, K rows per step of a grid-stride loop: the
-// products of every row with at most 64 A entries and at most
-// kBitmapBlock * ITEMS products are gathered into registers (pass 2 reads
-// no memory); the rows then go through the bitmap one after another.  Other
-// rows take the two-gather expansion.
-template <int K, int ITEMS>
-__global__ __launch_bounds__(kBitmapBlock) void k_row_bitmap_rows(
-    const int32_t* __restrict__ bin_rows, const int32_t* __restrict__ bmeta, int path, int32_t ncols,
-    const int32_t* __restrict__ Ap, const int32_t* __restrict__ Ai, const double* __restrict__ Ax,
-    const int32_t* __restrict__ Bp, const int32_t* __restrict__ Bi, const double* __restrict__ Bx,
-    const int64_t* __restrict__ row_off, int32_t* __restrict__ slot_crd, double* __restrict__ slot_val,
-    int32_t* __restrict__ row_nnz, const int32_t* __restrict__ row_colbase, const int32_t* __restrict__ row_ncols) {
-  extern __shared__ double bml_d[];
-  __shared__ int32_t sh[kBitmapBlock / kWave + 1];
-  BitmapLds L;
-  L.init<kBitmapBlock>(bml_d, ncols);
-  const int wave = threadIdx.x / kWave;
-  const int32_t count = bmeta[kMetaCount + path];
-  const int32_t* rows = bin_rows + bmeta[kMetaOff + path];
-  for (int32_t r0 = blockIdx.x * K; r0 < count; r0 += gridDim.x * K) {
-    int32_t i[K], cb[K], nc[K], a_beg[K], a_end[K];
-    int64_t off[K];
-    bool take[K];
+// LDS of a row: its bitmap in vectors of 128 columns, then (values) vcap
+// sums, the rank of each word's first column (16 bits) and vcap columns (16
+// bits below kBitsNarrow columns).
+__host__ __device__ constexpr int32_t rowbits_vecs(int32_t ncols) { return (ncols + 127) >> 7; }
+__host__ __device__ constexpr size_t rowbits_lds_bytes(int32_t ncols, int64_t vcap, bool values) {
+  const size_t nv = (size_t)rowbits_vecs(ncols);
+  return nv * 16 + (values ? nv * 8 + (size_t)vcap * (ncols <= kBitsNarrow ? 10 : 12) : 0);
+}
+
+// A row of the list as the pipeline carries it.
+struct RowAhead {
+  int32_t i, a_beg, a_end;  // uniform; i < 0: none
+  int32_t j;                // this lane's first A entry (-1: none), then its B row
+  int32_t bstart, blen;
+};
+
+// Items of the row in `r` (bounds of its first 64 entries loaded) for this
+// wavefront: columns (-1: none), B values and the positions of their A entries
+// in the row (a byte each), the loads left in flight.  `marks` is the
+// wavefront's own area of 64 * ITEMS bytes, zero on entry and on return.
+// Returns the row's products, or -1 when the row does not fit.
+template <int BLOCK, int ITEMS, bool kValues>
+__device__ __forceinline__ int32_t gather_marked(const RowAhead& r, uint8_t* __restrict__ marks,
+                                                 const int32_t* __restrict__ Ai, const int32_t* __restrict__ Bp,
+                                                 const int32_t* __restrict__ Bi, const double* __restrict__ Bx,
+                                                 int32_t (&col)[ITEMS], double (&bv)[ITEMS],
+                                                 uint32_t (&own)[(ITEMS + 3) / 4]) {
+  constexpr int kWaves = BLOCK / kWave;
+  static_assert(kBitsEntries <= 256, "positions of A entries in a byte");
+  const int lane = lane_id();
+  const int w = threadIdx.x / kWave;
 #pragma unroll
-    for (int k = 0; k < K; ++k) i[k] = r0 + k < count ? rows[r0 + k] : -1;
+  for (int u = 0; u < ITEMS; ++u) col[u] = -1;
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      a_beg[k] = a_end[k] = cb[k] = 0;
-      nc[k] = ncols;
-      off[k] = 0;
-      take[k] = false;
-      if (i[k] >= 0) {
-        a_beg[k] = Ap[i[k]];
-        a_end[k] = Ap[i[k] + 1];
-        off[k] = row_off[i[k]];
-        // the row's upper bound is its slot-region length
-        take[k] = row_off[i[k] + 1] - off[k] <= (int64_t)kBitmapBlock * ITEMS && a_end[k] - a_beg[k] <= kWave;
-        cb[k] = row_colbase ? row_colbase[i[k]] : 0;
-        if (row_ncols) nc[k] = row_ncols[i[k]];
+  for (int u = 0; u < (ITEMS + 3) / 4; ++u) own[u] = 0;
+  const int32_t na = r.a_end - r.a_beg;
+  if (na > kBitsEntries) return -1;
+  int32_t bstart = r.bstart, blen = r.blen, base = 0;
+  for (int32_t c = 0; c < na; c += kWave) {
+    if (c > 0) {
+      bstart = blen = 0;
+      if (c + lane < na) {
+        const int32_t j = Ai[r.a_beg + c + lane];
+        bstart = Bp[j];
+        blen = Bp[j + 1] - bstart;
       }
     }
-    int32_t pc[K][ITEMS];
-    double pv[K][ITEMS];
-    gather_rows_products<kBitmapBlock, K, ITEMS, false>(take, a_beg, a_end, Ai, Ax, Bp, Bi, Bx, pc, pv);
+    const int32_t incl = wave_incl_scan(blen);
+    const int32_t end = base + wave_last(incl);
+    if (end > BLOCK * ITEMS) return -1;  // uniform
+    const int32_t first = base + incl - blen;  // the entry's first product
+    const bool mine = blen > 0 && first / kWave % kWaves == w;
+    uint8_t* const my_mark = marks + first / BLOCK * kWave + first % kWave;
+    if (mine) *my_mark = (uint8_t)(lane + 1);
+    __builtin_amdgcn_wave_barrier();
+    const int32_t shifted = bstart - first;  // + product index = its B entry
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      if (i[k] < 0) continue;
-      int32_t w0, w1;
-      L.row_words<kBitmapBlock>(nc[k], &w0, &w1);
-      if (take[k]) {
-        bitmap_row<kBitmapBlock, true, false>(
-            i[k], cb[k], w0, w1, off[k], 0, L, sh, slot_crd, slot_val, row_nnz,
-            [&](auto&& f) {
-#pragma unroll
-              for (int u = 0; u < ITEMS; ++u)
-                if (pc[k][u] >= 0) f(pc[k][u], 0.0);
-            },
-            [&](auto&& f) {
-#pragma unroll
-              for (int u = 0; u < ITEMS; ++u)
-                if (pc[k][u] >= 0) f(pc[k][u], pv[k][u]);
-            });
-      } else {
-        const int32_t ab = a_beg[k], ae = a_end[k];
-        bitmap_row<kBitmapBlock, true, false>(
-            i[k], cb[k], w0, w1, off[k], 0, L, sh, slot_crd, slot_val, row_nnz,
-            [&](auto&& f) { expand_products<false>(ab, ae, wave, kBitmapBlock / kWave, Ai, Ax, Bp, Bi, Bx, f); },
-            [&](auto&& f) { expand_products<true>(ab, ae, wave, kBitmapBlock / kWave, Ai, Ax, Bp, Bi, Bx, f); });
+    for (int u = 0; u < ITEMS; ++u) {
+      const int32_t p0 = (u * kWaves + w) * kWave;
+      if (p0 >= end || p0 + kWave <= base) continue;  // uniform
+      // the last entry starting at or before the stride, then the marks inside
+      const uint64_t before = __ballot(blen > 0 && first <= p0);
+      const uint32_t mark = wave_incl_max((uint32_t)marks[u * kWave + lane]);
+      const int at = (int)max(mark, before ? (uint32_t)(kWave - __builtin_clzll(before)) : 1u) - 1;
+      const uint32_t kb = (uint32_t)(__shfl(shifted, at, kWave) + p0 + lane);
+      if (p0 + lane >= base && p0 + lane < end) {
+        col[u] = Bi[kb];
+        if (kValues) {
+          bv[u] = Bx[kb];
+          own[u / 4] |= (uint32_t)(c + at) << (8 * (u % 4));
+        }
       }
     }
+    __builtin_amdgcn_wave_barrier();
+    if (mine) *my_mark = 0;
+    base = end;
   }
+  return base;
+}
+
+// kValues: the rows' columns and sums to where dst says; else only row_nnz.
+// Dst: dst(i) -> {columns, values, shift subtracted from the columns}.
+struct RowOut {
+  int32_t* crd;
+  double* val;
+  int32_t shift;
+};
+
+struct SlotDst {  // the row's slot region
+  const int64_t* row_off;
+  int32_t* crd;
+  double* val;
+  __device__ RowOut operator()(int32_t i) const { return {crd + row_off[i], val + row_off[i], 0}; }
+};
+
+struct FinalDst {  // the row's place in C
+  const int32_t* C_pos;
+  int32_t* crd;
+  double* val;
+  __device__ RowOut operator()(int32_t i) const { return {crd + C_pos[i], val + C_pos[i], 0}; }
+};
+
+struct NoDst {
+  __device__ RowOut operator()(int32_t) const { return {nullptr, nullptr, 0}; }
+};
+
+// Waits for every vector memory operation issued so far.
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }  // vmcnt(0) alone
+
+template <int BLOCK, int ITEMS, bool kValues, bool kNarrow, class Dst>
+__global__ __launch_bounds__(BLOCK, !kValues ? 7 : ITEMS <= 4 ? 5 : 4) void k_row_bits(
+    const int32_t* __restrict__ bin_rows, const int32_t* __restrict__ bmeta, int path, int32_t ncols, int32_t vcap,
+    const int32_t* __restrict__ Ap, const int32_t* __restrict__ Ai, const double* __restrict__ Ax,
+    const int32_t* __restrict__ Bp, const int32_t* __restrict__ Bi, const double* __restrict__ Bx, Dst dst,
+    int32_t* __restrict__ row_nnz, const int32_t* __restrict__ row_colbase, const int32_t* __restrict__ row_ncols) {
+  constexpr int kWaves = BLOCK / kWave;
+  extern __shared__ __align__(16) uint4 rowbits_lds[];
+  __shared__ uint8_t s_marks[kWaves][ITEMS * kWave];
+  __shared__ int32_t s_tot[kWaves];
+  __shared__ int32_t s_new[2];
+  const int32_t nvec = rowbits_vecs(ncols);
+  uint4* const bm4 = rowbits_lds;
+  uint32_t* const bm = reinterpret_cast<uint32_t*>(bm4);
+  double* const acc = reinterpret_cast<double*>(bm4 + nvec);
+  uint16_t* const pre = reinterpret_cast<uint16_t*>(acc + vcap);
+  using ListT = std::conditional_t<kNarrow, uint16_t, int32_t>;  // columns from the row's first
+  ListT* const list = reinterpret_cast<ListT*>(pre + 4 * (size_t)nvec);
+  const int lane = lane_id();
+  const int w = threadIdx.x / kWave;
+  const int t = threadIdx.x;
+  // the bitmap and the marks are zero between rows
+  for (int32_t v = t; v < nvec; v += BLOCK) bm4[v] = make_uint4(0, 0, 0, 0);
+  for (int e = lane; e < ITEMS * kWave; e += kWave) s_marks[w][e] = 0;
+  if (t < 2) s_new[t] = 0;
+  __syncthreads();
+
+  const int32_t count = bmeta[kMetaCount + path];
+  const int32_t* const rows = bin_rows + bmeta[kMetaOff + path];
+  const int32_t step = gridDim.x;
+  const auto row_at = [&](int64_t r) -> int32_t { return r < count ? rows[r] : -1; };
+  const auto bounds = [&](RowAhead& x) {
+    x.a_beg = x.a_end = 0;
+    if (x.i >= 0) {
+      x.a_beg = Ap[x.i];
+      x.a_end = Ap[x.i + 1];
+    }
+  };
+  const auto entries = [&](RowAhead& x) {
+    x.j = x.a_beg + lane < x.a_end ? Ai[x.a_beg + lane] : -1;
+  };
+  const auto brows = [&](RowAhead& x) {
+    x.bstart = x.blen = 0;
+    if (x.j >= 0) {
+      x.bstart = Bp[x.j];
+      x.blen = Bp[x.j + 1] - x.bstart;
+    }
+  };
+  int64_t r = blockIdx.x;
+  if (r >= count) return;  // uniform
+  RowAhead x0, x1, x2;
+  x0.i = row_at(r);
+  x1.i = row_at(r + step);
+  x2.i = row_at(r + 2 * (int64_t)step);
+  bounds(x0);
+  bounds(x1);
+  entries(x0);
+  brows(x0);
+  entries(x1);
+  int32_t col[ITEMS];
+  double bv[ITEMS];
+  uint32_t own[(ITEMS + 3) / 4];
+  int32_t total = gather_marked<BLOCK, ITEMS, kValues>(x0, s_marks[w], Ai, Bp, Bi, Bx, col, bv, own);
+  int parity = 0;
+  for (; r < count; r += step, parity ^= 1) {
+    // further rows: one level of loads each
+    brows(x1);
+    bounds(x2);
+    const int32_t i3 = row_at(r + 3 * (int64_t)step);
+    const int32_t i = x0.i;
+    const int32_t cb = row_colbase ? row_colbase[i] : 0;
+    const int32_t nv = rowbits_vecs(row_ncols ? row_ncols[i] : ncols);  // vectors of this row
+    const int32_t a_beg = x0.a_beg, a_end = x0.a_end;
+    const bool taken = total >= 0;  // uniform
+    if constexpr (!kValues) {
+      int32_t fresh = 0;
+      const auto set = [&](int32_t c) {
+        const uint32_t cc = (uint32_t)(c - cb), bit = 1u << (cc & 31);
+        return (atomicOr(&bm[cc >> 5], bit) & bit) == 0;
+      };
+      if (taken) {
+#pragma unroll
+        for (int u = 0; u < ITEMS; ++u)
+          if (col[u] >= 0) fresh += set(col[u]) ? 1 : 0;
+      } else {
+        expand_products<false, 1>(a_beg, a_end, w, kWaves, Ai, Ax, Bp, Bi, Bx,
+                                  [&](int32_t c, double) { fresh += set(c) ? 1 : 0; });
+      }
+      fresh = wave_sum(fresh);
+      if (lane == 0) atomicAdd(&s_new[parity], fresh);
+      __syncthreads();
+      if (t == 0) {
+        row_nnz[i] = s_new[parity];
+        s_new[parity ^ 1] = 0;
+      }
+      // the words this row set are cleared again
+      if (taken) {
+#pragma unroll
+        for (int u = 0; u < ITEMS; ++u)
+          if (col[u] >= 0) bm[(uint32_t)(col[u] - cb) >> 5] = 0u;
+      } else {
+        for (int32_t v = t; v < nv; v += BLOCK) bm4[v] = make_uint4(0, 0, 0, 0);
+      }
+      entries(x2);
+      total = gather_marked<BLOCK, ITEMS, kValues>(x1, s_marks[w], Ai, Bp, Bi, Bx, col, bv, own);
+      __syncthreads();
+    } else {
+      const RowOut out = dst(i);
+      const int32_t add_col = cb - out.shift;
+      if (taken) {
+#pragma unroll
+        for (int u = 0; u < ITEMS; ++u)
+          if (col[u] >= 0) {
+            const uint32_t cc = (uint32_t)(col[u] - cb);
+            atomicOr(&bm[cc >> 5], 1u << (cc & 31));
+          }
+      } else {
+        expand_products<false, 1>(a_beg, a_end, w, kWaves, Ai, Ax, Bp, Bi, Bx, [&](int32_t c, double) {
+          const uint32_t cc = (uint32_t)(c - cb);
+          atomicOr(&bm[cc >> 5], 1u << (cc & 31));
+        });
+      }
+      __syncthreads();
+      // ranks: each thread its consecutive vectors
+      const int32_t per = (nv + BLOCK - 1) / BLOCK;
+      const int32_t v0 = min(t * per, nv), v1 = min(v0 + per, nv);
+      int32_t c = 0;
+      for (int32_t v = v0; v < v1; ++v) {
+        const uint4 q = bm4[v];
+        c += __popc(q.x) + __popc(q.y) + __popc(q.z) + __popc(q.w);
+      }
+      const int32_t incl = wave_incl_scan(c);
+      if (lane == kWave - 1) s_tot[w] = incl;
+      __syncthreads();
+      int32_t run = incl - c, nnz = 0;
+#pragma unroll
+      for (int q = 0; q < kWaves; ++q) {
+        if (q < w) run += s_tot[q];
+        nnz += s_tot[q];
+      }
+      for (int32_t v = v0; v < v1; ++v) {
+        const uint4 q = bm4[v];
+        const int32_t p1 = run + __popc(q.x), p2 = p1 + __popc(q.y), p3 = p2 + __popc(q.z);
+        reinterpret_cast<uint2*>(pre)[v] =
+            make_uint2((uint32_t)run | ((uint32_t)p1 << 16), (uint32_t)p2 | ((uint32_t)p3 << 16));
+        run = p3 + __popc(q.w);
+      }
+      for (int32_t e = t; e < nnz; e += BLOCK) acc[e] = 0.0;
+      entries(x2);
+      __syncthreads();
+      const auto add = [&](int32_t c2, double v) {
+        const uint32_t cc = (uint32_t)(c2 - cb);
+        const uint32_t word = cc >> 5;
+        const int32_t rank = (int32_t)pre[word] + __popc(bm[word] & ((1u << (cc & 31)) - 1u));
+        atomicAdd(&acc[rank], v);
+        list[rank] = (ListT)cc;
+      };
+      if (taken) {
+        double av[ITEMS];
+#pragma unroll
+        for (int u = 0; u < ITEMS; ++u)
+          if (col[u] >= 0) av[u] = Ax[a_beg + (int32_t)((own[u / 4] >> (8 * (u % 4))) & 0xFFu)];
+#pragma unroll
+        for (int u = 0; u < ITEMS; ++u)
+          if (col[u] >= 0) add(col[u], av[u] * bv[u]);
+      } else {
+        expand_products<true, 1>(a_beg, a_end, w, kWaves, Ai, Ax, Bp, Bi, Bx, add);
+      }
+      if (t == 0) row_nnz[i] = nnz;
+      total = gather_marked<BLOCK, ITEMS, kValues>(x1, s_marks[w], Ai, Bp, Bi, Bx, col, bv, own);
+      __syncthreads();
+      // One counter tracks loads and stores in order, so the next row's loads,
+      // issued above, are waited for without the stores below only if the
+      // number of these is known: a row from registers stores every item, past
+      // its end its last entry again; any other row waits for its loads first.
+      if (taken) {
+#pragma unroll
+        for (int u = 0; u < ITEMS; ++u) {
+          const int32_t e = min(u * BLOCK + t, nnz - 1);
+          out.crd[e] = (int32_t)list[e] + add_col;
+          out.val[e] = acc[e];
+        }
+      } else {
+        wait_loads();
+        for (int32_t e = t; e < nnz; e += BLOCK) {
+          out.crd[e] = (int32_t)list[e] + add_col;
+          out.val[e] = acc[e];
+        }
+      }
+      for (int32_t v = v0; v < v1; ++v) bm4[v] = make_uint4(0, 0, 0, 0);
+      __syncthreads();
+    }
+    x0 = x1;
+    x1 = x2;
+    x2.i = i3;
+  }
+}
+
+// Workgroups of k_row_bits that stay on the chip: LDS and eight wavefronts per
+// SIMD are the limits.
+inline unsigned rowbits_grid(int cus, int block, size_t lds_bytes, int64_t rows) {
+  const int64_t per_cu =
+      std::max<int64_t>(1, std::min<int64_t>(2048 / block, (160 * 1024) / (int64_t)(lds_bytes + 2304)));
+  return (unsigned)std::max<int64_t>(1, std::min<int64_t>(rows, per_cu * cus));
 }
 
 // ------------------------------------------------------------------ dense accumulator kernel
@@ -1640,6 +1890,13 @@ __global__ __launch_bounds__(kWideBlock) void k_row_wide(const int32_t* __restri
 
 constexpr int kCompactUnroll = 8;
 
+// Rows whose upper bound lies in (lo, hi] are in C already (written by
+// k_row_bits at their place) and are not copied; lo = hi: none.
+struct DirectRows {
+  int64_t lo, hi;
+  __device__ bool operator()(int64_t ub) const { return ub > lo && ub <= hi; }
+};
+
 // (the batch engine compacts with its own kernel, which writes into request
 // output buffers, so this one is unused there)
 [[maybe_unused]] __global__ __launch_bounds__(256) void k_compact(int32_t m_host, const int32_t* __restrict__ m_dev,
@@ -1648,7 +1905,8 @@ constexpr int kCompactUnroll = 8;
                                                  const int32_t* __restrict__ slot_crd,
                                                  const double* __restrict__ slot_val,
                                                  const int32_t* __restrict__ row_coloff, int32_t* __restrict__ C_crd,
-                                                 double* __restrict__ C_val, int32_t* __restrict__ meta_zero) {
+                                                 double* __restrict__ C_val, int32_t* __restrict__ meta_zero,
+                                                 DirectRows direct) {
   // the product's metadata block, read by the host before this launch, is
   // left zero for the next product
   if (meta_zero && blockIdx.x == 0 && threadIdx.x < kMetaBlockInts) meta_zero[threadIdx.x] = 0;
@@ -1659,6 +1917,7 @@ constexpr int kCompactUnroll = 8;
     const int32_t dst = C_pos[i];
     const int32_t n = C_pos[i + 1] - dst;
     const int64_t src = row_off[i];
+    if (direct(row_off[i + 1] - src)) continue;
     const int32_t shift = row_coloff ? row_coloff[i] : 0;
     // kCompactUnroll strides loaded before any is stored: the copy is
     // bandwidth-bound, not bound by one load's latency per stride

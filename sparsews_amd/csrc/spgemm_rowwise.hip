@@ -22,10 +22,11 @@
 //                         (2*ub slots), LDS atomicCAS keys + ds_add_f64
 //                         values, register bitonic sort across the wavefront;
 //        block  / block2  one workgroup per row: with at most 2^17 columns,
-//                         the row's products gathered once into registers,
 //                         an LDS bitmap of the columns (rank = popcount
 //                         prefix) and ds_add_f64 at each column's rank, no
-//                         sort; wider outputs use an LDS table and an LDS
+//                         sort; with many such rows they are only counted
+//                         here, and computed at their place in C after
+//                         step 5.  Wider outputs use an LDS table and an LDS
 //                         bitonic sort;
 //        dense / wide     longer rows: with at most 2^17 columns, the column
 //                         bitmap with the products staged in the output
@@ -51,6 +52,10 @@
 namespace spws {
 
 // ------------------------------------------------------------------ host driver
+
+// least products in the block bins for their rows to be counted first and
+// computed in place (see rowwise_run)
+constexpr int64_t kDirectProducts = 4 << 20;
 
 static int validate_tuning(const spws_rowwise_tuning& t) {
   SPWS_REQUIRE(t.wave_ub >= 1 && t.wave_ub <= kWaveUbMax, SPWS_ERR_INVALID, "wave_ub must be in [1, %d]",
@@ -303,32 +308,62 @@ static int rowwise_run(spws_ctx* ctx, int32_t m, int32_t kdim, int32_t n, const 
                 0, rows, bmeta, (int)P_WAVE2, Ap, Ai, Ax, Bp, Bi, Bx, roff, scrd, sval, rnnz, 0);
   }
   // block bins: the LDS bitmap kernel while all columns fit the bitmap, else
-  // the LDS hash table and bitonic sort
-  for (int path : {(int)P_BLOCK, (int)P_BLOCK2}) {
-    if (!counts[path]) continue;
-    if (n <= kBitmapCols) {
-      const int64_t vcap = std::min<int64_t>(maxub[path], n);
-      const unsigned lds = (unsigned)bitmap_lds_bytes(n, vcap, kValues, kBitmapBlock);
-      const unsigned grid_k = grid_for(div_up(counts[path], kBitmapRowsK), kBitmapRowsGrid);
-      if (!kValues)
-        SPWS_LAUNCH(ctx, "row_bitmap", (k_row_bitmap<false>), dim3(grid_for(counts[path], 1 << 16)),
-                    dim3(kBitmapBlock), lds, rows, bmeta, path, n, Ap, Ai, Ax, Bp, Bi, Bx, roff, scrd, sval, rnnz,
-                    (const int32_t*)nullptr, (const int32_t*)nullptr);
+  // the LDS hash table and bitonic sort.  With enough products in them the
+  // bitmap's rows are counted first and, once C_pos is known, computed into
+  // their place in C: the count reads 4 bytes per product again, mostly from
+  // the caches, where slots and their compaction move 24 bytes per entry
+  // through HBM: 140 us for 71M products against 380 us.  Below 4M products
+  // the copy is cheaper than two more launches.
+  int cus = 0;
+  SPWS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+  const bool bits = n <= kBitmapCols;
+  const bool direct = kValues && bits && t.force_path < 0 &&
+                      counts[P_BLOCK] * (int64_t)(t.wave2_ub + 1) + counts[P_BLOCK2] * (int64_t)(t.block_ub + 1) >=
+                          kDirectProducts;
+  enum { kCountRows, kSlotRows, kFinalRows };
+  auto block_rows = [&](int what) -> int {
+    for (int path : {(int)P_BLOCK, (int)P_BLOCK2}) {
+      if (!counts[path]) continue;
+      const int32_t vcap = what == kCountRows ? 0 : (int32_t)std::min<int64_t>(maxub[path], n);
+      const size_t lds = rowbits_lds_bytes(n, vcap, what != kCountRows);
+      const unsigned block = path == P_BLOCK ? kBits1Block : kBits2Block;
+      const unsigned grid = rowbits_grid(cus, block, lds, counts[path]);
+#define SPWS_ROW_BITS(NAME, BIN, VALUES, DST, ...)                                                                \
+  do {                                                                                                            \
+    if (VALUES && n > kBitsNarrow) SPWS_ROW_BITS_W(NAME, BIN, VALUES, false, DST, __VA_ARGS__);                   \
+    else SPWS_ROW_BITS_W(NAME, BIN, VALUES, true, DST, __VA_ARGS__);                                              \
+  } while (0)
+#define SPWS_ROW_BITS_W(NAME, BIN, VALUES, NARROW, DST, ...)                                                      \
+  SPWS_LAUNCH(ctx, NAME, (k_row_bits<kBits##BIN##Block, kBits##BIN##Items, VALUES, NARROW, DST>), dim3(grid), dim3(block),  \
+              (unsigned)lds, rows, bmeta, path, n, vcap, Ap, Ai, Ax, Bp, Bi, Bx, DST{__VA_ARGS__}, rnnz, (const int32_t*)nullptr,      \
+              (const int32_t*)nullptr)
+      if (what == kCountRows && path == P_BLOCK) SPWS_ROW_BITS("row_count", 1, false, NoDst);
+      else if (what == kCountRows) SPWS_ROW_BITS("row_count", 2, false, NoDst);
+      else if (what == kSlotRows && path == P_BLOCK)
+        SPWS_ROW_BITS("row_bitmap", 1, true, SlotDst, roff, scrd, sval);
+      else if (what == kSlotRows) SPWS_ROW_BITS("row_bitmap", 2, true, SlotDst, roff, scrd, sval);
       else if (path == P_BLOCK)
-        SPWS_LAUNCH(ctx, "row_bitmap", (k_row_bitmap_rows<kBitmapRowsK, kBitmapItems1>), dim3(grid_k),
-                    dim3(kBitmapBlock), lds, rows, bmeta, path, n, Ap, Ai, Ax, Bp, Bi, Bx, roff, scrd, sval, rnnz,
-                    (const int32_t*)nullptr, (const int32_t*)nullptr);
+        SPWS_ROW_BITS("row_bitmap", 1, true, FinalDst, ctx->out_pos.as<int32_t>(),
+                      ctx->out_crd.as<int32_t>(), ctx->out_val.as<double>());
       else
-        SPWS_LAUNCH(ctx, "row_bitmap", (k_row_bitmap_rows<kBitmapRowsK, kBitmapItems2>), dim3(grid_k),
-                    dim3(kBitmapBlock), lds, rows, bmeta, path, n, Ap, Ai, Ax, Bp, Bi, Bx, roff, scrd, sval, rnnz,
-                    (const int32_t*)nullptr, (const int32_t*)nullptr);
-    } else if (path == P_BLOCK) {
-      SPWS_LAUNCH(ctx, "row_block", (k_row_block<2048, 1024, 256, kValues>), dim3(grid_for(counts[path], 1 << 16)),
-                  dim3(256), 0, rows, bmeta, path, Ap, Ai, Ax, Bp, Bi, Bx, roff, scrd, sval, rnnz);
-    } else {
-      SPWS_LAUNCH(ctx, "row_block", (k_row_block<8192, 4096, 512, kValues>), dim3(grid_for(counts[path], 1 << 16)),
-                  dim3(512), 0, rows, bmeta, path, Ap, Ai, Ax, Bp, Bi, Bx, roff, scrd, sval, rnnz);
+        SPWS_ROW_BITS("row_bitmap", 2, true, FinalDst, ctx->out_pos.as<int32_t>(),
+                      ctx->out_crd.as<int32_t>(), ctx->out_val.as<double>());
+#undef SPWS_ROW_BITS
+#undef SPWS_ROW_BITS_W
     }
+    return SPWS_OK;
+  };
+  if (bits) {
+    if ((rc = block_rows(!kValues || direct ? kCountRows : kSlotRows))) return rc;
+  } else {
+    if (counts[P_BLOCK])
+      SPWS_LAUNCH(ctx, "row_block", (k_row_block<2048, 1024, 256, kValues>),
+                  dim3(grid_for(counts[P_BLOCK], 1 << 16)), dim3(256), 0, rows, bmeta, (int)P_BLOCK, Ap, Ai, Ax, Bp,
+                  Bi, Bx, roff, scrd, sval, rnnz);
+    if (counts[P_BLOCK2])
+      SPWS_LAUNCH(ctx, "row_block", (k_row_block<8192, 4096, 512, kValues>),
+                  dim3(grid_for(counts[P_BLOCK2], 1 << 16)), dim3(512), 0, rows, bmeta, (int)P_BLOCK2, Ap, Ai, Ax, Bp,
+                  Bi, Bx, roff, scrd, sval, rnnz);
   }
   // rows longer than the block bins: while the columns fit the LDS bitmap,
   // the bitmap kernel accumulating in the rows' slot regions replaces both
@@ -348,10 +383,9 @@ static int rowwise_run(spws_ctx* ctx, int32_t m, int32_t kdim, int32_t n, const 
                     Bx, roff, scrd, sval, rnnz, (const int32_t*)nullptr, (const int32_t*)nullptr,
                     ctx->out_crd.as<int32_t>(), ctx->out_val.as<double>(), acc_cap);
       else
-        SPWS_LAUNCH(ctx, "row_bitmap_long", (k_row_bitmap<false, true, kBitmapLongBlock>),
-                    dim3(grid_for(counts[path], 4096)), dim3(kBitmapLongBlock),
-                    bitmap_lds_bytes(n, 0, false, kBitmapLongBlock), rows, bmeta, path, n, Ap, Ai, Ax, Bp, Bi, Bx,
-                    roff, scrd, sval, rnnz, (const int32_t*)nullptr, (const int32_t*)nullptr);
+        SPWS_LAUNCH(ctx, "row_bitmap_long", k_row_bitmap<kBitmapLongBlock>, dim3(grid_for(counts[path], 4096)),
+                    dim3(kBitmapLongBlock), bitmap_lds_bytes(n, 0, false, kBitmapLongBlock), rows, bmeta, path, n, Ap,
+                    Ai, Bp, Bi, rnnz);
       counts[path] = 0;
     }
   }
@@ -387,11 +421,14 @@ static int rowwise_run(spws_ctx* ctx, int32_t m, int32_t kdim, int32_t n, const 
   }
   rc = exclusive_scan<int32_t, int32_t>(ctx, rnnz, ctx->out_pos.as<int32_t>(), m);
   if (rc) return rc;
+  // (the long rows staged their products in C's arrays: before this point only)
+  if (direct && (rc = block_rows(kFinalRows))) return rc;
   if (kValues && m > 0) {
     unsigned g = (unsigned)div_up(m, 4);
     if (g > 65536) g = 65536;
     SPWS_LAUNCH(ctx, "compact", k_compact, dim3(g), dim3(256), 0, m, nullptr, roff, ctx->out_pos.as<int32_t>(), scrd,
-                sval, nullptr, ctx->out_crd.as<int32_t>(), ctx->out_val.as<double>(), bmeta);
+                sval, nullptr, ctx->out_crd.as<int32_t>(), ctx->out_val.as<double>(), bmeta,
+                direct ? DirectRows{t.wave2_ub, t.block2_ub} : DirectRows{0, 0});
   }
   SPWS_HIP(hipMemcpyAsync(h32, ctx->out_pos.as<int32_t>() + m, 4, hipMemcpyDeviceToHost, s));
   SPWS_HIP(hipStreamSynchronize(s));

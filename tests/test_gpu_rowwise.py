@@ -296,6 +296,46 @@ def test_rows_of_many_a_entries(ctx, a_len, b_len, ncols, path):
     np.testing.assert_array_equal(spgemm_rowwise_symbolic(ctx, dA, dB), C.pos)
 
 
+# (B rows of 45 entries, B rows of 1) that a row of each kind takes
+ROW_KINDS = [
+    (30, 0),    # 1,350 products, the bulk: second block bin, from registers
+    (20, 236),  # 256 A entries: four chunks, from registers
+    (20, 256),  # 276 A entries: plain expansion
+    (45, 0),    # 2,025 products: the registers' edge
+    (50, 0),    # 2,250 products: plain expansion
+    (10, 0), (1, 255), (0, 257), (1, 256),  # first block bin, both ways
+    (3, 0), (1, 0), (0, 0), (0, 60),  # wavefront bins, empty rows
+    (100, 0),   # long rows
+]
+
+
+@pytest.mark.parametrize("bulk", [4200, 300])
+@pytest.mark.parametrize("ncols", [700, 65_536, 65_537, 131_072])
+def test_block_rows_in_place(ctx, ncols, bulk):
+    """Every kind of row in one product, with enough products in the block
+    bins (bulk 4200) for their rows to be counted first and computed at their
+    place in C, and without (300: slots and compaction); column lists of 16
+    and of 32 bits; twice, the second time on used buffers."""
+    print(f"case: block rows in place ncols={ncols} bulk={bulk}", flush=True)
+    rng = np.random.default_rng(ncols + bulk)
+    B = random_csr(2000, ncols, np.repeat([45, 1], 1000), 70, 1)
+    B.crd[B.pos[1000]], B.crd[B.pos[1001]] = 0, ncols - 1
+    kinds = np.repeat(np.arange(len(ROW_KINDS)), [bulk] + [12] * (len(ROW_KINDS) - 1))
+    rng.shuffle(kinds)
+    rows = []
+    for kind in kinds:
+        long, short = ROW_KINDS[kind]
+        rows.append(np.sort(np.concatenate([rng.permutation(1000)[:long], 1000 + rng.permutation(1000)[:short]])))
+    pos = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    crd = np.concatenate(rows).astype(np.int32)
+    A = CSR(len(rows), 2000, pos, crd, rng.uniform(-1, 1, len(crd)))
+    dA, dB = DeviceCSR.upload(ctx, A), DeviceCSR.upload(ctx, B)
+    for _ in range(2):
+        check(spgemm_rowwise(ctx, dA, dB).download(), A, B)
+    G = oracle.spgemm_gustavson(A, B)
+    np.testing.assert_array_equal(spgemm_rowwise_symbolic(ctx, dA, dB), G.pos)
+
+
 @pytest.mark.parametrize("every,path", [(10, 0), (2, 1)])
 def test_wave_bins_with_many_a_entries(ctx, every, path):
     """Rows of 300 A entries whose B rows are mostly empty: at most 64 (or
