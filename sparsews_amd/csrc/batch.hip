@@ -335,26 +335,7 @@ __global__ __launch_bounds__(256) void k_batch_compact(const spws_batch_desc* __
       }
     }
     if (direct(row_off[i + 1] - src)) continue;
-    for (int32_t e0 = 0; e0 < n; e0 += kWave * kCompactUnroll) {
-      int32_t c[kCompactUnroll];
-      double v[kCompactUnroll];
-#pragma unroll
-      for (int u = 0; u < kCompactUnroll; ++u) {
-        const int32_t e = e0 + u * kWave + lane;
-        if (e < n) {
-          c[u] = slot_crd[src + e];
-          v[u] = slot_val[src + e];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < kCompactUnroll; ++u) {
-        const int32_t e = e0 + u * kWave + lane;
-        if (e < n) {
-          oc[e] = c[u] - shift;
-          ov[e] = v[u];
-        }
-      }
-    }
+    compact_entries(lane, kWave, n, shift, slot_crd + src, slot_val + src, oc, ov);
   }
 }
 
@@ -439,7 +420,7 @@ static void enqueue_batch(spws_batch* b) {
     const size_t bm_bytes = bitmap_lds_bytes(c.max_cols, 0, false, kBitmapLongBlock);
     const int32_t acc_cap = (int32_t)std::min<int64_t>(c.max_cols, (int64_t)((kLdsBudget - bm_bytes) / 8));
     hipLaunchKernelGGL(k_row_bitmap_staged<kBitmapLongBlock>, dim3(gblk), dim3(kBitmapLongBlock),
-                       bitmap_lds_bytes(c.max_cols, acc_cap, true, kBitmapLongBlock), s, bin_rows, bmeta,
+                       bitmap_lds_bytes(c.max_cols, std::max(acc_cap, kLongAccMin), true, kBitmapLongBlock), s, bin_rows, bmeta,
                        (int)P_WIDE, c.max_cols, Ap, Ai, Ax, Bp, Bi, Bx, row_off, scrd, sval, row_nnz, coloff,
                        row_ncols, Ci, Cx, acc_cap);
   } else {

@@ -150,6 +150,17 @@ void prof_collect(spws_ctx* ctx);
     ::spws::prof_end(ctx, name, e0__);                                        \
   } while (0)
 
+// Launches inside the scope go to stream s (when not null) instead of the
+// context's stream, timing included.
+struct StreamScope {
+  spws_ctx* ctx;
+  hipStream_t saved;
+  StreamScope(spws_ctx* c, hipStream_t s) : ctx(c), saved(c->stream) {
+    if (s) c->stream = s;
+  }
+  ~StreamScope() { ctx->stream = saved; }
+};
+
 // ---------------------------------------------------------------- scan
 
 // Exclusive prefix sum of n values into out[0..n]; out[n] receives the total.

@@ -1235,15 +1235,28 @@ __global__ __launch_bounds__(BLOCK) void k_row_bitmap(const int32_t* __restrict_
 }
 
 // Numeric rows beyond the block bins (at most kBitmapCols columns): pass 1
-// gathers every product once, sets its column bit and stages (column,
-// value) in the row's region [off, off + ub) of a scratch pair (the final
-// output arrays, unused until the compaction), each wavefront taking slots
-// from an LDS cursor; pass 2 reads the staged products back coalesced
-// instead of gathering B again (B rows of power-law inputs are mostly 1-3
-// entries long, so a second gather costs a cache line per product).  Values
-// accumulate in LDS when the row has at most acc_cap entries (the dynamic
-// LDS holds acc_cap accumulators after the bitmap), else with FP64 atomics
-// in the row's slot region.
+// gathers every product once, sets its column bit and stages (column, value)
+// in the row's region [off, off + ub) of a scratch pair (the final output
+// arrays, unused until the compaction); pass 2 reads the staged products back
+// coalesced instead of gathering B again (B rows of power-law inputs are
+// mostly 1-3 entries long, so a second gather costs a cache line per product).
+// Values accumulate in LDS when the row has at most acc_cap entries (the
+// dynamic LDS holds acc_cap accumulators after the bitmap), else with FP64
+// atomics in the row's slot region.
+//
+// Pass 1 lists the non-empty A entries in LDS (up to ecap at a time, in the
+// accumulators' place) with their products' prefix, and deals the products out
+// evenly over the threads, each finding its entry by a binary search: with
+// the entries dealt out instead, the wavefront that gets a B row of 4,096
+// entries works alone while fifteen wait.  20k power-law rows, 108 of them
+// long: 117 -> 102 us, as long as the longest row takes.  (All workgroups on all
+// rows, with FP64 atomics into dense rows in HBM: 135 us, about 20 G scattered
+// atomics a second.)
+constexpr int kLongItems = 8;      // products per thread in flight
+constexpr int kLongEntries = 4096; // A entries listed at a time at most
+// accumulators the kernel's LDS holds at least (16 bytes per listed entry)
+constexpr int32_t kLongAccMin = 2 * kBitmapLongBlock;
+
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_row_bitmap_staged(
     const int32_t* __restrict__ bin_rows, const int32_t* __restrict__ bmeta, int path, int32_t ncols,
@@ -1254,15 +1267,17 @@ __global__ __launch_bounds__(BLOCK) void k_row_bitmap_staged(
     int32_t* __restrict__ stage_crd, double* __restrict__ stage_val, int32_t acc_cap) {
   extern __shared__ double bml_d[];
   __shared__ int32_t sh[BLOCK / kWave + 1];
-  __shared__ int32_t cursor;
-  if (threadIdx.x == 0) cursor = 0;
+  __shared__ int64_t sh64[BLOCK / kWave + 1];
   BitmapLds L;
   L.init<BLOCK>(bml_d, ncols);  // ends with a barrier
-  const int wave = threadIdx.x / kWave;
-  const int lane = lane_id();
-  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   const int32_t count = bmeta[kMetaCount + path];
   const int32_t* rows = bin_rows + bmeta[kMetaOff + path];
+  // listed entries: values, then first products, then B row start - first
+  const int32_t ecap = min(kLongEntries, max(acc_cap, kLongAccMin) / 2) / BLOCK * BLOCK;
+  double* const ea = L.acc;
+  int32_t* const efirst = reinterpret_cast<int32_t*>(ea + ecap);
+  int32_t* const ebase = efirst + ecap;
+  constexpr int kPer = kLongEntries / BLOCK;  // entries per thread
   for (int32_t r = blockIdx.x; r < count; r += gridDim.x) {
     const int32_t i = rows[r];
     const int32_t cb = row_colbase ? row_colbase[i] : 0;
@@ -1276,28 +1291,83 @@ __global__ __launch_bounds__(BLOCK) void k_row_bitmap_staged(
     bitmap_row<BLOCK, true, true>(
         i, cb, w0, w1, off, acc_cap, L, sh, slot_crd, slot_val, row_nnz,
         [&](auto&& f) {
-          expand_products<true>(a_beg, a_end, wave, BLOCK / kWave, Ai, Ax, Bp, Bi, Bx, [&](int32_t col, double v) {
-            // the active lanes of this wavefront take consecutive slots
-            const uint64_t act = __ballot(1);
-            const int leader = __ffsll((long long)act) - 1;
-            int32_t base = 0;
-            if (lane == leader) base = atomicAdd(&cursor, __popcll(act));
-            base = __shfl(base, leader, kWave);
-            const int32_t slot = base + __popcll(act & lt);
-            sc[slot] = col;
-            sv[slot] = v;
-            f(col, v);
-          });
+          int32_t done = 0;  // products of the entries listed before
+          for (int32_t c0 = a_beg; c0 < a_end; c0 += ecap) {
+            int32_t bstart[kPer], blen[kPer];
+            double av[kPer];
+            int64_t mine = 0;  // non-empty entries << 40 | their products
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) {
+              bstart[u] = blen[u] = 0;
+              const int32_t e = u * BLOCK + (int32_t)threadIdx.x;
+              if (e < ecap && c0 + e < a_end) {
+                const int32_t j = Ai[c0 + e];
+                av[u] = Ax[c0 + e];
+                bstart[u] = Bp[j];
+                blen[u] = Bp[j + 1] - bstart[u];
+              }
+              if (blen[u] > 0) mine += ((int64_t)1 << 40) + blen[u];
+            }
+            int64_t all;
+            const int64_t at = block_excl_scan<int64_t, BLOCK>(mine, sh64, &all);
+            int32_t s = (int32_t)(at >> 40), first = (int32_t)(at & (((int64_t)1 << 40) - 1));
+#pragma unroll
+            for (int u = 0; u < kPer; ++u)
+              if (blen[u] > 0) {
+                ea[s] = av[u];
+                efirst[s] = first;
+                ebase[s] = bstart[u] - first;
+                first += blen[u];
+                ++s;
+              }
+            __syncthreads();
+            const int32_t listed = (int32_t)(all >> 40), total = (int32_t)(all & (((int64_t)1 << 40) - 1));
+            int top = 1;  // a power of two, at least `listed`
+            while (top < listed) top <<= 1;
+            for (int32_t q0 = 0; q0 < total; q0 += BLOCK * kLongItems) {
+              int32_t col[kLongItems], own[kLongItems];
+              double bv[kLongItems];
+#pragma unroll
+              for (int u = 0; u < kLongItems; ++u) own[u] = 0;
+              // the last entry whose first product is at most the product
+              for (int d = top >> 1; d > 0; d >>= 1) {
+#pragma unroll
+                for (int u = 0; u < kLongItems; ++u) {
+                  const int32_t q = q0 + u * BLOCK + (int32_t)threadIdx.x;
+                  const int32_t mid = own[u] + d;
+                  if (mid < listed && efirst[mid] <= q) own[u] = mid;
+                }
+              }
+#pragma unroll
+              for (int u = 0; u < kLongItems; ++u) {
+                const int32_t q = q0 + u * BLOCK + (int32_t)threadIdx.x;
+                if (q < total) {
+                  const uint32_t kb = (uint32_t)(ebase[own[u]] + q);
+                  col[u] = Bi[kb];
+                  bv[u] = Bx[kb];
+                }
+              }
+#pragma unroll
+              for (int u = 0; u < kLongItems; ++u) {
+                const int32_t q = q0 + u * BLOCK + (int32_t)threadIdx.x;
+                if (q < total) {
+                  sc[done + q] = col[u];
+                  sv[done + q] = ea[own[u]] * bv[u];
+                  f(col[u], 0.0);
+                }
+              }
+            }
+            done += total;
+            __syncthreads();  // the list's place is used again
+          }
           __threadfence_block();  // the staged products are read by other wavefronts in pass 2
         },
         [&](auto&& f) {
-          if (threadIdx.x == 0) cursor = 0;  // pass 1 of every wavefront is done
-          constexpr int kU = 4;
-          for (int32_t q0 = 0; q0 < ub; q0 += BLOCK * kU) {
-            int32_t c[kU];
-            double v[kU];
+          for (int32_t q0 = 0; q0 < ub; q0 += BLOCK * kLongItems) {
+            int32_t c[kLongItems];
+            double v[kLongItems];
 #pragma unroll
-            for (int u = 0; u < kU; ++u) {
+            for (int u = 0; u < kLongItems; ++u) {
               const int32_t q = q0 + u * BLOCK + (int32_t)threadIdx.x;
               if (q < ub) {
                 c[u] = sc[q];
@@ -1305,7 +1375,7 @@ __global__ __launch_bounds__(BLOCK) void k_row_bitmap_staged(
               }
             }
 #pragma unroll
-            for (int u = 0; u < kU; ++u)
+            for (int u = 0; u < kLongItems; ++u)
               if (q0 + u * BLOCK + (int32_t)threadIdx.x < ub) f(c[u], v[u]);
           }
         });
@@ -1897,53 +1967,73 @@ struct DirectRows {
   __device__ bool operator()(int64_t ub) const { return ub > lo && ub <= hi; }
 };
 
-// (the batch engine compacts with its own kernel, which writes into request
-// output buffers, so this one is unused there)
-[[maybe_unused]] __global__ __launch_bounds__(256) void k_compact(int32_t m_host, const int32_t* __restrict__ m_dev,
-                                                 const int64_t* __restrict__ row_off,
-                                                 const int32_t* __restrict__ C_pos,
-                                                 const int32_t* __restrict__ slot_crd,
-                                                 const double* __restrict__ slot_val,
-                                                 const int32_t* __restrict__ row_coloff, int32_t* __restrict__ C_crd,
-                                                 double* __restrict__ C_val, int32_t* __restrict__ meta_zero,
-                                                 DirectRows direct) {
-  // the product's metadata block, read by the host before this launch, is
-  // left zero for the next product
-  if (meta_zero && blockIdx.x == 0 && threadIdx.x < kMetaBlockInts) meta_zero[threadIdx.x] = 0;
-  const int32_t m = dev_or(m_dev, m_host);
-  const int lane = lane_id();
-  const int32_t waves = gridDim.x * (blockDim.x / kWave);
-  for (int32_t i = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; i < m; i += waves) {
-    const int32_t dst = C_pos[i];
-    const int32_t n = C_pos[i + 1] - dst;
-    const int64_t src = row_off[i];
-    if (direct(row_off[i + 1] - src)) continue;
-    const int32_t shift = row_coloff ? row_coloff[i] : 0;
-    // kCompactUnroll strides loaded before any is stored: the copy is
-    // bandwidth-bound, not bound by one load's latency per stride
-    for (int32_t e0 = 0; e0 < n; e0 += kWave * kCompactUnroll) {
-      int32_t c[kCompactUnroll];
-      double v[kCompactUnroll];
+// Workgroups of a compaction: `plain` of them take the rows a wavefront each;
+// when the rows beyond the block bins are listed, those are left to the
+// further workgroups, kParts per row (a row of 20k entries copied by one
+// wavefront takes 57 us, whatever the rest of the product).
+struct CompactGrid {
+  int32_t plain;
+  const int32_t* long_rows;  // null: no row is left out
+  int64_t long_ub;           // rows above this upper bound are in the list
+  static constexpr int kParts = 8;
+};
+
+// kCompactUnroll strides loaded before any is stored: the copy is
+// bandwidth-bound, not bound by one load's latency per stride
+__device__ __forceinline__ void compact_entries(int32_t e0, int32_t step, int32_t n, int32_t shift,
+                                                const int32_t* __restrict__ from_crd,
+                                                const double* __restrict__ from_val, int32_t* __restrict__ to_crd,
+                                                double* __restrict__ to_val) {
+  for (; e0 < n; e0 += step * kCompactUnroll) {
+    int32_t c[kCompactUnroll];
+    double v[kCompactUnroll];
 #pragma unroll
-      for (int u = 0; u < kCompactUnroll; ++u) {
-        const int32_t e = e0 + u * kWave + lane;
-        if (e < n) {
-          c[u] = slot_crd[src + e];
-          v[u] = slot_val[src + e];
-        }
+    for (int u = 0; u < kCompactUnroll; ++u) {
+      const int32_t e = e0 + u * step;
+      if (e < n) {
+        c[u] = from_crd[e];
+        v[u] = from_val[e];
       }
+    }
 #pragma unroll
-      for (int u = 0; u < kCompactUnroll; ++u) {
-        const int32_t e = e0 + u * kWave + lane;
-        if (e < n) {
-          C_crd[dst + e] = c[u] - shift;
-          C_val[dst + e] = v[u];
-        }
+    for (int u = 0; u < kCompactUnroll; ++u) {
+      const int32_t e = e0 + u * step;
+      if (e < n) {
+        to_crd[e] = c[u] - shift;
+        to_val[e] = v[u];
       }
     }
   }
 }
 
+// (the batch engine compacts with its own kernel, which writes into request
+// output buffers, so this one is unused there)
+[[maybe_unused]] __global__ __launch_bounds__(256) void k_compact(
+    int32_t m, const int64_t* __restrict__ row_off, const int32_t* __restrict__ C_pos,
+    const int32_t* __restrict__ slot_crd, const double* __restrict__ slot_val, int32_t* __restrict__ C_crd,
+    double* __restrict__ C_val, int32_t* __restrict__ meta_zero, DirectRows direct, CompactGrid grid) {
+  // the product's metadata block, read by the host before this launch, is
+  // left zero for the next product
+  if (meta_zero && blockIdx.x == 0 && threadIdx.x < kMetaBlockInts) meta_zero[threadIdx.x] = 0;
+  if ((int32_t)blockIdx.x >= grid.plain) {
+    const int32_t item = blockIdx.x - grid.plain;
+    const int32_t i = grid.long_rows[item / CompactGrid::kParts];
+    const int32_t dst = C_pos[i];
+    const int64_t src = row_off[i];
+    compact_entries(item % CompactGrid::kParts * blockDim.x + threadIdx.x, CompactGrid::kParts * blockDim.x,
+                    C_pos[i + 1] - dst, 0, slot_crd + src, slot_val + src, C_crd + dst, C_val + dst);
+    return;
+  }
+  const int32_t waves = grid.plain * (blockDim.x / kWave);
+  for (int32_t i = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; i < m; i += waves) {
+    const int32_t dst = C_pos[i];
+    const int64_t src = row_off[i];
+    const int64_t ub = row_off[i + 1] - src;
+    if (direct(ub) || (grid.long_rows && ub > grid.long_ub)) continue;
+    compact_entries(lane_id(), kWave, C_pos[i + 1] - dst, 0, slot_crd + src, slot_val + src, C_crd + dst,
+                    C_val + dst);
+  }
+}
 
 }  // namespace
 }  // namespace spws

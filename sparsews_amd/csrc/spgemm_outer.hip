@@ -1379,17 +1379,6 @@ static size_t outer_output_capacity(const spws_ctx* ctx) {
   return ctx->out_crd.bytes / 4 < ctx->out_val.bytes / 8 ? ctx->out_crd.bytes / 4 : ctx->out_val.bytes / 8;
 }
 
-// Launches inside the scope go to stream s (when not null) instead of the
-// context's stream, timing included.
-struct StreamScope {
-  spws_ctx* ctx;
-  hipStream_t saved;
-  StreamScope(spws_ctx* c, hipStream_t s) : ctx(c), saved(c->stream) {
-    if (s) c->stream = s;
-  }
-  ~StreamScope() { ctx->stream = saved; }
-};
-
 static int outer_output_grow(spws_ctx* ctx, int64_t base, int64_t U) {
   hipStream_t s = ctx->stream;
   int rc;

@@ -56,6 +56,8 @@ namespace spws {
 // least products in the block bins for their rows to be counted first and
 // computed in place (see rowwise_run)
 constexpr int64_t kDirectProducts = 4 << 20;
+// rows beyond the block bins that the compaction splits over workgroups at most
+constexpr int64_t kCompactSplitMax = 1 << 16;
 
 static int validate_tuning(const spws_rowwise_tuning& t) {
   SPWS_REQUIRE(t.wave_ub >= 1 && t.wave_ub <= kWaveUbMax, SPWS_ERR_INVALID, "wave_ub must be in [1, %d]",
@@ -70,6 +72,32 @@ static int validate_tuning(const spws_rowwise_tuning& t) {
   SPWS_REQUIRE(t.force_path >= -1 && t.force_path <= P_WIDE, SPWS_ERR_INVALID, "force_path must be in [-1, 5]");
   return SPWS_OK;
 }
+
+// Work on the context's second stream, after everything enqueued on its own
+// stream so far; join() (also at the end of the scope) makes the own stream
+// wait for it.
+struct Fork {
+  spws_ctx* ctx;
+  hipStream_t stream = nullptr;  // null: not forked
+  explicit Fork(spws_ctx* c) : ctx(c) {}
+  int begin() {
+    hipStream_t aux;
+    if (int rc = ctx_aux_stream(ctx, &aux)) return rc;
+    SPWS_HIP(hipEventRecord(ctx->aux_ready, ctx->stream));
+    SPWS_HIP(hipStreamWaitEvent(aux, ctx->aux_ready, 0));
+    stream = aux;
+    return SPWS_OK;
+  }
+  int join() {
+    if (!stream) return SPWS_OK;
+    hipStream_t aux = stream;
+    stream = nullptr;
+    SPWS_HIP(hipEventRecord(ctx->aux_done[0], aux));
+    SPWS_HIP(hipStreamWaitEvent(ctx->stream, ctx->aux_done[0], 0));
+    return SPWS_OK;
+  }
+  ~Fork() { (void)join(); }
+};
 
 // The short-row product in two launches (k_short_rows, k_short_compact)
 // into the context's C arrays.  *ok is false when it does not apply (more
@@ -298,6 +326,41 @@ static int rowwise_run(spws_ctx* ctx, int32_t m, int32_t kdim, int32_t n, const 
   int32_t* rnnz = ctx->row_nnz.as<int32_t>();
   auto grid_for = [](int64_t cnt, int64_t cap) { return (unsigned)(cnt < cap ? cnt : cap); };
 
+  const bool bits = n <= kBitmapCols;
+  // rows longer than the block bins: while the columns fit the LDS bitmap,
+  // the bitmap kernel accumulating in the rows' slot regions replaces both
+  // the dense accumulator and the HBM hash table
+  // (P_DENSE and P_WIDE rows follow one another in the bins' list).  They run
+  // beside the other bins, on the context's second stream: a workgroup per
+  // row leaves most of the chip idle for as long as the longest row takes
+  // (20k power-law rows: call 276 -> 243 us).
+  const int64_t nlong = counts[P_DENSE] + counts[P_WIDE];
+  const int64_t nother = counts[P_WAVE] + counts[P_WAVE2] + counts[P_BLOCK] + counts[P_BLOCK2];
+  const int32_t* const long_rows = rows + nother;
+  Fork fork(ctx);
+  if (bits && nlong > 0) {
+    if (nother > 0 && (rc = fork.begin())) return rc;
+    StreamScope scope(ctx, fork.stream);
+    for (int path : {(int)P_DENSE, (int)P_WIDE}) {
+      if (!counts[path]) continue;
+      // staged in the output arrays, which the compaction fills later; rows
+      // of at most acc_cap entries accumulate in LDS
+      const size_t bm_bytes = bitmap_lds_bytes(n, 0, false, kBitmapLongBlock);
+      const int32_t acc_cap = (int32_t)std::min<int64_t>(std::min<int64_t>(maxub[path], n),
+                                                         (int64_t)((kLdsBudget - bm_bytes) / 8));
+      if (kValues)
+        SPWS_LAUNCH(ctx, "row_bitmap_long", k_row_bitmap_staged<kBitmapLongBlock>,
+                    dim3(grid_for(counts[path], 4096)), dim3(kBitmapLongBlock),
+                    bitmap_lds_bytes(n, std::max(acc_cap, kLongAccMin), true, kBitmapLongBlock), rows, bmeta, path, n,
+                    Ap, Ai, Ax, Bp, Bi, Bx, roff, scrd, sval, rnnz, (const int32_t*)nullptr, (const int32_t*)nullptr,
+                    ctx->out_crd.as<int32_t>(), ctx->out_val.as<double>(), acc_cap);
+      else
+        SPWS_LAUNCH(ctx, "row_bitmap_long", k_row_bitmap<kBitmapLongBlock>, dim3(grid_for(counts[path], 4096)),
+                    dim3(kBitmapLongBlock), bitmap_lds_bytes(n, 0, false, kBitmapLongBlock), rows, bmeta, path, n, Ap,
+                    Ai, Bp, Bi, rnnz);
+      counts[path] = 0;
+    }
+  }
   if (counts[P_WAVE]) {
     SPWS_LAUNCH(ctx, "row_wave", (k_row_wave<128, 1, kValues, kWaveRowsK>),
                 dim3(grid_for(div_up(counts[P_WAVE], kWaveRowsK), 1 << 20)), dim3(64), 0, rows, bmeta, (int)P_WAVE,
@@ -316,7 +379,6 @@ static int rowwise_run(spws_ctx* ctx, int32_t m, int32_t kdim, int32_t n, const 
   // the copy is cheaper than two more launches.
   int cus = 0;
   SPWS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-  const bool bits = n <= kBitmapCols;
   const bool direct = kValues && bits && t.force_path < 0 &&
                       counts[P_BLOCK] * (int64_t)(t.wave2_ub + 1) + counts[P_BLOCK2] * (int64_t)(t.block_ub + 1) >=
                           kDirectProducts;
@@ -365,30 +427,6 @@ static int rowwise_run(spws_ctx* ctx, int32_t m, int32_t kdim, int32_t n, const 
                   dim3(grid_for(counts[P_BLOCK2], 1 << 16)), dim3(512), 0, rows, bmeta, (int)P_BLOCK2, Ap, Ai, Ax, Bp,
                   Bi, Bx, roff, scrd, sval, rnnz);
   }
-  // rows longer than the block bins: while the columns fit the LDS bitmap,
-  // the bitmap kernel accumulating in the rows' slot regions replaces both
-  // the dense accumulator and the HBM hash table
-  if (n <= kBitmapCols) {
-    for (int path : {(int)P_DENSE, (int)P_WIDE}) {
-      if (!counts[path]) continue;
-      // staged in the output arrays, which the compaction fills later; rows
-      // of at most acc_cap entries accumulate in LDS
-      const size_t bm_bytes = bitmap_lds_bytes(n, 0, false, kBitmapLongBlock);
-      const int32_t acc_cap = (int32_t)std::min<int64_t>(std::min<int64_t>(maxub[path], n),
-                                                         (int64_t)((kLdsBudget - bm_bytes) / 8));
-      if (kValues)
-        SPWS_LAUNCH(ctx, "row_bitmap_long", k_row_bitmap_staged<kBitmapLongBlock>,
-                    dim3(grid_for(counts[path], 4096)), dim3(kBitmapLongBlock),
-                    bitmap_lds_bytes(n, acc_cap, true, kBitmapLongBlock), rows, bmeta, path, n, Ap, Ai, Ax, Bp, Bi,
-                    Bx, roff, scrd, sval, rnnz, (const int32_t*)nullptr, (const int32_t*)nullptr,
-                    ctx->out_crd.as<int32_t>(), ctx->out_val.as<double>(), acc_cap);
-      else
-        SPWS_LAUNCH(ctx, "row_bitmap_long", k_row_bitmap<kBitmapLongBlock>, dim3(grid_for(counts[path], 4096)),
-                    dim3(kBitmapLongBlock), bitmap_lds_bytes(n, 0, false, kBitmapLongBlock), rows, bmeta, path, n, Ap,
-                    Ai, Bp, Bi, rnnz);
-      counts[path] = 0;
-    }
-  }
   if (counts[P_DENSE]) {
     // bounded scratch: at most ~2 GiB of dense accumulators
     const size_t per = (size_t)(n > 0 ? n : 1) * (kValues ? 9 : 1);
@@ -419,16 +457,18 @@ static int rowwise_run(spws_ctx* ctx, int32_t m, int32_t kdim, int32_t n, const 
     SPWS_LAUNCH(ctx, "row_wide", (k_row_wide<kValues>), dim3((unsigned)g), dim3(kWideBlock), 0, rows, bmeta,
                 (int)P_WIDE, Ap, Ai, Ax, Bp, Bi, Bx, ctx->row_ub.as<int64_t>(), roff, scrd, sval, rnnz, tk, tv, tab);
   }
+  if ((rc = fork.join())) return rc;
   rc = exclusive_scan<int32_t, int32_t>(ctx, rnnz, ctx->out_pos.as<int32_t>(), m);
   if (rc) return rc;
   // (the long rows staged their products in C's arrays: before this point only)
   if (direct && (rc = block_rows(kFinalRows))) return rc;
   if (kValues && m > 0) {
-    unsigned g = (unsigned)div_up(m, 4);
-    if (g > 65536) g = 65536;
-    SPWS_LAUNCH(ctx, "compact", k_compact, dim3(g), dim3(256), 0, m, nullptr, roff, ctx->out_pos.as<int32_t>(), scrd,
-                sval, nullptr, ctx->out_crd.as<int32_t>(), ctx->out_val.as<double>(), bmeta,
-                direct ? DirectRows{t.wave2_ub, t.block2_ub} : DirectRows{0, 0});
+    const unsigned g = (unsigned)std::min<int64_t>(div_up(m, 4), 65536);
+    const bool split = nlong > 0 && nlong <= kCompactSplitMax && t.force_path < 0;
+    SPWS_LAUNCH(ctx, "compact", k_compact, dim3(g + (split ? (unsigned)nlong * CompactGrid::kParts : 0u)), dim3(256), 0,
+                m, roff, ctx->out_pos.as<int32_t>(), scrd, sval, ctx->out_crd.as<int32_t>(),
+                ctx->out_val.as<double>(), bmeta, direct ? DirectRows{t.wave2_ub, t.block2_ub} : DirectRows{0, 0},
+                CompactGrid{(int32_t)g, split ? long_rows : nullptr, t.block2_ub});
   }
   SPWS_HIP(hipMemcpyAsync(h32, ctx->out_pos.as<int32_t>() + m, 4, hipMemcpyDeviceToHost, s));
   SPWS_HIP(hipStreamSynchronize(s));

@@ -336,6 +336,30 @@ def test_block_rows_in_place(ctx, ncols, bulk):
     np.testing.assert_array_equal(spgemm_rowwise_symbolic(ctx, dA, dB), G.pos)
 
 
+@pytest.mark.parametrize("ncols", [6000, 100_000, 131_072])
+def test_long_rows_listed_entries(ctx, ncols):
+    """Long rows beside every other bin: one A entry only, A entries just
+    below, at and above the counts listed at a time (1,024 and 4,096, and
+    several lists), two in three of their B rows empty, one B row that
+    outweighs all the others."""
+    print(f"case: long rows, listed entries ncols={ncols}", flush=True)
+    k = 14_000
+    lengths = np.tile([0, 7, 0], k // 3 + 1)[:k]
+    lengths[1] = 5000
+    B = random_csr(k, ncols, lengths, 81, 1)
+    rng = np.random.default_rng(81)
+    counts = [1, 2, 1023, 1024, 1025, 2048, 4095, 4096, 4097, 8192, 8193, 12_289, 14_000] + [3, 40, 120, 300, 0] * 30
+    rows = [np.unique(np.concatenate([[1] if c != 300 else [], rng.permutation(k)[:max(c - 1, 0)]])) if c else
+            np.zeros(0) for c in counts]
+    for q in range(13, len(rows)):  # the shorter rows without the heavy B row
+        rows[q] = rows[q][rows[q] != 1]
+    crd = np.concatenate(rows).astype(np.int32)
+    pos = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    A = CSR(len(rows), k, pos, crd, rng.uniform(-1, 1, len(crd)))
+    check(run(ctx, A, B), A, B)
+    assert ctx.stats()["rows_per_path"][4] + ctx.stats()["rows_per_path"][5] == 13
+
+
 @pytest.mark.parametrize("every,path", [(10, 0), (2, 1)])
 def test_wave_bins_with_many_a_entries(ctx, every, path):
     """Rows of 300 A entries whose B rows are mostly empty: at most 64 (or
