@@ -145,8 +145,10 @@ void prof_collect(spws_ctx* ctx) {
 // tiles' sums itself and scans its tile (coalesced: each wavefront takes a
 // quarter of the tile 64 values at a time, DPP wavefront scans with a
 // running carry); beyond that, a single-workgroup scan of the tile sums
-// and a rescan of each tile with its offset.  Inputs of at most four tiles
-// take a single-workgroup path.
+// and a rescan of each tile with its offset.
+//
+// Inputs of at most kScanSmall values take one launch: every workgroup sums
+// all the values before its tile itself.  PERF_SCAN
 
 constexpr int kScanBlock = 256;
 constexpr int kScanItems = 16;
@@ -172,6 +174,66 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_tile_reduce(const Tin* __re
     for (int w = 0; w < kScanBlock / kWave; ++w) t += sh[w];
     tile_sums[blockIdx.x] = t;
   }
+}
+
+// Exclusive scan of n <= kScanSmall values in one launch, a tile of
+// kScanSmallTile per workgroup (16-byte loads of 32-bit values; the input is
+// 16-byte aligned); out[n] = total.
+constexpr int kScanSmallBlock = 1024;
+constexpr int kScanSmallTile = 4 * kScanSmallBlock;
+constexpr int64_t kScanSmall = 1 << 16;
+
+template <class Tin, class Tout>
+__global__ __launch_bounds__(kScanSmallBlock) void k_scan_small(const Tin* __restrict__ in, int32_t n,
+                                                                Tout* __restrict__ out) {
+  struct alignas(16) Quad {
+    Tin v[4];
+  };
+  constexpr int kWaves = kScanSmallBlock / kWave;
+  constexpr int kU = 4;  // tiles before this one summed together
+  __shared__ Tout sh[2 * kWaves];
+  const Quad* const quads = reinterpret_cast<const Quad*>(in);
+  const int lane = lane_id();
+  const int w = threadIdx.x / kWave;
+  const int32_t mine = blockIdx.x * kScanSmallTile + 4 * (int32_t)threadIdx.x;
+  Tout v[4];
+  if (mine + 4 <= n) {
+    const Quad q = quads[mine / 4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (Tout)q.v[e];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = mine + e < n ? (Tout)in[mine + e] : (Tout)0;
+  }
+  Tout before = 0;
+  for (int32_t b = 0; b < (int32_t)blockIdx.x; b += kU) {
+    Quad q[kU] = {};
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      if (b + u < (int32_t)blockIdx.x) q[u] = quads[(b + u) * kScanSmallBlock + threadIdx.x];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) before += ((Tout)q[u].v[0] + q[u].v[1]) + ((Tout)q[u].v[2] + q[u].v[3]);
+  }
+  const Tout local = (v[0] + v[1]) + (v[2] + v[3]);
+  const Tout incl = wave_incl_scan(local);
+  before = wave_sum(before);
+  if (lane == kWave - 1) {
+    sh[w] = before;
+    sh[kWaves + w] = incl;
+  }
+  __syncthreads();
+  Tout run = incl - local, total = 0;
+#pragma unroll
+  for (int q = 0; q < kWaves; ++q) {
+    total += sh[q] + sh[kWaves + q];
+    run += sh[q] + (q < w ? sh[kWaves + q] : (Tout)0);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (mine + e < n) out[mine + e] = run;
+    run += v[e];
+  }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = total;
 }
 
 // Single-workgroup exclusive scan of n values (any n); out[n] = total.
@@ -292,6 +354,11 @@ size_t scan_scratch_bytes(int64_t n, size_t elem_bytes) {
 
 template <class Tin, class Tout>
 int exclusive_scan(spws_ctx* ctx, const Tin* in, Tout* out, int64_t n) {
+  if (n <= kScanSmall && reinterpret_cast<uintptr_t>(in) % 16 == 0) {
+    const unsigned g = (unsigned)std::max<int64_t>(1, div_up(n, kScanSmallTile));
+    SPWS_LAUNCH(ctx, "scan_small", (k_scan_small<Tin, Tout>), dim3(g), dim3(kScanSmallBlock), 0, in, (int32_t)n, out);
+    return SPWS_OK;
+  }
   if (n <= 4 * (int64_t)kScanTile) {
     SPWS_LAUNCH(ctx, "scan_single", (k_scan_single<Tin, Tout>), dim3(1), dim3(kScanBlock), 0, in, n, out);
     return SPWS_OK;

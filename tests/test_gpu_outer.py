@@ -434,6 +434,17 @@ def test_device_transpose(ctx, m, n, lo, hi, seed):
     np.testing.assert_array_equal(T.vals, O.vals)
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 4095, 4096, 4097, 8193, 16_384, 16_385, 20_483, 65_535, 65_536, 65_537, 200_001])
+def test_prefix_sum_lengths(ctx, n):
+    """Row pointers (a prefix sum of n counts, most of them zero at the larger
+    n) of a transpose into n rows, at the edges of the scan's tiles."""
+    print(f"case: prefix sum of {n} counts", flush=True)
+    from sparsews_amd.device import DeviceCSR, csr_transpose
+    A = uniform_rows(700, n, 0, min(n, 9), n, 0)
+    T = csr_transpose(ctx, DeviceCSR.upload(ctx, A)).download()
+    np.testing.assert_array_equal(T.pos, np.concatenate([[0], np.cumsum(np.bincount(A.crd, minlength=n))]))
+
+
 @pytest.mark.parametrize("method", METHODS)
 @pytest.mark.parametrize("m,k,n,seed", [(300, 250, 400, 81), (2000, 1500, 1000, 82), (50, 3000, 70_000, 83)])
 def test_device_fused_vs_nonfused_transposed_output(ctx, method, m, k, n, seed):
