@@ -403,7 +403,7 @@ def run_mttkrp(args):
     def step():
         out["r"] = mttkrp(ctx, dX, I, J, K, R, dB, dC)
 
-    names = ("mttkrp_accum", "radix_scatter", "mttkrp_keys")
+    names = ("mttkrp_accum", "radix_scatter")
     sec, dom, dom_times, bd = timed_steps(ctx, step, args.steps, args.warmup,
                                           lambda bd: max(names, key=lambda k: bd.get(k, (0, 1))[0]))
     calibration_copy(ctx, args.calibrate_copy)
@@ -413,8 +413,9 @@ def run_mttkrp(args):
     per_step = {
         # sorted (key, value) records + factor matrices once + the output rows
         "mttkrp_accum": 16 * nnz + 8 * R * (J + K) + 8 * R * nrows,
-        "radix_scatter": 2 * 16 * nnz * passes,
-        "mttkrp_keys": 4 * nnz + 4 * nnz + 8 * nnz,
+        # key + value read and written per pass; the first reads the leaves'
+        # coordinates instead of keys
+        "radix_scatter": 2 * 16 * nnz * passes - 4 * nnz,
     }
     # compulsory bytes: X as COO (three int32 coordinates + FP64 value per
     # nonzero), both factor matrices once, the dense output once
@@ -475,9 +476,9 @@ def run_ttm(args):
     F = out["r"][0].count
     roots_path = "tw_heavy" in bd or "tw_light" in bd
     # sorting path: the nonzeros are grouped by one stable radix sort on the
-    # (i, j) bits of their packed (i, j, k) keys: 8-bit digits
+    # (i, j) bits of their packed (i, j, k) keys: digits of at most 9 bits
     sort_bits = max(1, (I - 1).bit_length()) + max(1, (J - 1).bit_length())
-    passes = -(-sort_bits // 8)
+    passes = -(-sort_bits // 9)
     # roots path: nonzeros of heavy roots (more than 256) and light roots
     rl = np.diff(csf.l3_pos[csf.l2_pos.astype(np.int64)])
     heavy_nnz = int(rl[rl > 256].sum())
@@ -485,12 +486,10 @@ def run_ttm(args):
     per_step = {
         # sorting path
         #   ttm_accum      per nonzero key + value read; per fiber R values written; U once
-        #   radix_scatter  per nonzero and pass key + value read and written
-        #   ttm_keys       per nonzero leaf fiber, fiber root, three coordinates and
-        #                  value read; key + value written
+        #   radix_scatter  per nonzero and pass key + value read and written; the
+        #                  first pass reads the leaves' coordinates instead of keys
         "ttm_accum": nnz * (8 + 8) + 8 * R * F + 8 * R * K,
-        "radix_scatter": nnz * 32 * passes,
-        "ttm_keys": nnz * (4 + 4 + 4 + 4 + 4 + 8 + 16),
+        "radix_scatter": nnz * 32 * passes - 4 * nnz,
         # roots path
         #   tw_scatter     per heavy nonzero column, value and k read, key + value written
         #   tw_heavy       per heavy nonzero key + value read; its fibers' R values and
@@ -749,7 +748,7 @@ def run_transpose(args):
         check(lib().spws_csr_transpose_dev(ctx.h, m, n, nnz, dA.pos.ptr, dA.crd.ptr, dA.vals.ptr, out_pos.ptr,
                                            out_crd.ptr, out_val.ptr))
 
-    names = ("radix_scatter", "tr_keys", "tr_out")
+    names = ("radix_scatter", "radix_hist", "tr_pos")
     sec, dom, dom_times, bd = timed_steps(ctx, step, args.steps, args.warmup,
                                           lambda bd: max(names, key=lambda k: bd.get(k, (0, 1))[0]))
     calibration_copy(ctx, args.calibrate_copy)
@@ -760,14 +759,14 @@ def run_transpose(args):
     rows = np.repeat(np.arange(m, dtype=np.int32), np.diff(A.pos))
     lim = int(np.searchsorted(cols[order], 1000))
     assert np.array_equal(T.crd[:lim], rows[order][:lim]) and np.array_equal(T.vals[:lim], A.vals[order][:lim])
-    passes = -(-max(1, (n - 1).bit_length()) // 8)
+    passes = -(-max(1, (n - 1).bit_length()) // 9)
     per_step = {
-        # per entry and pass: key + value read and written
-        "radix_scatter": nnz * 32 * passes,
-        # per entry: column and value read, key and value written; row pointers
-        "tr_keys": nnz * (4 + 8 + 8 + 8) + 4 * (m + 1),
-        # per entry: key and value read, row index and value written
-        "tr_out": nnz * (8 + 8 + 4 + 8),
+        # per entry and pass: key + value read and written; the first pass reads
+        # columns and row pointers instead of keys
+        "radix_scatter": nnz * 32 * passes - 4 * nnz + 4 * (m + 1),
+        # per entry: its column, then its key
+        "radix_hist": nnz * (4 + 8 * (passes - 1)),
+        "tr_pos": 4 * nnz + 4 * (n + 1),
     }
     algorithmic = 24 * nnz + 4 * (m + 1) + 4 * (n + 1)
     res = {

@@ -1,4 +1,28 @@
-// Stable LSD radix sort of (key, FP64 value) pairs on the device.
+// Stable LSD radix sort of (key, FP64 value) pairs on the device, up to 9
+// bits per pass.
+//
+// The key bits are split evenly over ceil(bits / 9) passes (34 bits: 9, 9,
+// 8, 8).  Per pass, three steps over tiles of kSortTile keys:
+//   1. k_radix_hist     per-tile digit histogram (LDS atomics), written
+//                       digit-major: hist[d * ntiles + t].
+//   2. exclusive scan   of the digit-major histogram -> global offset of
+//                       (digit d, tile t).
+//   3. k_radix_scatter  stable tile-local ranks by wavefront multisplit:
+//                       each wave walks its contiguous quarter of the tile
+//                       64 keys at a time; one ballot per digit bit gives
+//                       the lanes holding the same digit, the group's rank
+//                       is the running per-wave digit count (LDS) plus the
+//                       lanes before it.  Keys, then values, are staged in
+//                       LDS in digit order (one buffer, two rounds) and
+//                       written out so that consecutive threads store
+//                       consecutive addresses of each digit's run.
+//
+// Where the pairs of the first pass come from and where those of the last go
+// is a template parameter each, so that keys made from a sparse structure are
+// never stored before they are first moved, nor stored as keys when the caller
+// wants them in parts.  (20M nonzeros of a CSF: the key pass took 95 us and
+// two launches; the first scatter that makes them takes 20 us more than one
+// that reads them.)
 #pragma once
 #include "common.hpp"
 
@@ -32,5 +56,312 @@ inline size_t radix_hist_entries(int64_t n) {
 template <class K>
 int radix_sort_pairs(spws_ctx* ctx, K* keys, double* vals, K* keys_alt, double* vals_alt, int64_t n, int begin_bit,
                      int end_bit, bool* in_alt, const double* vals_first = nullptr);
+
+inline int radix_passes(int bits) { return (bits + kSortDigitMax - 1) / kSortDigitMax; }
+
+// ------------------------------------------------------------ segment owners
+
+// The last s in [0, n) with pos[s] <= x (pos[0] <= x, pos nondecreasing), by
+// the whole wavefront: 64 probes a round.
+template <class PosT>
+__device__ __forceinline__ int32_t last_at_or_before(const PosT* __restrict__ pos, int32_t n, int64_t x) {
+  int32_t lo = 0, hi = n;
+  while (hi - lo > 1) {
+    const int32_t step = (hi - lo + kWave - 1) / kWave;
+    const int64_t at = lo + (int64_t)lane_id() * step;
+    const uint64_t ok = __ballot(at < hi && (int64_t)pos[at] <= x);
+    lo += (kWave - 1 - __builtin_clzll(ok)) * step;  // lane 0 always holds
+    hi = min(hi, lo + step);
+  }
+  return lo;
+}
+
+// owner[r] = the segment s with pos[s] <= e < pos[s + 1] of item
+// e = base + w * kSub + r * 64 + lane (w: the wavefront, kSub = 64 * ITEMS),
+// for the items of one workgroup's tile [base, end).  Segments mark their
+// first item in LDS (`marks`: a uint32 per item of the tile), and a max-scan
+// carries each mark to the items after it.  Ends with a barrier after the last
+// use of `marks`; every thread of the workgroup calls it.
+template <int BLOCK, int ITEMS, class PosT>
+__device__ __forceinline__ void tile_owners(const PosT* __restrict__ pos, int32_t nseg, int64_t base, int64_t end,
+                                            uint32_t* __restrict__ marks, int32_t (&owner)[ITEMS]) {
+  constexpr int kWaves = BLOCK / kWave;
+  __shared__ uint32_t top[kWaves];
+  const int lane = lane_id();
+  const int w = threadIdx.x / kWave;
+  const int32_t s0 = last_at_or_before(pos, nseg, base);
+  for (int e = threadIdx.x; e < BLOCK * ITEMS; e += BLOCK) marks[e] = 0;
+  __syncthreads();
+  for (int32_t s = s0 + (int32_t)threadIdx.x; s < nseg; s += BLOCK) {
+    const int64_t p = (int64_t)pos[s];
+    if (p >= end) break;
+    if ((int64_t)pos[s + 1] > p) marks[p > base ? p - base : 0] = (uint32_t)(s - s0) + 1;
+  }
+  __syncthreads();
+  uint32_t m[ITEMS];
+  uint32_t mine = 0;
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    m[r] = marks[(w * ITEMS + r) * kWave + lane];
+    mine = max(mine, m[r]);
+  }
+  mine = wave_max(mine);
+  if (lane == 0) top[w] = mine;
+  __syncthreads();
+  uint32_t carry = 0;
+#pragma unroll
+  for (int q = 0; q < kWaves; ++q)
+    if (q < w) carry = max(carry, top[q]);
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const uint32_t x = max(wave_incl_max(m[r]), carry);
+    owner[r] = s0 + (int32_t)x - 1;
+    carry = wave_last(x);
+  }
+}
+
+// ------------------------------------------------------------ sources and sinks
+
+// A source gives pair idx of the first pass: its value, and raw(idx), from
+// which key() makes the key.  With kOwners, key() also gets the item's segment,
+// found by owners() while the raw parts and values are in flight.
+// digit_bits(raw) holds the first digit's bits, all the histogram needs; with
+// kOwnedDigits that takes the segment too, and the histogram calls key().
+template <class K>
+struct PairSource {
+  static constexpr bool kOwners = false, kOwnedDigits = false;
+  using Raw = K;
+  const K* __restrict__ keys;
+  const double* __restrict__ vals;
+  __device__ K raw(int64_t idx) const { return keys[idx]; }
+  __device__ double val(int64_t idx) const { return vals[idx]; }
+  __device__ K digit_bits(K k) const { return k; }
+  __device__ K key(K k, int32_t) const { return k; }
+};
+
+// A sink takes the key and the value that belong at position `at`.
+template <class K>
+struct PairSink {
+  K* __restrict__ keys;
+  double* __restrict__ vals;
+  __device__ void key(int64_t at, K k) const { keys[at] = k; }
+  __device__ void val(int64_t at, double v) const { vals[at] = v; }
+};
+
+template <class K>
+__device__ __forceinline__ int radix_digit(K key, int shift, uint32_t mask) {
+  return (int)((key >> shift) & (K)mask);
+}
+
+template <class K, class Source>
+__global__ __launch_bounds__(kSortBlock) void k_radix_hist(Source in, int64_t n, int shift, uint32_t mask,
+                                                           int32_t* __restrict__ hist, int64_t ntiles) {
+  __shared__ int32_t h[kSortBucketsMax];
+  const int nb = (int)mask + 1;
+  for (int d = threadIdx.x; d < nb; d += kSortBlock) h[d] = 0;
+  __syncthreads();
+  const int64_t base = (int64_t)blockIdx.x * kSortTile;
+  typename Source::Raw raw[kSortItems];
+  if constexpr (Source::kOwnedDigits) {
+    __shared__ uint32_t marks[kSortTile];
+    int32_t owner[kSortItems];
+    in.owners(base, base + kSortTile < n ? base + kSortTile : n, marks, owner);
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r) {
+      const int64_t idx = base + (int64_t)((threadIdx.x / kWave) * kSortItems + r) * kWave + lane_id();
+      if (idx < n) atomicAdd(&h[radix_digit(in.key(in.raw(idx), owner[r]), shift, mask)], 1);
+    }
+  } else {
+#pragma unroll
+    for (int it = 0; it < kSortItems; ++it) {
+      const int64_t idx = base + (int64_t)it * kSortBlock + threadIdx.x;
+      if (idx < n) raw[it] = in.raw(idx);
+    }
+#pragma unroll
+    for (int it = 0; it < kSortItems; ++it) {
+      const int64_t idx = base + (int64_t)it * kSortBlock + threadIdx.x;
+      if (idx < n) atomicAdd(&h[radix_digit<K>(in.digit_bits(raw[it]), shift, mask)], 1);
+    }
+  }
+  __syncthreads();
+  for (int d = threadIdx.x; d < nb; d += kSortBlock) hist[(int64_t)d * ntiles + blockIdx.x] = h[d];
+}
+
+template <class K, class Source, class Sink>
+__global__ __launch_bounds__(kSortBlock, 4) void k_radix_scatter(Source in, Sink out, int64_t n, int shift,
+                                                                 uint32_t mask, int nbits,
+                                                                 const int32_t* __restrict__ offs, int64_t ntiles) {
+  constexpr int kWaves = kSortBlock / kWave;
+  constexpr int kSub = kSortTile / kWaves;  // keys per wave
+  static_assert(kSortBucketsMax == 2 * kSortBlock, "two digits per thread in the prefix step");
+  static_assert(sizeof(K) <= sizeof(double), "one staging buffer for keys and values");
+  __shared__ double stage[kSortTile];  // keys, then values, in digit order
+  // per (wavefront, digit): counts, then their prefixes over the wavefronts
+  // (at most kSortTile = 4096, so 16 bits: 38.9 KB of LDS in all, four
+  // workgroups per CU)
+  __shared__ uint16_t wcnt[kWaves][kSortBucketsMax];
+  static_assert(kSortTile < 65536, "per-wavefront digit prefixes fit 16 bits");
+  __shared__ int32_t dstart[kSortBucketsMax];
+  __shared__ int32_t scan_sh[kSortBlock / kWave + 1];
+  K* sk = reinterpret_cast<K*>(stage);
+
+  const int lane = lane_id();
+  const int w = threadIdx.x / kWave;
+  const int nb = (int)mask + 1;
+  const int64_t base = (int64_t)blockIdx.x * kSortTile;
+  const int64_t wbase = base + (int64_t)w * kSub;
+  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  typename Source::Raw raw[kSortItems];
+  K key[kSortItems];
+  double val[kSortItems];
+  int32_t rank[kSortItems];
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) {
+    const int64_t idx = wbase + (int64_t)r * kWave + lane;
+    raw[r] = {};
+    val[r] = 0.0;
+    if (idx < n) {
+      raw[r] = in.raw(idx);
+      val[r] = in.val(idx);
+    }
+  }
+  int32_t owner[kSortItems] = {};
+  if constexpr (Source::kOwners)
+    in.owners(base, base + kSortTile < n ? base + kSortTile : n, reinterpret_cast<uint32_t*>(stage), owner);
+  for (int d = threadIdx.x; d < kWaves * kSortBucketsMax; d += kSortBlock) (&wcnt[0][0])[d] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) key[r] = in.key(raw[r], owner[r]);
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) {
+    const int64_t idx = wbase + (int64_t)r * kWave + lane;
+    const bool valid = idx < n;
+    const int d = radix_digit(key[r], shift, mask);
+    uint64_t match = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < kSortDigitMax; ++b) {
+      if (b < nbits) {  // uniform
+        const bool bit = (d >> b) & 1;
+        const uint64_t m = __ballot(bit);
+        match &= bit ? m : ~m;
+      }
+    }
+    rank[r] = 0;
+    if (valid) {
+      const int before = __popcll(match & lt);
+      const int32_t old = wcnt[w][d];
+      rank[r] = old + before;
+      if (before == 0) wcnt[w][d] = (uint16_t)(old + __popcll(match));
+    }
+  }
+  __syncthreads();
+  {
+    // thread t: digits 2t and 2t + 1: exclusive prefixes over the waves,
+    // then the tile-wide exclusive prefix of the digit totals
+    int32_t tot[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int d = 2 * threadIdx.x + e;
+      int32_t run = 0;
+      if (d < nb) {
+#pragma unroll
+        for (int q = 0; q < kWaves; ++q) {
+          const int32_t c = wcnt[q][d];
+          wcnt[q][d] = (uint16_t)run;
+          run += c;
+        }
+      }
+      tot[e] = run;
+    }
+    int32_t all;
+    const int32_t st = block_excl_scan<int32_t, kSortBlock>(tot[0] + tot[1], scan_sh, &all);
+    if (2 * (int)threadIdx.x < nb) dstart[2 * threadIdx.x] = st;
+    if (2 * (int)threadIdx.x + 1 < nb) dstart[2 * threadIdx.x + 1] = st + tot[0];
+  }
+  __syncthreads();
+  const int64_t remain = n - base;
+  const int tile_n = remain < kSortTile ? (int)remain : kSortTile;
+  // round 1: keys in digit order, written out; their destinations kept
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) {
+    const int64_t idx = wbase + (int64_t)r * kWave + lane;
+    if (idx < n) {
+      const int d = radix_digit(key[r], shift, mask);
+      sk[dstart[d] + wcnt[w][d] + rank[r]] = key[r];
+    }
+  }
+  __syncthreads();
+  int32_t dst[kSortItems];
+#pragma unroll
+  for (int it = 0; it < kSortItems; ++it) {
+    const int i = it * kSortBlock + threadIdx.x;
+    dst[it] = 0;
+    if (i < tile_n) {
+      const K k = sk[i];
+      const int d = radix_digit(k, shift, mask);
+      dst[it] = offs[(int64_t)d * ntiles + blockIdx.x] + (i - dstart[d]);
+      out.key(dst[it], k);
+    }
+  }
+  __syncthreads();
+  // round 2: the values through the same buffer
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) {
+    const int64_t idx = wbase + (int64_t)r * kWave + lane;
+    if (idx < n) {
+      const int d = radix_digit(key[r], shift, mask);
+      stage[dstart[d] + wcnt[w][d] + rank[r]] = val[r];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < kSortItems; ++it) {
+    const int i = it * kSortBlock + threadIdx.x;
+    if (i < tile_n) out.val(dst[it], stage[i]);
+  }
+}
+
+// One pass over n pairs (below 2^31) on `nbits` bits from `shift`.
+template <class K, class Source, class Sink>
+int radix_pass(spws_ctx* ctx, const Source& in, const Sink& out, int64_t n, int shift, int nbits) {
+  const int64_t ntiles = div_up(n, kSortTile);
+  int rc = ctx->radix_hist.ensure((2 * radix_hist_entries(n) + 1) * sizeof(int32_t));
+  if (rc) return rc;
+  int32_t* hist = ctx->radix_hist.as<int32_t>();
+  int32_t* offs = hist + radix_hist_entries(n);
+  const uint32_t mask = (1u << nbits) - 1u;
+  SPWS_LAUNCH(ctx, "radix_hist", (k_radix_hist<K, Source>), dim3((unsigned)ntiles), dim3(kSortBlock), 0, in, n, shift,
+              mask, hist, ntiles);
+  rc = exclusive_scan<int32_t, int32_t>(ctx, hist, offs, ntiles << nbits);
+  if (rc) return rc;
+  SPWS_LAUNCH(ctx, "radix_scatter", (k_radix_scatter<K, Source, Sink>), dim3((unsigned)ntiles), dim3(kSortBlock), 0,
+              in, out, n, shift, mask, nbits, (const int32_t*)offs, ntiles);
+  return SPWS_OK;
+}
+
+// Sorts n pairs (0 < n < 2^31) from `in` by bits [begin_bit, end_bit), at
+// least one, into `out`: pass p writes buffer p mod 2 (keys[], vals[], n
+// entries each; the second only from three passes on), the last one `out`,
+// which may be the buffer whose turn it is.
+template <class K, class Source, class Sink>
+int radix_sort_from(spws_ctx* ctx, const Source& in, K* const (&keys)[2], double* const (&vals)[2], const Sink& out,
+                    int64_t n, int begin_bit, int end_bit) {
+  const int passes = radix_passes(end_bit - begin_bit);
+  int shift = begin_bit;
+  for (int p = 0; p < passes; ++p) {
+    // the remaining bits split evenly over the remaining passes
+    const int nbits = (int)div_up(end_bit - shift, passes - p);
+    const PairSource<K> from{keys[(p + 1) & 1], vals[(p + 1) & 1]};
+    const PairSink<K> to{keys[p & 1], vals[p & 1]};
+    int rc;
+    if (p == 0 && passes == 1) rc = radix_pass<K>(ctx, in, out, n, shift, nbits);
+    else if (p == 0) rc = radix_pass<K>(ctx, in, to, n, shift, nbits);
+    else if (p + 1 == passes) rc = radix_pass<K>(ctx, from, out, n, shift, nbits);
+    else rc = radix_pass<K>(ctx, from, to, n, shift, nbits);
+    if (rc) return rc;
+    shift += nbits;
+  }
+  return SPWS_OK;
+}
 
 }  // namespace spws

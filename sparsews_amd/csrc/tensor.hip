@@ -5,13 +5,13 @@
 //   reference (B(k,l,i) in benchmark/MTTKRP/COO_CSF_DCSR_DCSR_hash_free.h:233;
 //   its C and D factors are Bf and Cf here, given dense, row-major R wide).
 //   Bucket workspace over output rows:
-//     1. k_seg_tile_first + k_seg_owner   fiber -> root owners, then the
-//                           leaves' owner walk writes each nonzero's packed
-//                           key (i << (bj+bk) | j << bk | k) directly
-//                           (CsfKeyOut); with factor masks, leaf -> fiber
-//                           owners and k_mttkrp_keys instead.
-//     2. radix sort         stable on the i bits only: the buckets are the
-//                           output rows, CSF (j,k) order kept inside each.
+//     1. k_seg_owner        fiber -> root owners (with factor masks also
+//                           leaf -> fiber owners, and k_mttkrp_keys).
+//     2. radix sort         of packed keys (i << (bj+bk) | j << bk | k), stable
+//                           on the i bits only: the buckets are the output
+//                           rows, CSF (j,k) order kept inside each.  Its first
+//                           pass makes the keys from the CSF itself
+//                           (CsfSource); they are not stored unsorted.
 //     3. k_mttkrp_accum     each group of 16 or 32 lanes (a rank per lane)
 //                           walks a segment of the bucketed nonzeros, loading
 //                           factor rows Bf(j,:), Cf(k,:) as coalesced rows
@@ -31,15 +31,13 @@
 //   level, as in the reference's hash_il (B(k,i,j) in
 //   benchmark/TTM/COO_CSF_DCSR_hash_il.h:247), whose hash workspace is keyed
 //   on the output fiber (i,j).  Here the fibers are grouped by sorting:
-//     1. k_seg_tile_first + k_seg_owner   fiber -> root owners, then the
-//                           leaves' owner walk writes each nonzero's packed
-//                           (i, j, k) key directly (CsfKeyOut); with a U row
-//                           mask, leaf -> fiber owners and k_ttm_direct_keys
-//                           instead.  The sort reads the values straight
-//                           from the CSF.
-//     2. radix sort         stable, on the (i, j) bits only: each fiber's
-//                           nonzeros end up together and keep the CSF order,
-//                           increasing k -- the order hash_il sums them.
+//     1. k_seg_owner        fiber -> root owners (with a U row mask also
+//                           leaf -> fiber owners, and k_ttm_direct_keys).
+//     2. radix sort         of packed (i, j, k) keys, stable, on the (i, j)
+//                           bits only: each fiber's nonzeros end up together
+//                           and keep the CSF order, increasing k -- the order
+//                           hash_il sums them.  Its first pass makes the keys
+//                           and takes the values from the CSF itself.
 //     3. k_ttm_seg_starts + scan: fiber starts per segment of 32 to 128
 //                           nonzeros, so each segment knows its first fiber.
 //     4. k_ttm_accum        one 16-lane group per segment sums X * U(k,:) in
@@ -62,33 +60,11 @@
 
 namespace spws {
 
+// owner[e] = s for e in [pos[s], pos[s+1]), s in [0, nseg); pos[nseg] =
+// nitems; a tile of items per workgroup.
 constexpr int kOwnBlock = 256;
 constexpr int kOwnItems = 8;
 constexpr int kOwnTile = kOwnBlock * kOwnItems;
-
-// owner[e] = s for e in [pos[s], pos[s+1]), s in [0, nseg); pos[nseg] = nitems.
-// First the owner of every tile's first item (one thread per tile, a binary
-// search over pos: the last s with pos[s] <= e, which is the non-empty
-// segment holding e); then one tile of items per workgroup, each item's
-// owner by a binary search in the LDS slice of pos between its tile's first
-// owner and the next tile's (the owner of the tile's last item is at most
-// the latter).
-__global__ __launch_bounds__(256) void k_seg_tile_first(const int32_t* __restrict__ pos, int32_t nseg, int64_t nitems,
-                                                        int64_t ntiles, int32_t* __restrict__ first) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t > ntiles) return;
-  if (t == ntiles) {
-    first[t] = nseg - 1;
-    return;
-  }
-  const int64_t x = t * kOwnTile;
-  int32_t lo = 0, hi = nseg - 1;
-  while (lo < hi) {
-    const int32_t mid = (lo + hi + 1) >> 1;
-    if (pos[mid] <= x) lo = mid; else hi = mid - 1;
-  }
-  first[t] = lo;
-}
 
 // What k_seg_owner does with item e of segment s: store s.
 struct OwnerOut {
@@ -96,69 +72,63 @@ struct OwnerOut {
   __device__ void operator()(int64_t e, int32_t s) const { owner[e] = s; }
 };
 
-// Or, over a CSF's leaves (s = the nonzero's fiber): its packed sort key
-// (hi << (bj + bk)) | (mid << bk) | k with k = the fiber's coordinate and,
-// for TTM, hi = the root's and mid = the leaf's coordinate; for MTTKRP the
-// other way round.
-template <bool kMttkrp>
-struct CsfKeyOut {
-  const int32_t* __restrict__ fiber_root;
+// Or, over a CSF's fibers (s = the fiber's root): its part of the sort key.
+struct FiberKeyOut {
   const int32_t* __restrict__ l1_crd;
   const int32_t* __restrict__ l2_crd;
-  const int32_t* __restrict__ l3_crd;
-  int bj, bk;
-  uint64_t* __restrict__ keys;
-  __device__ void operator()(int64_t e, int32_t f) const {
-    const uint64_t root = (uint32_t)l1_crd[fiber_root[f]];
-    const uint64_t k = (uint32_t)l2_crd[f];
-    const uint64_t leaf = (uint32_t)l3_crd[e];
-    const uint64_t hi = kMttkrp ? leaf : root, mid = kMttkrp ? root : leaf;
-    keys[e] = (hi << (bj + bk)) | (mid << bk) | k;
+  int root_shift;
+  uint64_t* __restrict__ fiber_key;
+  __device__ void operator()(int64_t f, int32_t s) const {
+    fiber_key[f] = ((uint64_t)(uint32_t)l1_crd[s] << root_shift) | (uint32_t)l2_crd[f];
   }
 };
 
 template <class Out>
-__global__ __launch_bounds__(kOwnBlock) void k_seg_owner(const int32_t* __restrict__ pos, int64_t nitems,
-                                                         const int32_t* __restrict__ first, Out out) {
-  __shared__ int32_t spos[kOwnTile + 1];
-  const int64_t e0 = (int64_t)blockIdx.x * kOwnTile;
-  const int64_t e_end = e0 + kOwnTile < nitems ? e0 + kOwnTile : nitems;
-  const int32_t lo0 = first[blockIdx.x];
-  const int32_t span = first[blockIdx.x + 1] - lo0 + 1;  // candidate owners lo0 .. lo0 + span - 1
-  const bool fits = span <= kOwnTile;
-  if (fits)
-    for (int i = threadIdx.x; i < span; i += kOwnBlock) spos[i] = pos[lo0 + i];
-  __syncthreads();
-  for (int it = 0; it < kOwnItems; ++it) {
-    const int64_t e = e0 + (int64_t)it * kOwnBlock + threadIdx.x;
-    if (e >= e_end) break;
-    int32_t lo = 0, hi = span - 1;
-    if (fits) {
-      while (lo < hi) {
-        const int32_t mid = (lo + hi + 1) >> 1;
-        if (spos[mid] <= e) lo = mid; else hi = mid - 1;
-      }
-    } else {
-      while (lo < hi) {
-        const int32_t mid = (lo + hi + 1) >> 1;
-        if (pos[lo0 + mid] <= e) lo = mid; else hi = mid - 1;
-      }
-    }
-    out(e, lo0 + lo);
+__global__ __launch_bounds__(kOwnBlock) void k_seg_owner(const int32_t* __restrict__ pos, int32_t nseg, int64_t nitems,
+                                                         Out out) {
+  __shared__ uint32_t marks[kOwnTile];
+  const int64_t base = (int64_t)blockIdx.x * kOwnTile;
+  int32_t own[kOwnItems];
+  tile_owners<kOwnBlock, kOwnItems>(pos, nseg, base, base + kOwnTile < nitems ? base + kOwnTile : nitems, marks, own);
+#pragma unroll
+  for (int r = 0; r < kOwnItems; ++r) {
+    const int64_t e = base + ((threadIdx.x / kWave) * kOwnItems + r) * kWave + lane_id();
+    if (e < nitems) out(e, own[r]);
   }
 }
 
-// first: ntiles + 1 entries of scratch (ntiles = tiles of kOwnTile items).
 template <class Out>
-static int seg_owner(spws_ctx* ctx, const int32_t* pos, int32_t nseg, int64_t nitems, Out out, int32_t* first,
-                     const char* name = "seg_owner") {
+static int seg_owner(spws_ctx* ctx, const int32_t* pos, int32_t nseg, int64_t nitems, Out out) {
   if (nitems <= 0) return SPWS_OK;
-  const int64_t ntiles = div_up(nitems, kOwnTile);
-  SPWS_LAUNCH(ctx, "seg_owner", k_seg_tile_first, dim3((unsigned)div_up(ntiles + 1, 256)), dim3(256), 0, pos, nseg,
-              nitems, ntiles, first);
-  SPWS_LAUNCH(ctx, name, k_seg_owner<Out>, dim3((unsigned)ntiles), dim3(kOwnBlock), 0, pos, nitems, first, out);
+  SPWS_LAUNCH(ctx, "seg_owner", k_seg_owner<Out>, dim3((unsigned)div_up(nitems, kOwnTile)), dim3(kOwnBlock), 0, pos,
+              nseg, nitems, out);
   return SPWS_OK;
 }
+
+// A CSF's nonzeros as the sort's first pass reads them: nonzero e of fiber f
+// has the key (hi << (bj + bk)) | (mid << bk) | k with k = the fiber's
+// coordinate and, for TTM, hi = the root's and mid = the leaf's coordinate;
+// for MTTKRP the other way round.  The sort starts at the leaf's bits, so the
+// first pass's histogram reads the leaves' coordinates alone, unless its digit
+// reaches into the root's (kRootDigits: TTM with fewer leaf bits than that).
+template <bool kMttkrp, bool kRootDigits>
+struct CsfSource {
+  static constexpr bool kOwners = true, kOwnedDigits = kRootDigits;
+  using Raw = uint32_t;
+  const uint64_t* __restrict__ fiber_key;  // per fiber, the key's part from its root and its own coordinate
+  const int32_t* __restrict__ l3_pos;
+  const int32_t* __restrict__ l3_crd;
+  const double* __restrict__ vals;
+  int32_t nfibers;
+  int leaf_shift;  // the leaf's bits in the key
+  __device__ uint32_t raw(int64_t e) const { return (uint32_t)l3_crd[e]; }
+  __device__ double val(int64_t e) const { return vals[e]; }
+  __device__ uint64_t digit_bits(uint32_t leaf) const { return (uint64_t)leaf << leaf_shift; }
+  __device__ void owners(int64_t base, int64_t end, uint32_t* marks, int32_t (&own)[kSortItems]) const {
+    tile_owners<kSortBlock, kSortItems>(l3_pos, nfibers, base, end, marks, own);
+  }
+  __device__ uint64_t key(uint32_t leaf, int32_t f) const { return fiber_key[f] | ((uint64_t)leaf << leaf_shift); }
+};
 
 static int bits_of(int64_t v) {  // bits for values in [0, v)
   int b = 0;
@@ -771,37 +741,39 @@ __global__ __launch_bounds__(256) void k_ttm_direct_keys(int64_t nnz, const int3
 
 static int csf_owners(spws_ctx* ctx, const Csf3& x, int32_t** leaf_fiber, int32_t** fiber_root) {
   int rc;
-  // obuf[0]: the nonzeros' fibers, then the tile owners both passes use in
-  // turn (nfibers <= nnz)
-  const size_t nz = (size_t)(x.nnz > 0 ? x.nnz : 1);
-  const size_t tiles = (size_t)div_up((int64_t)nz, kOwnTile) + 1;
-  if ((rc = ctx->obuf[0].ensure((nz + tiles) * 4)) ||
+  if ((rc = ctx->obuf[0].ensure((size_t)(x.nnz > 0 ? x.nnz : 1) * 4)) ||
       (rc = ctx->obuf[1].ensure((size_t)(x.nfibers > 0 ? x.nfibers : 1) * 4)))
     return rc;
   *leaf_fiber = ctx->obuf[0].as<int32_t>();
   *fiber_root = ctx->obuf[1].as<int32_t>();
-  int32_t* first = *leaf_fiber + nz;
-  if ((rc = seg_owner(ctx, x.l3_pos, x.nfibers, x.nnz, OwnerOut{*leaf_fiber}, first))) return rc;
-  return seg_owner(ctx, x.l2_pos, x.nroots, x.nfibers, OwnerOut{*fiber_root}, first);
+  if ((rc = seg_owner(ctx, x.l3_pos, x.nfibers, x.nnz, OwnerOut{*leaf_fiber}))) return rc;
+  return seg_owner(ctx, x.l2_pos, x.nroots, x.nfibers, OwnerOut{*fiber_root});
 }
 
-// The nonzeros' packed sort keys straight from the CSF (CsfKeyOut): the
-// fibers' roots first, then the keys from the leaves' owner walk, with no
-// per-nonzero fiber array.
+// The nonzeros (at least one) sorted by the key's bits [begin_bit, end_bit)
+// straight from the CSF, with no array of unsorted keys: into ctx->keys[i] and
+// ctx->vals[i] for the *i returned.
 template <bool kMttkrp>
-static int csf_keys(spws_ctx* ctx, const Csf3& x, int bj, int bk, uint64_t* keys) {
+static int csf_sort(spws_ctx* ctx, const Csf3& x, int bj, int bk, int begin_bit, int end_bit, int* i) {
   int rc;
-  const size_t nz = (size_t)(x.nnz > 0 ? x.nnz : 1);
-  const size_t tiles = (size_t)div_up((int64_t)nz, kOwnTile) + 1;
-  if ((rc = ctx->obuf[0].ensure(tiles * 4)) ||
-      (rc = ctx->obuf[1].ensure((size_t)(x.nfibers > 0 ? x.nfibers : 1) * 4)))
+  if ((rc = ctx->obuf[1].ensure((size_t)(x.nfibers > 0 ? x.nfibers : 1) * 8))) return rc;
+  uint64_t* fiber_key = ctx->obuf[1].as<uint64_t>();
+  const int leaf_shift = kMttkrp ? bj + bk : bk;
+  if ((rc = seg_owner(ctx, x.l2_pos, x.nroots, x.nfibers,
+                      FiberKeyOut{x.l1_crd, x.l2_crd, kMttkrp ? bk : bj + bk, fiber_key})))
     return rc;
-  int32_t* first = ctx->obuf[0].as<int32_t>();
-  int32_t* fiber_root = ctx->obuf[1].as<int32_t>();
-  if ((rc = seg_owner(ctx, x.l2_pos, x.nroots, x.nfibers, OwnerOut{fiber_root}, first))) return rc;
-  return seg_owner(ctx, x.l3_pos, x.nfibers, x.nnz,
-                   CsfKeyOut<kMttkrp>{fiber_root, x.l1_crd, x.l2_crd, x.l3_crd, bj, bk, keys}, first,
-                   kMttkrp ? "mttkrp_keys" : "ttm_keys");
+  uint64_t* const keys[2] = {ctx->keys[0].as<uint64_t>(), ctx->keys[1].as<uint64_t>()};
+  double* const vals[2] = {ctx->vals[0].as<double>(), ctx->vals[1].as<double>()};
+  const int passes = radix_passes(end_bit - begin_bit);
+  *i = (passes - 1) & 1;
+  const PairSink<uint64_t> out{keys[*i], vals[*i]};
+  if (!kMttkrp && div_up(end_bit - begin_bit, passes) > bj)
+    return radix_sort_from<uint64_t>(
+        ctx, CsfSource<kMttkrp, !kMttkrp>{fiber_key, x.l3_pos, x.l3_crd, x.vals, x.nfibers, leaf_shift}, keys, vals,
+        out, x.nnz, begin_bit, end_bit);
+  return radix_sort_from<uint64_t>(
+      ctx, CsfSource<kMttkrp, false>{fiber_key, x.l3_pos, x.l3_crd, x.vals, x.nfibers, leaf_shift}, keys, vals, out,
+      x.nnz, begin_bit, end_bit);
 }
 
 // mB / mC (device, J and K entries; both null or both set): per factor row,
@@ -839,25 +811,24 @@ static int mttkrp_run(spws_ctx* ctx, const Csf3& x, int32_t I, int32_t J, int32_
   if (masked) SPWS_HIP(hipMemsetAsync(rmask, 0, ii * 8 + 8, s));
   int64_t kept = x.nnz;
   if (x.nnz > 0) {
-    uint64_t* keys = ctx->keys[0].as<uint64_t>();
-    double* vals = ctx->vals[0].as<double>();
+    int in = 0;  // which of the two buffers holds the sorted nonzeros
     if (masked) {
       int32_t *leaf_fiber, *fiber_root;
       if ((rc = csf_owners(ctx, x, &leaf_fiber, &fiber_root))) return rc;
       const unsigned g = (unsigned)std::min<int64_t>(div_up(x.nnz, 256), 65536);
       SPWS_LAUNCH(ctx, "mttkrp_keys", k_mttkrp_keys<true>, dim3(g), dim3(256), 0, x.nnz, leaf_fiber, fiber_root,
-                  x.l1_crd, x.l2_crd, x.l3_crd, bj, bk, keys, mB, mC, (uint64_t)I, dropped);
-    } else if ((rc = csf_keys<true>(ctx, x, bj, bk, keys))) {
+                  x.l1_crd, x.l2_crd, x.l3_crd, bj, bk, ctx->keys[0].as<uint64_t>(), mB, mC, (uint64_t)I, dropped);
+      bool in_alt = false;
+      if ((rc = radix_sort_pairs<uint64_t>(ctx, ctx->keys[0].as<uint64_t>(), ctx->vals[0].as<double>(),
+                                           ctx->keys[1].as<uint64_t>(), ctx->vals[1].as<double>(), x.nnz, bj + bk,
+                                           bj + bk + bi, &in_alt, x.vals)))
+        return rc;
+      in = in_alt ? 1 : 0;
+    } else if ((rc = csf_sort<true>(ctx, x, bj, bk, bj + bk, bj + bk + bi, &in))) {
       return rc;
     }
-    bool in_alt = false;
-    if ((rc = radix_sort_pairs<uint64_t>(ctx, keys, vals, ctx->keys[1].as<uint64_t>(), ctx->vals[1].as<double>(),
-                                         x.nnz, bj + bk, bj + bk + bi, &in_alt, x.vals)))
-      return rc;
-    if (in_alt) {
-      keys = ctx->keys[1].as<uint64_t>();
-      vals = ctx->vals[1].as<double>();
-    }
+    const uint64_t* keys = ctx->keys[in].as<uint64_t>();
+    const double* vals = ctx->vals[in].as<double>();
     if (masked) {
       // the nonzeros that take part come first after the sort
       int64_t* hd = ctx->host_meta.as<int64_t>();
@@ -1016,31 +987,30 @@ static int ttm_run(spws_ctx* ctx, const Csf3& x, int32_t I, int32_t J, int32_t K
   if (x.nnz > 0 && direct) {
     // one sort of the nonzeros on (i, j, k)
     const int bk = bk_all;
-    uint64_t* nkeys = ctx->keys[0].as<uint64_t>();
-    double* nvals = ctx->vals[0].as<double>();
-    const unsigned g = (unsigned)std::min<int64_t>(div_up(x.nnz, 256), 65536);
+    // the sort covers (i, j) only: within an i slice the CSF order already
+    // has each (i, j)'s nonzeros in increasing k, and the sort is stable
+    int in = 0;  // which of the two buffers holds the sorted nonzeros
     unsigned long long* dropped = nullptr;
     if (masked) {
+      const unsigned g = (unsigned)std::min<int64_t>(div_up(x.nnz, 256), 65536);
       int32_t *leaf_fiber, *fiber_root;
       if ((rc = csf_owners(ctx, x, &leaf_fiber, &fiber_root))) return rc;
       if ((rc = ctx->obuf[6].ensure(256))) return rc;
       dropped = ctx->obuf[6].as<unsigned long long>();
       SPWS_HIP(hipMemsetAsync(dropped, 0, 8, s));
       SPWS_LAUNCH(ctx, "ttm_keys", k_ttm_direct_keys<true>, dim3(g), dim3(256), 0, x.nnz, leaf_fiber, fiber_root,
-                  x.l1_crd, x.l2_crd, x.l3_crd, bj, bk, nkeys, umask, (uint64_t)I, dropped);
-    } else if ((rc = csf_keys<false>(ctx, x, bj, bk, nkeys))) {
+                  x.l1_crd, x.l2_crd, x.l3_crd, bj, bk, ctx->keys[0].as<uint64_t>(), umask, (uint64_t)I, dropped);
+      bool alt = false;
+      if ((rc = radix_sort_pairs<uint64_t>(ctx, ctx->keys[0].as<uint64_t>(), ctx->vals[0].as<double>(),
+                                           ctx->keys[1].as<uint64_t>(), ctx->vals[1].as<double>(), x.nnz, bk,
+                                           bi + bj + bk, &alt, x.vals)))
+        return rc;
+      in = alt ? 1 : 0;
+    } else if ((rc = csf_sort<false>(ctx, x, bj, bk, bk, bi + bj + bk, &in))) {
       return rc;
     }
-    // the sort covers (i, j) only: within an i slice the CSF order already
-    // has each (i, j)'s nonzeros in increasing k, and the sort is stable
-    bool alt = false;
-    if ((rc = radix_sort_pairs<uint64_t>(ctx, nkeys, nvals, ctx->keys[1].as<uint64_t>(), ctx->vals[1].as<double>(),
-                                         x.nnz, bk, bi + bj + bk, &alt, x.vals)))
-      return rc;
-    if (alt) {
-      nkeys = ctx->keys[1].as<uint64_t>();
-      nvals = ctx->vals[1].as<double>();
-    }
+    const uint64_t* nkeys = ctx->keys[in].as<uint64_t>();
+    const double* nvals = ctx->vals[in].as<double>();
     // the nonzeros that take part come first after the sort
     int64_t kept = x.nnz;
     if (masked) {

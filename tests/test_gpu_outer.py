@@ -434,6 +434,32 @@ def test_device_transpose(ctx, m, n, lo, hi, seed):
     np.testing.assert_array_equal(T.vals, O.vals)
 
 
+# one, two and three passes of the sort; rows longer than its tiles of 4,096,
+# tiles that start and end with runs of empty rows, rows that end on a tile
+@pytest.mark.parametrize("n", [1, 2, 512, 513, 262_145])
+@pytest.mark.parametrize("pos64", [False, True])
+def test_transpose_tiles_and_passes(ctx, n, pos64):
+    print(f"case: transpose tiles n={n} int64 positions {pos64}", flush=True)
+    from sparsews_amd.device import DeviceCSR, DeviceCSR64, csr64_transpose, csr_transpose
+    rng = np.random.default_rng(n)
+    lengths = np.concatenate([np.zeros(9000), [4096, 0, 0, 4095, 1], np.zeros(70), [9000, 0, 1, 4000], np.ones(5000),
+                              np.zeros(300), [3], np.zeros(9000)]).astype(np.int64)
+    pos = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    # columns may repeat within a row: the sort keeps their order
+    crd = np.concatenate([np.sort(rng.integers(0, n, c)) for c in lengths if c]).astype(np.int32)
+    A = CSR(len(lengths), n, pos, crd, rng.uniform(-1, 1, len(crd)))
+    if pos64:
+        dA = DeviceCSR64(A.nrows, n, A.nnz, DeviceArray.from_host(ctx, pos.astype(np.int64)),
+                         DeviceArray.from_host(ctx, crd), DeviceArray.from_host(ctx, A.vals))
+        T = csr64_transpose(ctx, dA).download()
+    else:
+        T = csr_transpose(ctx, DeviceCSR.upload(ctx, A)).download()
+    order = np.argsort(crd, kind="stable")
+    np.testing.assert_array_equal(T.pos, np.concatenate([[0], np.cumsum(np.bincount(crd, minlength=n))]))
+    np.testing.assert_array_equal(T.crd, np.repeat(np.arange(A.nrows), lengths)[order])
+    np.testing.assert_array_equal(T.vals, A.vals[order])
+
+
 @pytest.mark.parametrize("n", [1, 3, 4, 4095, 4096, 4097, 8193, 16_384, 16_385, 20_483, 65_535, 65_536, 65_537, 200_001])
 def test_prefix_sum_lengths(ctx, n):
     """Row pointers (a prefix sum of n counts, most of them zero at the larger

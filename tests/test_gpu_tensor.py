@@ -113,6 +113,33 @@ def test_mttkrp_factor_over_4_gib(ctx):
     check_mttkrp(ctx, dims, idx, rng.uniform(-1, 1, (dims[1], R)), Cf, 7)
 
 
+# leaf modes of fewer bits than the sort's first digit (it then reaches into
+# the root's bits), of as many and of more; one to three passes; nonzero counts
+# at the edges of its tiles of 4,096; fibers longer than a tile
+@pytest.mark.parametrize("dims,nnz", [
+    ((70_000, 1, 9), 5000), ((70_000, 2, 9), 4097), ((3000, 5, 700), 8192), ((300, 513, 40), 4095), ((2, 2, 50), 150),
+    ((5, 20_000, 3), 60_000), ((1, 1, 1), 1), ((40, 262_145, 3), 4096),
+])
+def test_tensor_sort_sources(ctx, dims, nnz):
+    print(f"case: sort from the CSF dims={dims} nnz={nnz}", flush=True)
+    rng = np.random.default_rng(nnz)
+    I, J, K = dims
+    at = np.unique(rng.choice(I * J * K, nnz, replace=False)) if I * J * K < 1 << 22 else \
+        np.unique(rng.integers(0, I * J * K, 2 * nnz))
+    at = np.sort(rng.permutation(at)[:nnz])
+    X = gen.COO3(dims, np.stack([at // (J * K), at // K % J, at % K], axis=1).astype(np.int32),
+                 rng.uniform(-1, 1, len(at)))
+    U = rng.uniform(-1, 1, (K, 7))
+    fi, fj, Y = run_ttm(ctx, X, U, method=1)
+    fib, start = np.unique(at // K, return_index=True)  # (i, j) and its first nonzero
+    np.testing.assert_array_equal(fi, fib // J)
+    np.testing.assert_array_equal(fj, fib % J)
+    t = X.vals[:, None] * U[X.idx[:, 2]]
+    assert oracle.max_value_error(Y.ravel(), np.add.reduceat(t, start, axis=0).ravel(),
+                                  np.add.reduceat(np.abs(t), start, axis=0).ravel()) <= TOL
+    check_mttkrp(ctx, dims, X.idx, rng.uniform(-1, 1, (J, 7)), U, 9)
+
+
 def test_mttkrp_taco_entry():
     print("case: mttkrp taco entry", flush=True)
     X = gen.zipf_coo3((120, 90, 70), 3000, (1.5, 1.5, 1.5), 12, 5, 0.0, 1.0)
