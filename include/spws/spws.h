@@ -61,7 +61,7 @@ typedef struct {
   int64_t rows_per_path[8]; /* rows sent to each row-wise path (index = force_path id), [6] = empty */
   int64_t chunks;           /* outer product: output-row chunks processed */
   int64_t sort_bits;        /* outer product: key bits radix-sorted per chunk (LSD method) */
-  int64_t outer_method;     /* outer product: 1 LSD radix sort, 2 row/window buckets */
+  int64_t outer_method;     /* outer product: the method that ran (spws_ctx_set_outer_method), 5 by rows */
   int64_t window_bits;      /* outer product, bucket method: log2 of the column window */
 } spws_stats;
 
@@ -159,8 +159,10 @@ int spws_ctx_set_outer_chunking(spws_ctx* ctx, int64_t max_products, int32_t max
  *   4  as 3, the products added into the LDS window by atomic adds (no
  *      ordering of equal columns): sums reassociated within the 1e-12 bar,
  *      not reproducible bit for bit;
- *   0  automatic (4 unless the windows would be too sparse or too many,
- *      then 1).
+ *   0  automatic: 4 unless the windows would be too sparse or too many; then
+ *      by rows (A's columns transposed into rows, then the row-wise product;
+ *      outputs of at most 2^17 columns; reported as method 5, sums in any
+ *      order as 4), else 1.
  * window_log2 sets the column window of methods 2-4 (6..11; 0 = chosen
  * from the average products per row).  Methods 1-3 sum each entry in
  * increasing j and give identical results. */

@@ -170,6 +170,14 @@ int exclusive_scan(spws_ctx* ctx, const Tin* in, Tout* out, int64_t n);
 // Bytes of ctx->scan_tmp that exclusive_scan of n values of elem_bytes uses.
 size_t scan_scratch_bytes(int64_t n, size_t elem_bytes);
 
+// The m x n CSR's transpose in the given device arrays, and the row-wise
+// product C = A * B (in ctx->out_pos, out_crd, out_val), for other drivers.
+int csr_transpose_run(spws_ctx* ctx, int32_t m, int32_t n, int64_t nnz, const int32_t* pos, const int32_t* crd,
+                      const double* vals, int32_t* out_pos, int32_t* out_crd, double* out_vals);
+int rowwise_product(spws_ctx* ctx, int32_t m, int32_t k, int32_t n, const int32_t* A_pos, const int32_t* A_crd,
+                    const double* A_vals, const int32_t* B_pos, const int32_t* B_crd, const double* B_vals,
+                    int64_t* nnz);
+
 // Resolves the no-allocation entry point's scratch address on `device`
 // (current), once per device; spws_ctx_create calls it for its device.
 int noalloc_scratch_init(int device);

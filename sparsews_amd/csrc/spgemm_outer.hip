@@ -11,6 +11,8 @@
 //   k_outer_match     j co-iteration as a parallel search: for each stored
 //                     column of A, the matching stored row of B (or none).
 //   k_outer_row_ub    products per output row: ub_i += |B(j,:)| over A(i,j).
+//   k_outer_stats     sums and maxima over the rows, read by the host, which
+//                     picks the method.
 //   -- host: prefix of ub, row chunks [r0, r1) bounded by products and by the
 //      key width (32-bit keys while rows*2^kb fits).
 //   per chunk:
@@ -28,7 +30,10 @@
 // Values of each entry are summed in increasing j, exactly Gustavson's
 // left-to-right order.
 //
-// Second sort method (the default): an MSD radix sort whose first digit is
+// The automatic choice replaces that sort by rows (outer_rows) where it may:
+// A's columns are transposed into rows and the row-wise product computes C.
+//
+// Second sort method: an MSD radix sort whose first digit is
 // (row i, column window k >> s).  The digit counts need no pass over the
 // products: the products of A(i,j) that land in window w are the entries of
 // B(j,:) in that window, a range found by binary search in the sorted row.
@@ -86,6 +91,61 @@ __global__ __launch_bounds__(256) void k_outer_match(int32_t a_ncols, const int3
   }
   match[ja] = jb;
   blen[ja] = jb >= 0 ? B2_pos[jb + 1] - B2_pos[jb] : 0;
+}
+
+// What the host decides the method on: sums and maxima over the rows' products
+// and matched A entries, and the operands' entry counts.
+enum OuterStat { kOsProducts, kOsBusyRows, kOsPairs, kOsMaxPairs, kOsNnzA, kOsNnzB, kOsCount };
+
+__global__ __launch_bounds__(256) void k_outer_stats(int32_t m, const int64_t* __restrict__ row_ub,
+                                                     const int32_t* __restrict__ row_pairs,
+                                                     const int32_t* __restrict__ A_end,
+                                                     const int32_t* __restrict__ B_end,
+                                                     unsigned long long* __restrict__ out) {
+  int64_t products = 0, busy = 0, pairs = 0;
+  int32_t most = 0;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t u = row_ub[i];
+    const int32_t p = row_pairs[i];
+    products += u;
+    busy += u > 0;
+    pairs += p;
+    most = max(most, p);
+  }
+  products = wave_sum(products);
+  busy = wave_sum(busy);
+  pairs = wave_sum(pairs);
+  most = wave_max(most);
+  if (lane_id() == 0 && busy) {
+    atomicAdd(&out[kOsProducts], (unsigned long long)products);
+    atomicAdd(&out[kOsBusyRows], (unsigned long long)busy);
+    atomicAdd(&out[kOsPairs], (unsigned long long)pairs);
+    atomicMax(&out[kOsMaxPairs], (unsigned long long)most);
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    out[kOsNnzA] = A_end ? (unsigned long long)*A_end : 0;
+    out[kOsNnzB] = B_end ? (unsigned long long)*B_end : 0;
+  }
+}
+
+// For the row-wise method: A's column positions become B's row positions (an
+// unmatched column the empty row b_nrows, added behind B's row pointers).
+__global__ __launch_bounds__(256) void k_outer_to_rows(int64_t nnz, int32_t* __restrict__ crd,
+                                                       const int32_t* __restrict__ match, int32_t b_nrows,
+                                                       const int32_t* __restrict__ B2_pos,
+                                                       int32_t* __restrict__ B_pos) {
+  const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t e = t0; e < nnz; e += step) {
+    const int32_t jb = match[crd[e]];
+    crd[e] = jb >= 0 ? jb : b_nrows;
+  }
+  for (int64_t q = t0; q < (int64_t)b_nrows + 2; q += step) B_pos[q] = B2_pos[q <= b_nrows ? q : b_nrows];
+}
+
+__global__ __launch_bounds__(256) void k_widen_pos(int64_t n, const int32_t* __restrict__ in,
+                                                   int64_t* __restrict__ out) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    out[i] = in[i];
 }
 
 // One wavefront per stored column of A (columns range from 1 to ~2e4 rows).
@@ -1724,15 +1784,13 @@ constexpr int kFzNumWavesPerCu = 8;   // k_fz_rows<true>: bounded by the LDS win
 // within a row), one record per entry, the symbolic pass and its prefix
 // (exact row pointers, and an output allocated to the exact size), then the
 // numeric pass writing every entry in place.
-static int outer_fused(spws_ctx* ctx, const OuterArgs& a, const std::vector<int64_t>& pair_prefix,
-                       const int32_t* row_pairs, int s, bool ordered, bool off32, int64_t* nnz_out) {
+static int outer_fused(spws_ctx* ctx, const OuterArgs& a, int64_t En64, const int32_t* row_pairs, int s, bool ordered, bool off32, int64_t* nnz_out) {
   hipStream_t st = ctx->stream;
   int rc;
   const int32_t m = a.m;
   const int32_t na = a.a_ncols;
   const size_t nac = (size_t)(na > 0 ? na : 1);
   const int32_t W = (int32_t)std::max<int64_t>(1, div_up((int64_t)a.n, (int64_t)1 << s));
-  const int64_t En64 = pair_prefix[m];
   SPWS_REQUIRE(En64 < ((int64_t)1 << 31), SPWS_ERR_UNSUPPORTED, "%lld matched A entries exceed the int32 range",
                (long long)En64);
   const int32_t En = (int32_t)En64;
@@ -1848,6 +1906,43 @@ static int outer_fused(spws_ctx* ctx, const OuterArgs& a, const std::vector<int6
   return SPWS_OK;
 }
 
+// The product by rows: A's columns transposed into rows, then the row-wise
+// product with B (whose int32 row pointers are widened to the outer product's).
+constexpr int32_t kOuterRowsCols = 1 << 17;  // columns at most (the row kernels' bitmap)
+
+static int outer_rows(spws_ctx* ctx, const OuterArgs& a, int64_t a_nnz, int64_t* nnz_out) {
+  int rc;
+  const size_t nn = (size_t)(a_nnz > 0 ? a_nnz : 1);
+  if ((rc = ctx->tr_out[0].ensure(((size_t)a.m + 1) * 4)) || (rc = ctx->tr_out[1].ensure(nn * 4)) ||
+      (rc = ctx->tr_out[2].ensure(nn * 8)))
+    return rc;
+  int32_t* Ap = ctx->tr_out[0].as<int32_t>();
+  int32_t* Ai = ctx->tr_out[1].as<int32_t>();
+  double* Ax = ctx->tr_out[2].as<double>();
+  if ((rc = csr_transpose_run(ctx, a.a_ncols, a.m, a_nnz, a.A2_pos, a.A2_crd, a.Ax, Ap, Ai, Ax))) return rc;
+  const int32_t* Bp = a.B2_pos;
+  int32_t k = a.b_nrows;
+  // stored columns and rows with the same positions need no lookup
+  if (a.A1_crd || a.B1_crd || a.a_ncols > a.b_nrows) {
+    if ((rc = ctx->obuf[3].ensure(((size_t)a.b_nrows + 2) * 4))) return rc;
+    SPWS_LAUNCH(ctx, "outer_to_rows", k_outer_to_rows,
+                dim3((unsigned)std::min<int64_t>(div_up(std::max<int64_t>(a_nnz, (int64_t)a.b_nrows + 2), 256), 16384)),
+                dim3(256), 0, a_nnz, Ai, (const int32_t*)ctx->obuf[0].as<int32_t>(), a.b_nrows, a.B2_pos,
+                ctx->obuf[3].as<int32_t>());
+    Bp = ctx->obuf[3].as<int32_t>();
+    ++k;
+  }
+  if ((rc = rowwise_product(ctx, a.m, k, a.n, Ap, Ai, Ax, Bp, a.B2_crd, a.Bx, nnz_out))) return rc;
+  ctx->stats.outer_method = 5;
+  if ((rc = ctx->obuf[5].ensure(((size_t)a.m + 1) * 8))) return rc;
+  SPWS_LAUNCH(ctx, "widen_pos", k_widen_pos, dim3((unsigned)std::min<int64_t>(div_up((int64_t)a.m + 1, 256), 4096)),
+              dim3(256), 0, (int64_t)a.m + 1, (const int32_t*)ctx->out_pos.as<int32_t>(),
+              ctx->obuf[5].as<int64_t>());
+  std::swap(ctx->out_pos, ctx->obuf[5]);
+  SPWS_HIP(hipStreamSynchronize(ctx->stream));
+  return SPWS_OK;
+}
+
 static int outer_run(spws_ctx* ctx, const OuterArgs& a, int64_t* nnz_out) {
   int rc = ctx_activate(ctx);
   if (rc) return rc;
@@ -1861,13 +1956,15 @@ static int outer_run(spws_ctx* ctx, const OuterArgs& a, int64_t* nnz_out) {
   const int32_t m = a.m;
   const size_t nac = (size_t)(a.a_ncols > 0 ? a.a_ncols : 1);
   const size_t mm = (size_t)(m > 0 ? m : 1);
+  // the statistics follow the rows' products
   if ((rc = ctx->obuf[0].ensure(nac * 4)) || (rc = ctx->obuf[1].ensure(nac * 4)) ||
-      (rc = ctx->row_ub.ensure(mm * 8)) || (rc = ctx->obuf[7].ensure(mm * 4)))
+      (rc = ctx->row_ub.ensure((mm + kOsCount) * 8)) || (rc = ctx->obuf[7].ensure(mm * 4)))
     return rc;
   int32_t* match = ctx->obuf[0].as<int32_t>();
   int32_t* blen = ctx->obuf[1].as<int32_t>();
   int32_t* row_pairs = ctx->obuf[7].as<int32_t>();
-  SPWS_HIP(hipMemsetAsync(ctx->row_ub.ptr, 0, mm * 8, s));
+  unsigned long long* stat = ctx->row_ub.as<unsigned long long>() + mm;
+  SPWS_HIP(hipMemsetAsync(ctx->row_ub.ptr, 0, (mm + kOsCount) * 8, s));
   SPWS_HIP(hipMemsetAsync(row_pairs, 0, mm * 4, s));
   if (a.a_ncols > 0) {
     const unsigned g = (unsigned)div_up(a.a_ncols, 256);
@@ -1877,22 +1974,15 @@ static int outer_run(spws_ctx* ctx, const OuterArgs& a, int64_t* nnz_out) {
     SPWS_LAUNCH(ctx, "outer_row_ub", k_outer_row_ub, dim3(g2), dim3(256), 0, a.a_ncols, a.A2_pos, a.A2_crd, blen,
                 (unsigned long long*)ctx->row_ub.ptr, row_pairs);
   }
-  std::vector<int64_t> ub(mm), prefix((size_t)m + 1, 0), pair_prefix((size_t)m + 1, 0);
-  std::vector<int32_t> pairs(mm);
-  int32_t b_nnz = 0;  // B's entries (the fused method's offset width)
-  if (m > 0) {
-    SPWS_HIP(hipMemcpyAsync(ub.data(), ctx->row_ub.ptr, (size_t)m * 8, hipMemcpyDeviceToHost, s));
-    SPWS_HIP(hipMemcpyAsync(pairs.data(), row_pairs, (size_t)m * 4, hipMemcpyDeviceToHost, s));
-    if (a.b_nrows > 0) SPWS_HIP(hipMemcpyAsync(&b_nnz, a.B2_pos + a.b_nrows, 4, hipMemcpyDeviceToHost, s));
-    SPWS_HIP(hipStreamSynchronize(s));
-  }
-  int64_t busy_rows = 0;
-  for (int32_t i = 0; i < m; ++i) {
-    prefix[i + 1] = prefix[i] + ub[i];
-    pair_prefix[i + 1] = pair_prefix[i] + pairs[i];
-    busy_rows += ub[i] > 0;
-  }
-  ctx->stats.products = prefix[m];
+  SPWS_LAUNCH(ctx, "outer_stats", k_outer_stats, dim3((unsigned)std::min<int64_t>(div_up(m > 0 ? m : 1, 1024), 64)),
+              dim3(256), 0, m, (const int64_t*)ctx->row_ub.as<int64_t>(), (const int32_t*)row_pairs,
+              a.a_ncols > 0 ? a.A2_pos + a.a_ncols : nullptr, a.b_nrows > 0 ? a.B2_pos + a.b_nrows : nullptr, stat);
+  int64_t* hs = ctx->host_meta.as<int64_t>() + 128;
+  SPWS_HIP(hipMemcpyAsync(hs, stat, kOsCount * 8, hipMemcpyDeviceToHost, s));
+  SPWS_HIP(hipStreamSynchronize(s));
+  const int64_t products = hs[kOsProducts], busy_rows = hs[kOsBusyRows], matched = hs[kOsPairs];
+  const int64_t max_pairs = hs[kOsMaxPairs], a_nnz = hs[kOsNnzA], b_nnz = hs[kOsNnzB];
+  ctx->stats.products = products;
   const int64_t max_products = ctx->outer_max_products > 0 ? ctx->outer_max_products : ((int64_t)1 << 30);
   const int64_t user_rows = ctx->outer_max_rows > 0 ? ctx->outer_max_rows : INT32_MAX;
 
@@ -1906,25 +1996,50 @@ static int outer_run(spws_ctx* ctx, const OuterArgs& a, int64_t* nnz_out) {
   int wlog = ctx->outer_window_log2;
   if (wlog == 0) {
     // about 1024 products per (row, window) bucket on average
-    const double avg = busy_rows > 0 ? (double)prefix[m] / (double)busy_rows : 1.0;
+    const double avg = busy_rows > 0 ? (double)products / (double)busy_rows : 1.0;
     const double want = 1024.0 * (double)std::max(a.n, 1) / std::max(avg, 1.0);
     wlog = kBkMinLog2;
     while (wlog < kBkMaxLog2 && (double)((int64_t)1 << wlog) * 1.41421356 < want) ++wlog;
   }
   const int64_t W = std::max<int64_t>(1, div_up((int64_t)a.n, (int64_t)1 << wlog));
   if (method == 0) {
-    const double per_bucket = busy_rows > 0 ? (double)prefix[m] / ((double)busy_rows * (double)W) : 0.0;
-    int32_t max_pairs = 0;
-    for (int32_t i = 0; i < m; ++i) max_pairs = std::max(max_pairs, pairs[i]);
+    const double per_bucket = busy_rows > 0 ? (double)products / ((double)busy_rows * (double)W) : 0.0;
     const int fused = ctx->outer_auto_ordered ? 3 : 4;
-    method = (per_bucket >= 64.0 && W <= 4096 && (int64_t)max_pairs * W <= ((int64_t)1 << 28)) ? fused : 1;
+    method = (per_bucket >= 64.0 && W <= 4096 && max_pairs * W <= ((int64_t)1 << 28)) ? fused : 1;
+    // Too few products per window: by rows, where the order of the sums may
+    // change and the row kernels' column bitmap covers the output.  2,000
+    // rows of 8 squared (128k products): 276 us by the sort, 196 by rows;
+    // 30,000 rows of 2..32 (8.7M products): 2,770 and 370.
+    if (method == 1 && !ctx->outer_auto_ordered && ctx->outer_max_products == 0 && ctx->outer_max_rows == 0 &&
+        a.n <= kOuterRowsCols && products <= INT32_MAX && ctx->rw.force_path < 0 && m > 0 && a.a_ncols > 0 &&
+        a.b_nrows > 0 && a.b_nrows < INT32_MAX - 1)
+      method = 5;
+  }
+  if (method == 5) {
+    if ((rc = outer_rows(ctx, a, a_nnz, nnz_out))) return rc;
+    ctx->stats.nnz = *nnz_out;
+    return SPWS_OK;
+  }
+  // the methods by chunks of output rows need every row's products and
+  // matched entries on the host
+  std::vector<int64_t> prefix((size_t)m + 1, 0), pair_prefix((size_t)m + 1, 0);
+  if (m > 0 && (method == 1 || method == 2)) {
+    std::vector<int64_t> ub(mm);
+    std::vector<int32_t> pairs(mm);
+    SPWS_HIP(hipMemcpyAsync(ub.data(), ctx->row_ub.ptr, (size_t)m * 8, hipMemcpyDeviceToHost, s));
+    SPWS_HIP(hipMemcpyAsync(pairs.data(), row_pairs, (size_t)m * 4, hipMemcpyDeviceToHost, s));
+    SPWS_HIP(hipStreamSynchronize(s));
+    for (int32_t i = 0; i < m; ++i) {
+      prefix[i + 1] = prefix[i] + ub[i];
+      pair_prefix[i + 1] = pair_prefix[i] + pairs[i];
+    }
   }
   if (method == 3 || method == 4) {
     // 32-bit byte offsets into B's values while B has fewer than 2^29
     // entries; SPWS_OUTER_WIDE_OFFSETS=1 takes the 64-bit addresses anyway
     const char* wide = getenv("SPWS_OUTER_WIDE_OFFSETS");
     const bool off32 = b_nnz < (1 << 29) && !(wide && wide[0] == '1');
-    rc = outer_fused(ctx, a, pair_prefix, row_pairs, wlog, method == 3, off32, nnz_out);
+    rc = outer_fused(ctx, a, matched, row_pairs, wlog, method == 3, off32, nnz_out);
   } else if (method == 2) {
     rc = outer_chunks_bucket(ctx, a, prefix, pair_prefix, row_pairs, wlog, max_products,
                              (int32_t)std::min<int64_t>(user_rows, INT32_MAX), nnz_out);

@@ -478,6 +478,12 @@ static int rowwise_run(spws_ctx* ctx, int32_t m, int32_t kdim, int32_t n, const 
   return SPWS_OK;
 }
 
+int rowwise_product(spws_ctx* ctx, int32_t m, int32_t k, int32_t n, const int32_t* A_pos, const int32_t* A_crd,
+                    const double* A_vals, const int32_t* B_pos, const int32_t* B_crd, const double* B_vals,
+                    int64_t* nnz) {
+  return rowwise_run<true>(ctx, m, k, n, A_pos, A_crd, A_vals, B_pos, B_crd, B_vals, nnz);
+}
+
 }  // namespace spws
 
 using namespace spws;

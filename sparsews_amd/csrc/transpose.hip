@@ -158,6 +158,11 @@ struct TransposeScratch {
 
 }  // namespace
 
+int csr_transpose_run(spws_ctx* ctx, int32_t m, int32_t n, int64_t nnz, const int32_t* pos, const int32_t* crd,
+                      const double* vals, int32_t* out_pos, int32_t* out_crd, double* out_vals) {
+  return transpose_run(ctx, m, n, nnz, pos, crd, vals, out_pos, out_crd, out_vals);
+}
+
 int noalloc_scratch_init(int device) {
   unsigned char* p;
   return scratch_address(device, &p);

@@ -257,6 +257,38 @@ def test_outer_auto_method(ctx):
     check(C, A, Bw)
 
 
+def keep_columns(A, keep):
+    """A's CSR with only the columns whose keep flag is set."""
+    rows = np.repeat(np.arange(A.nrows), np.diff(A.pos))
+    on = keep[A.crd]
+    pos = np.concatenate([[0], np.cumsum(np.bincount(rows[on], minlength=A.nrows))]).astype(np.int32)
+    return CSR(A.nrows, A.ncols, pos, A.crd[on], A.vals[on])
+
+
+# short rows, every bin of the row kernels, rows of thousands of products; the
+# widest output it takes and one column more (the sort again)
+@pytest.mark.parametrize("m,k,n,a,b,method", [
+    (700, 600, 40_000, (0, 7), (0, 7), 5), (2000, 900, 100_000, (0, 40), (0, 40), 5),
+    (60, 9000, 131_072, (0, 900), (0, 9), 5), (60, 9000, 131_073, (0, 900), (0, 9), 1), (1, 1, 9000, (1, 1), (1, 1), 5),
+])
+@pytest.mark.parametrize("stored", ["dense", "compressed", "unmatched"])
+def test_outer_by_rows(ctx, m, k, n, a, b, method, stored):
+    """The automatic choice where windows would hold too few products, with
+    dense outer levels, with empty columns and rows left out, and with stored
+    columns of A that meet no stored row of B and the other way round."""
+    print(f"case: outer by rows m={m} k={k} n={n} {stored}", flush=True)
+    A, B = uniform_rows(m, k, *a, 90, 0), uniform_rows(k, n, *b, 90, 1)
+    if stored == "unmatched" and k > 1:
+        rng = np.random.default_rng(90)
+        A = keep_columns(A, rng.random(k) < 0.7)
+        lengths = np.where(rng.random(k) < 0.6, np.diff(B.pos), 0)
+        B = random_csr(k, n, lengths, 91, 1)
+    for _ in range(2):
+        C = run_outer(ctx, A, B, dense_outer=stored == "dense")
+        assert ctx.stats()["outer_method"] == method
+        check(C, A, B, exact_order=method == 1)
+
+
 def test_outer_wide_columns_64bit_keys(ctx):
     """ncols > 2^24 switches to 64-bit sort keys."""
     print("case: outer 64-bit keys", flush=True)
