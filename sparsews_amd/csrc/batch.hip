@@ -400,14 +400,15 @@ static void enqueue_batch(spws_batch* b) {
     // every request is at most max_cols wide: LDS bitmap over each row's own
     // column range; the rows are counted here and computed in place below
     const size_t lds = rowbits_lds_bytes(c.max_cols, 0, false);
-    hipLaunchKernelGGL((k_row_bits<kBits1Block, kBits1Items, false, true, NoDst>),
-                       dim3(rowbits_grid(b->cus, kBits1Block, lds, c.max_rows)), dim3(kBits1Block), lds, s, bin_rows,
-                       bmeta, (int)P_BLOCK, c.max_cols, 0, Ap, Ai, Ax, Bp, Bi, Bx, NoDst{}, row_nnz, coloff,
-                       row_ncols);
-    hipLaunchKernelGGL((k_row_bits<kBits2Block, kBits2Items, false, true, NoDst>),
-                       dim3(rowbits_grid(b->cus, kBits2Block, lds, c.max_rows)), dim3(kBits2Block), lds, s, bin_rows,
-                       bmeta, (int)P_BLOCK2, c.max_cols, 0, Ap, Ai, Ax, Bp, Bi, Bx, NoDst{}, row_nnz, coloff,
-                       row_ncols);
+#define SPWS_BATCH_COUNT(BIN, PATH, LO, HI)                                                                          \
+  hipLaunchKernelGGL((k_row_bits<kBits##BIN##Block, kBits##BIN##Items, false, true, NoDst>),                         \
+                     dim3(rowbits_grid(b->cus, kBits##BIN##Block, lds, c.max_rows)), dim3(kBits##BIN##Block), lds,   \
+                     s, bin_rows, bmeta, (int)PATH, (const int64_t*)row_ub, (int64_t)(LO), (int64_t)(HI),            \
+                     c.max_cols, 0, Ap, Ai, Ax, Bp, Bi, Bx, NoDst{}, row_nnz, coloff, row_ncols)
+    SPWS_BATCH_COUNT(1, P_BLOCK, 0, INT64_MAX);
+    SPWS_BATCH_COUNT(2, P_BLOCK2, 0, kBits2Products);
+    if (b->pp.block2_ub > kBits2Products) SPWS_BATCH_COUNT(3, P_BLOCK2, kBits2Products, INT64_MAX);
+#undef SPWS_BATCH_COUNT
   } else {
     hipLaunchKernelGGL((k_row_block<2048, 1024, 256, true>), dim3(gblk), dim3(256), 0, s, bin_rows, bmeta,
                        (int)P_BLOCK, Ap, Ai, Ax, Bp, Bi, Bx, row_off, scrd, sval, row_nnz);
@@ -439,20 +440,25 @@ static void enqueue_batch(spws_batch* b) {
     // the block bins' rows at their place (the long rows staged their
     // products in the pools: before this point only)
     const BatchDst dst{Cp, coloff, coloff + 2 * (size_t)c.max_rows, d_req, req_nnz, Ci, Cx};
-    const int32_t v1 = std::min<int32_t>(b->pp.block_ub, c.max_cols);
-    const int32_t v2 = std::min<int32_t>(b->pp.block2_ub, c.max_cols);
-    const bool narrow = c.max_cols <= kBitsNarrow;
-    const size_t l1 = rowbits_lds_bytes(c.max_cols, v1, true), l2 = rowbits_lds_bytes(c.max_cols, v2, true);
-    hipLaunchKernelGGL((narrow ? k_row_bits<kBits1Block, kBits1Items, true, true, BatchDst>
-                               : k_row_bits<kBits1Block, kBits1Items, true, false, BatchDst>),
-                       dim3(rowbits_grid(b->cus, kBits1Block, l1, c.max_rows)),
-                       dim3(kBits1Block), l1, s, bin_rows, bmeta, (int)P_BLOCK, c.max_cols, v1, Ap, Ai, Ax, Bp, Bi,
-                       Bx, dst, row_nnz, coloff, row_ncols);
-    hipLaunchKernelGGL((narrow ? k_row_bits<kBits2Block, kBits2Items, true, true, BatchDst>
-                               : k_row_bits<kBits2Block, kBits2Items, true, false, BatchDst>),
-                       dim3(rowbits_grid(b->cus, kBits2Block, l2, c.max_rows)),
-                       dim3(kBits2Block), l2, s, bin_rows, bmeta, (int)P_BLOCK2, c.max_cols, v2, Ap, Ai, Ax, Bp, Bi,
-                       Bx, dst, row_nnz, coloff, row_ncols);
+#define SPWS_BATCH_ROWS_W(BIN, PATH, LO, HI, VCAP, NARROW)                                                           \
+  hipLaunchKernelGGL(                                                                                                \
+      (k_row_bits<kBits##BIN##Block, kBits##BIN##Items, true, NARROW, BatchDst>),                                    \
+      dim3(rowbits_grid(b->cus, kBits##BIN##Block, rowbits_lds_bytes(c.max_cols, VCAP, true), c.max_rows)),          \
+      dim3(kBits##BIN##Block), rowbits_lds_bytes(c.max_cols, VCAP, true), s, bin_rows, bmeta, (int)PATH,             \
+      (const int64_t*)row_ub, (int64_t)(LO), (int64_t)(HI), c.max_cols, VCAP, Ap, Ai, Ax, Bp, Bi, Bx, dst, row_nnz,  \
+      coloff, row_ncols)
+#define SPWS_BATCH_ROWS(BIN, PATH, LO, HI, MOST)                                        \
+  do {                                                                                  \
+    const int32_t vcap = std::min<int32_t>(MOST, c.max_cols);                           \
+    if (c.max_cols <= kBitsNarrow) SPWS_BATCH_ROWS_W(BIN, PATH, LO, HI, vcap, true);    \
+    else SPWS_BATCH_ROWS_W(BIN, PATH, LO, HI, vcap, false);                             \
+  } while (0)
+    SPWS_BATCH_ROWS(1, P_BLOCK, 0, INT64_MAX, b->pp.block_ub);
+    SPWS_BATCH_ROWS(2, P_BLOCK2, 0, kBits2Products, std::min(b->pp.block2_ub, kBits2Products));
+    if (b->pp.block2_ub > kBits2Products)
+      SPWS_BATCH_ROWS(3, P_BLOCK2, kBits2Products, INT64_MAX, b->pp.block2_ub);
+#undef SPWS_BATCH_ROWS
+#undef SPWS_BATCH_ROWS_W
   }
   hipLaunchKernelGGL(k_batch_total, dim3(1), dim3(64), 0, s, Cp, d_desc, (int64_t*)P(BP_TOTAL));
   (void)hipMemcpyAsync(b->h_total, P(BP_TOTAL), 8, hipMemcpyDeviceToHost, s);

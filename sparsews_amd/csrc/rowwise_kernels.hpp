@@ -1407,6 +1407,10 @@ __global__ __launch_bounds__(BLOCK) void k_row_bitmap_staged(
 // wavefront), as were registers bounded below 120 (spills, each waited for).
 constexpr int kBits1Block = 256, kBits1Items = 4;  // threads and products per thread of the two bins
 constexpr int kBits2Block = 256, kBits2Items = 8;
+// rows of the second bin beyond those registers, in a launch of their own with
+// LDS for them (a workgroup's LDS for 4,096 entries leaves two on a CU)
+constexpr int kBits3Block = 512, kBits3Items = 8;
+constexpr int32_t kBits2Products = kBits2Block * kBits2Items;
 constexpr int kBitsEntries = 256;
 constexpr int32_t kBitsNarrow = 1 << 16;  // row widths whose columns are staged in 16 bits
 
@@ -1521,7 +1525,8 @@ __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70
 
 template <int BLOCK, int ITEMS, bool kValues, bool kNarrow, class Dst>
 __global__ __launch_bounds__(BLOCK, !kValues ? 7 : ITEMS <= 4 ? 5 : 4) void k_row_bits(
-    const int32_t* __restrict__ bin_rows, const int32_t* __restrict__ bmeta, int path, int32_t ncols, int32_t vcap,
+    const int32_t* __restrict__ bin_rows, const int32_t* __restrict__ bmeta, int path,
+    const int64_t* __restrict__ row_ub, int64_t ub_lo, int64_t ub_hi, int32_t ncols, int32_t vcap,
     const int32_t* __restrict__ Ap, const int32_t* __restrict__ Ai, const double* __restrict__ Ax,
     const int32_t* __restrict__ Bp, const int32_t* __restrict__ Bi, const double* __restrict__ Bx, Dst dst,
     int32_t* __restrict__ row_nnz, const int32_t* __restrict__ row_colbase, const int32_t* __restrict__ row_ncols) {
@@ -1549,7 +1554,24 @@ __global__ __launch_bounds__(BLOCK, !kValues ? 7 : ITEMS <= 4 ? 5 : 4) void k_ro
   const int32_t count = bmeta[kMetaCount + path];
   const int32_t* const rows = bin_rows + bmeta[kMetaOff + path];
   const int32_t step = gridDim.x;
-  const auto row_at = [&](int64_t r) -> int32_t { return r < count ? rows[r] : -1; };
+  // this workgroup's rows (blockIdx.x, + step, ...) with ub_lo < ub <= ub_hi,
+  // 64 looked at together
+  int64_t ahead = blockIdx.x;
+  int32_t seen = -1;
+  uint64_t left = 0;
+  const auto next_row = [&]() -> int32_t {
+    while (!left) {
+      if (ahead >= count) return -1;
+      const int64_t r = ahead + (int64_t)lane * step;
+      seen = r < count ? rows[r] : -1;
+      const int64_t ub = seen >= 0 ? row_ub[seen] : 0;
+      left = __ballot(ub > ub_lo && ub <= ub_hi);
+      ahead += (int64_t)kWave * step;
+    }
+    const int l = __builtin_ctzll(left);
+    left &= left - 1;
+    return __builtin_amdgcn_readlane(seen, l);
+  };
   const auto bounds = [&](RowAhead& x) {
     x.a_beg = x.a_end = 0;
     if (x.i >= 0) {
@@ -1567,12 +1589,11 @@ __global__ __launch_bounds__(BLOCK, !kValues ? 7 : ITEMS <= 4 ? 5 : 4) void k_ro
       x.blen = Bp[x.j + 1] - x.bstart;
     }
   };
-  int64_t r = blockIdx.x;
-  if (r >= count) return;  // uniform
   RowAhead x0, x1, x2;
-  x0.i = row_at(r);
-  x1.i = row_at(r + step);
-  x2.i = row_at(r + 2 * (int64_t)step);
+  x0.i = next_row();
+  if (x0.i < 0) return;  // uniform
+  x1.i = next_row();
+  x2.i = next_row();
   bounds(x0);
   bounds(x1);
   entries(x0);
@@ -1583,11 +1604,11 @@ __global__ __launch_bounds__(BLOCK, !kValues ? 7 : ITEMS <= 4 ? 5 : 4) void k_ro
   uint32_t own[(ITEMS + 3) / 4];
   int32_t total = gather_marked<BLOCK, ITEMS, kValues>(x0, s_marks[w], Ai, Bp, Bi, Bx, col, bv, own);
   int parity = 0;
-  for (; r < count; r += step, parity ^= 1) {
+  for (; x0.i >= 0; parity ^= 1) {
     // further rows: one level of loads each
     brows(x1);
     bounds(x2);
-    const int32_t i3 = row_at(r + 3 * (int64_t)step);
+    const int32_t i3 = next_row();
     const int32_t i = x0.i;
     const int32_t cb = row_colbase ? row_colbase[i] : 0;
     const int32_t nv = rowbits_vecs(row_ncols ? row_ncols[i] : ncols);  // vectors of this row

@@ -384,32 +384,37 @@ static int rowwise_run(spws_ctx* ctx, int32_t m, int32_t kdim, int32_t n, const 
                           kDirectProducts;
   enum { kCountRows, kSlotRows, kFinalRows };
   auto block_rows = [&](int what) -> int {
-    for (int path : {(int)P_BLOCK, (int)P_BLOCK2}) {
-      if (!counts[path]) continue;
-      const int32_t vcap = what == kCountRows ? 0 : (int32_t)std::min<int64_t>(maxub[path], n);
+    for (int bin = 1; bin <= 3; ++bin) {
+      const int path = bin == 1 ? P_BLOCK : P_BLOCK2;
+      // the second bin's rows by what the registers of its two kernels hold
+      const int64_t lo = bin == 3 ? kBits2Products : 0, hi = bin == 2 ? kBits2Products : INT64_MAX;
+      if (!counts[path] || maxub[path] <= lo) continue;
+      const int32_t vcap =
+          what == kCountRows ? 0 : (int32_t)std::min<int64_t>(std::min<int64_t>(maxub[path], hi), n);
       const size_t lds = rowbits_lds_bytes(n, vcap, what != kCountRows);
-      const unsigned block = path == P_BLOCK ? kBits1Block : kBits2Block;
+      const unsigned block = bin == 3 ? kBits3Block : bin == 2 ? kBits2Block : kBits1Block;
       const unsigned grid = rowbits_grid(cus, block, lds, counts[path]);
-#define SPWS_ROW_BITS(NAME, BIN, VALUES, DST, ...)                                                                \
-  do {                                                                                                            \
-    if (VALUES && n > kBitsNarrow) SPWS_ROW_BITS_W(NAME, BIN, VALUES, false, DST, __VA_ARGS__);                   \
-    else SPWS_ROW_BITS_W(NAME, BIN, VALUES, true, DST, __VA_ARGS__);                                              \
-  } while (0)
 #define SPWS_ROW_BITS_W(NAME, BIN, VALUES, NARROW, DST, ...)                                                      \
-  SPWS_LAUNCH(ctx, NAME, (k_row_bits<kBits##BIN##Block, kBits##BIN##Items, VALUES, NARROW, DST>), dim3(grid), dim3(block),  \
-              (unsigned)lds, rows, bmeta, path, n, vcap, Ap, Ai, Ax, Bp, Bi, Bx, DST{__VA_ARGS__}, rnnz, (const int32_t*)nullptr,      \
+  SPWS_LAUNCH(ctx, NAME, (k_row_bits<kBits##BIN##Block, kBits##BIN##Items, VALUES, NARROW, DST>), dim3(grid),     \
+              dim3(block), (unsigned)lds, rows, bmeta, path, (const int64_t*)ctx->row_ub.as<int64_t>(), lo, hi, n, \
+              vcap, Ap, Ai, Ax, Bp, Bi, Bx, DST{__VA_ARGS__}, rnnz, (const int32_t*)nullptr,                      \
               (const int32_t*)nullptr)
-      if (what == kCountRows && path == P_BLOCK) SPWS_ROW_BITS("row_count", 1, false, NoDst);
-      else if (what == kCountRows) SPWS_ROW_BITS("row_count", 2, false, NoDst);
-      else if (what == kSlotRows && path == P_BLOCK)
-        SPWS_ROW_BITS("row_bitmap", 1, true, SlotDst, roff, scrd, sval);
-      else if (what == kSlotRows) SPWS_ROW_BITS("row_bitmap", 2, true, SlotDst, roff, scrd, sval);
-      else if (path == P_BLOCK)
-        SPWS_ROW_BITS("row_bitmap", 1, true, FinalDst, ctx->out_pos.as<int32_t>(),
-                      ctx->out_crd.as<int32_t>(), ctx->out_val.as<double>());
-      else
-        SPWS_ROW_BITS("row_bitmap", 2, true, FinalDst, ctx->out_pos.as<int32_t>(),
-                      ctx->out_crd.as<int32_t>(), ctx->out_val.as<double>());
+#define SPWS_ROW_BITS(BIN)                                                                                        \
+  do {                                                                                                            \
+    if (what == kCountRows) SPWS_ROW_BITS_W("row_count", BIN, false, true, NoDst);                                \
+    else if (what == kSlotRows && n > kBitsNarrow)                                                                \
+      SPWS_ROW_BITS_W("row_bitmap", BIN, true, false, SlotDst, roff, scrd, sval);                                 \
+    else if (what == kSlotRows) SPWS_ROW_BITS_W("row_bitmap", BIN, true, true, SlotDst, roff, scrd, sval);        \
+    else if (n > kBitsNarrow)                                                                                     \
+      SPWS_ROW_BITS_W("row_bitmap", BIN, true, false, FinalDst, ctx->out_pos.as<int32_t>(),                       \
+                      ctx->out_crd.as<int32_t>(), ctx->out_val.as<double>());                                     \
+    else                                                                                                          \
+      SPWS_ROW_BITS_W("row_bitmap", BIN, true, true, FinalDst, ctx->out_pos.as<int32_t>(),                        \
+                      ctx->out_crd.as<int32_t>(), ctx->out_val.as<double>());                                     \
+  } while (0)
+      if (bin == 1) SPWS_ROW_BITS(1);
+      else if (bin == 2) SPWS_ROW_BITS(2);
+      else SPWS_ROW_BITS(3);
 #undef SPWS_ROW_BITS
 #undef SPWS_ROW_BITS_W
     }
