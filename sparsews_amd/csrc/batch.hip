@@ -12,20 +12,24 @@
 // every size from a device-side descriptor and request table; a launch copies
 // the (pinned) table and descriptor in, so the same graph executes any batch
 // that fits the engine's capacities:
-//   H2D request table + descriptor
-//   k_batch_gather     operands -> engine pools, indices rebased
-//   k_meta_clear, k_rowstat, device-sized scan, k_bin_offsets, k_binscatter
+//   H2D descriptor + request table (one block)
+//   k_batch_gather     operands -> engine pools, indices rebased; clears the
+//                      bin metadata
+//   k_rowstat, k_batch_guard, device-sized scan, k_binscatter
 //   numeric kernels of the wave / wave2 / block / block2 / wide paths
 //   (persistent grids; each reads its row count from the bin metadata; when
 //   the engine bounds the request width by max_cols the block bins use the
 //   LDS bitmap kernel over each row's own column range, and only count here)
 //   device-sized scan -> C_pos
-//   k_batch_req_meta   each request's nnz (and whether its output buffer holds it)
+//   k_batch_req_meta   each request's nnz (and whether its output buffer holds
+//                      it), the batch's
 //   k_batch_compact    rows into their request's output buffer when it has
 //                      one, into the engine's pools otherwise (columns
 //                      shifted back per row)
 //   k_row_bits         the counted rows, computed straight into that place
-//   k_batch_total, D2H of the batch nnz and of each request's nnz
+//   D2H of each request's nnz and the batch's
+// One chain, no branches: the graph with the long rows and the compaction on a
+// second branch took 2,914 us for 64 products where the chain takes 1,968.
 // No memset is recorded into the graph: clears are kernels.  The dense path
 // is not used in batches: the stacked column space is the sum of the
 // requests' widths, so long rows take the HBM hash path instead.
@@ -67,10 +71,14 @@ struct spws_batch_desc {
   int32_t overflow, pad;  // set on the device when an upper bound was under-reported
 };
 
+// bytes the descriptor takes in front of the request table
+constexpr size_t kDescBytes = 64;
+static_assert(sizeof(spws_batch_desc) <= kDescBytes && kDescBytes % alignof(spws_batch_req) == 0, "descriptor block");
+
 enum BatchPool : int {
-  BP_REQ = 0, BP_DESC, BP_APOS, BP_ACRD, BP_AVAL, BP_BPOS, BP_BCRD, BP_BVAL, BP_COLOFF, BP_ROWUB, BP_ROWOFF,
-  BP_ROWNNZ, BP_BINROWS, BP_META, BP_SCRD, BP_SVAL, BP_CPOS, BP_CCRD, BP_CVAL, BP_WKEY, BP_WVAL, BP_SCAN, BP_TOTAL,
-  BP_REQNNZ, BP_COUNT
+  BP_DESC = 0, BP_APOS, BP_ACRD, BP_AVAL, BP_BPOS, BP_BCRD, BP_BVAL, BP_COLOFF, BP_ROWUB, BP_ROWOFF,
+  BP_ROWNNZ, BP_BINROWS, BP_META, BP_SCRD, BP_SVAL, BP_CPOS, BP_CCRD, BP_CVAL, BP_WKEY, BP_WVAL, BP_SCAN, BP_REQNNZ,
+  BP_COUNT
 };
 
 struct spws_batch {
@@ -110,7 +118,8 @@ __device__ __forceinline__ void dscan_range(int64_t n, int64_t* beg, int64_t* en
 }
 
 // Exclusive scan whose length lives in device memory: each of a fixed number
-// of blocks owns a contiguous range (reduce, scan of the partials, rescan).
+// of blocks owns a contiguous range (reduce, then each block sums the partials
+// before its own and rescans).
 template <class Tin, class Tout>
 __global__ __launch_bounds__(kDScanThreads) void k_dscan_reduce(const Tin* __restrict__ in,
                                                                 const int32_t* __restrict__ n_dev,
@@ -130,17 +139,6 @@ __global__ __launch_bounds__(kDScanThreads) void k_dscan_reduce(const Tin* __res
   }
 }
 
-template <class Tout>
-__global__ __launch_bounds__(kDScanThreads) void k_dscan_top(Tout* __restrict__ part) {
-  __shared__ Tout sh[kDScanThreads / kWave + 1];
-  static_assert(kDScanBlocks == kDScanThreads, "one partial per thread");
-  const Tout v = part[threadIdx.x];
-  Tout total;
-  const Tout pre = block_excl_scan<Tout, kDScanThreads>(v, sh, &total);
-  part[threadIdx.x] = pre;
-  if (threadIdx.x == 0) part[kDScanBlocks] = total;
-}
-
 template <class Tin, class Tout>
 __global__ __launch_bounds__(kDScanThreads) void k_dscan_apply(const Tin* __restrict__ in,
                                                                const int32_t* __restrict__ n_dev,
@@ -149,7 +147,14 @@ __global__ __launch_bounds__(kDScanThreads) void k_dscan_apply(const Tin* __rest
   const int64_t n = *n_dev;
   int64_t beg, end;
   dscan_range(n, &beg, &end);
-  Tout carry = part[blockIdx.x];
+  static_assert(kDScanBlocks == kDScanThreads, "one partial per thread");
+  Tout carry, total_all;
+  {
+    const Tout mine = part[threadIdx.x];
+    (void)block_excl_scan<Tout, kDScanThreads>(mine, sh, &total_all);
+    const Tout before = (int)threadIdx.x < (int)blockIdx.x ? mine : (Tout)0;
+    (void)block_excl_scan<Tout, kDScanThreads>(before, sh, &carry);
+  }
   for (int64_t base = beg; base < end; base += kDScanTile) {
     Tout v[kDScanItems];
     Tout local = 0;
@@ -171,7 +176,7 @@ __global__ __launch_bounds__(kDScanThreads) void k_dscan_apply(const Tin* __rest
     }
     carry += total;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = part[kDScanBlocks];
+  if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = total_all;
 }
 
 // dst_crd[p] = crd[p] + shift, dst_val[p] = val[p] for p = t0, t0 + st, ...:
@@ -212,8 +217,10 @@ __global__ __launch_bounds__(256) void k_batch_gather(const spws_batch_req* __re
                                                       int32_t* __restrict__ A_pos, int32_t* __restrict__ A_crd,
                                                       double* __restrict__ A_val, int32_t* __restrict__ B_pos,
                                                       int32_t* __restrict__ B_crd, double* __restrict__ B_val,
-                                                      int32_t* __restrict__ row_coloff, int32_t max_rows) {
+                                                      int32_t* __restrict__ row_coloff, int32_t max_rows,
+                                                      int32_t* __restrict__ bmeta) {
   const int32_t r = blockIdx.y;
+  if (blockIdx.x == 0 && r == 0 && threadIdx.x < kMetaBlockInts) bmeta[threadIdx.x] = 0;
   if (r >= desc->nreq) return;
   const spws_batch_req q = reqs[r];
   const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -229,11 +236,6 @@ __global__ __launch_bounds__(256) void k_batch_gather(const spws_batch_req* __re
   for (int64_t i = t0; i <= q.k; i += st) B_pos[q.brow0 + i] = (int32_t)(q.bnnz0 + q.B_pos[i]);
   copy_rebased(q.A_crd, q.A_val, q.annz, q.brow0, A_crd + q.annz0, A_val + q.annz0, t0, st);
   copy_rebased(q.B_crd, q.B_val, q.bnnz, q.col0, B_crd + q.bnnz0, B_val + q.bnnz0, t0, st);
-}
-
-__global__ void k_batch_total(const int32_t* __restrict__ C_pos, const spws_batch_desc* __restrict__ desc,
-                              int64_t* __restrict__ total) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *total = desc->overflow ? -2 : C_pos[desc->rows];
 }
 
 // The true upper bounds (k_rowstat) against the pools: the sum of all row
@@ -257,11 +259,13 @@ __global__ void k_batch_guard(spws_batch_desc* __restrict__ desc, int32_t* __res
 // Per request, after the output row pointers are known: req_nnz[r] = its
 // nnz, -1 when it has an output buffer smaller than that (its rows then stay
 // in the pools), -2 when the batch overflowed.  A request with no rows gets
-// its single row pointer here.
+// its single row pointer here.  *total = the batch's nnz (-2: overflow).
 __global__ __launch_bounds__(256) void k_batch_req_meta(const spws_batch_req* __restrict__ reqs,
                                                         const spws_batch_desc* __restrict__ desc,
                                                         const int32_t* __restrict__ C_pos,
-                                                        int64_t* __restrict__ req_nnz) {
+                                                        int64_t* __restrict__ req_nnz,
+                                                        int64_t* __restrict__ total) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *total = desc->overflow ? -2 : C_pos[desc->rows];
   for (int32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < desc->nreq; r += gridDim.x * blockDim.x) {
     if (desc->overflow) {
       req_nnz[r] = -2;
@@ -344,7 +348,6 @@ __global__ __launch_bounds__(256) void k_batch_compact(const spws_batch_desc* __
 template <class Tin, class Tout>
 static void dscan(hipStream_t s, const Tin* in, const int32_t* n_dev, Tout* part, Tout* out) {
   hipLaunchKernelGGL((k_dscan_reduce<Tin, Tout>), dim3(kDScanBlocks), dim3(kDScanThreads), 0, s, in, n_dev, part);
-  hipLaunchKernelGGL((k_dscan_top<Tout>), dim3(1), dim3(kDScanThreads), 0, s, part);
   hipLaunchKernelGGL((k_dscan_apply<Tin, Tout>), dim3(kDScanBlocks), dim3(kDScanThreads), 0, s, in, n_dev, part, out);
 }
 
@@ -353,10 +356,11 @@ static void enqueue_batch(spws_batch* b) {
   hipStream_t s = b->stream;
   const spws_batch_caps& c = b->caps;
   auto P = [&](int i) { return b->pool[i].ptr; };
-  spws_batch_req* d_req = (spws_batch_req*)P(BP_REQ);
+  // the descriptor, then the request table (h_desc and h_req alike)
   spws_batch_desc* d_desc = (spws_batch_desc*)P(BP_DESC);
-  (void)hipMemcpyAsync(d_req, b->h_req, sizeof(spws_batch_req) * (size_t)c.max_requests, hipMemcpyHostToDevice, s);
-  (void)hipMemcpyAsync(d_desc, b->h_desc, sizeof(spws_batch_desc), hipMemcpyHostToDevice, s);
+  spws_batch_req* d_req = (spws_batch_req*)((char*)P(BP_DESC) + kDescBytes);
+  (void)hipMemcpyAsync(d_desc, b->h_desc, kDescBytes + sizeof(spws_batch_req) * (size_t)c.max_requests,
+                       hipMemcpyHostToDevice, s);
   int32_t* Ap = (int32_t*)P(BP_APOS);
   int32_t* Ai = (int32_t*)P(BP_ACRD);
   double* Ax = (double*)P(BP_AVAL);
@@ -365,7 +369,7 @@ static void enqueue_batch(spws_batch* b) {
   double* Bx = (double*)P(BP_BVAL);
   int32_t* coloff = (int32_t*)P(BP_COLOFF);
   hipLaunchKernelGGL(k_batch_gather, dim3(64, c.max_requests), dim3(256), 0, s, d_req, d_desc, Ap, Ai, Ax, Bp, Bi, Bx,
-                     coloff, (int32_t)c.max_rows);
+                     coloff, (int32_t)c.max_rows, (int32_t*)P(BP_META));
   const int32_t* row_ncols = coloff + c.max_rows;
   const int32_t* m_dev = &d_desc->rows;
   int64_t* row_ub = (int64_t*)P(BP_ROWUB);
@@ -380,22 +384,34 @@ static void enqueue_batch(spws_batch* b) {
   int32_t* Ci = (int32_t*)P(BP_CCRD);
   double* Cx = (double*)P(BP_CVAL);
   const unsigned grows = (unsigned)std::min<int64_t>(div_up(c.max_rows, 256), 4096);
-  hipLaunchKernelGGL(k_meta_clear, dim3(1), dim3(64), 0, s, bmeta, maxub);
   const unsigned gstat = (unsigned)std::min<int64_t>(div_up(c.max_rows, kRsRows), 16384);
   hipLaunchKernelGGL(k_rowstat, dim3(gstat), dim3(kRsBlock), 0, s, 0, m_dev, 1, Ap, Ai, Bp, row_ub, bmeta, maxub,
                      b->pp);
   hipLaunchKernelGGL(k_batch_guard, dim3(1), dim3(64), 0, s, d_desc, bmeta, maxub, c.max_products,
                      c.max_row_products);
   dscan<int64_t, int64_t>(s, row_ub, m_dev, (int64_t*)P(BP_SCAN), row_off);
-  hipLaunchKernelGGL(k_bin_offsets, dim3(1), dim3(64), 0, s, bmeta);
   hipLaunchKernelGGL(k_binscatter, dim3(grows), dim3(256), 0, s, 0, m_dev, 1, row_ub, bmeta, bin_rows, row_nnz, b->pp);
   const unsigned gwave = (unsigned)std::min<int64_t>(c.max_rows, 8192);
   const unsigned gblk = (unsigned)std::min<int64_t>(c.max_rows, 1024);
+  const bool bits = c.max_cols > 0 && c.max_cols <= kBitmapCols;
+  if (bits) {
+    // products staged in the output pools, which the compaction fills later;
+    // rows of at most acc_cap entries accumulate in LDS
+    const size_t bm_bytes = bitmap_lds_bytes(c.max_cols, 0, false, kBitmapLongBlock);
+    const int32_t acc_cap = (int32_t)std::min<int64_t>(c.max_cols, (int64_t)((kLdsBudget - bm_bytes) / 8));
+    hipLaunchKernelGGL(k_row_bitmap_staged<kBitmapLongBlock>, dim3(gblk), dim3(kBitmapLongBlock),
+                       bitmap_lds_bytes(c.max_cols, std::max(acc_cap, kLongAccMin), true, kBitmapLongBlock),
+                       s, bin_rows, bmeta, (int)P_WIDE, c.max_cols, Ap, Ai, Ax, Bp, Bi, Bx, row_off, scrd, sval,
+                       row_nnz, coloff, row_ncols, Ci, Cx, acc_cap);
+  } else {
+    hipLaunchKernelGGL((k_row_wide<true>), dim3(b->wide_groups), dim3(kWideBlock), 0, s, bin_rows, bmeta,
+                       (int)P_WIDE, Ap, Ai, Ax, Bp, Bi, Bx, row_ub, row_off, scrd, sval, row_nnz,
+                       (int32_t*)P(BP_WKEY), (double*)P(BP_WVAL), b->wide_slots);
+  }
   hipLaunchKernelGGL((k_row_wave<128, 1, true, kWaveRowsK>), dim3(gwave), dim3(64), 0, s, bin_rows, bmeta, (int)P_WAVE,
                      Ap, Ai, Ax, Bp, Bi, Bx, row_off, scrd, sval, row_nnz);
   hipLaunchKernelGGL((k_row_wave<512, 4, true>), dim3(gwave), dim3(64), 0, s, bin_rows, bmeta, (int)P_WAVE2, Ap, Ai,
                      Ax, Bp, Bi, Bx, row_off, scrd, sval, row_nnz);
-  const bool bits = c.max_cols > 0 && c.max_cols <= kBitmapCols;
   if (bits) {
     // every request is at most max_cols wide: LDS bitmap over each row's own
     // column range; the rows are counted here and computed in place below
@@ -415,27 +431,13 @@ static void enqueue_batch(spws_batch* b) {
     hipLaunchKernelGGL((k_row_block<8192, 4096, 512, true>), dim3(gblk), dim3(512), 0, s, bin_rows, bmeta,
                        (int)P_BLOCK2, Ap, Ai, Ax, Bp, Bi, Bx, row_off, scrd, sval, row_nnz);
   }
-  if (bits) {
-    // products staged in the output pools, which the compaction fills later;
-    // rows of at most acc_cap entries accumulate in LDS
-    const size_t bm_bytes = bitmap_lds_bytes(c.max_cols, 0, false, kBitmapLongBlock);
-    const int32_t acc_cap = (int32_t)std::min<int64_t>(c.max_cols, (int64_t)((kLdsBudget - bm_bytes) / 8));
-    hipLaunchKernelGGL(k_row_bitmap_staged<kBitmapLongBlock>, dim3(gblk), dim3(kBitmapLongBlock),
-                       bitmap_lds_bytes(c.max_cols, std::max(acc_cap, kLongAccMin), true, kBitmapLongBlock), s, bin_rows, bmeta,
-                       (int)P_WIDE, c.max_cols, Ap, Ai, Ax, Bp, Bi, Bx, row_off, scrd, sval, row_nnz, coloff,
-                       row_ncols, Ci, Cx, acc_cap);
-  } else {
-    hipLaunchKernelGGL((k_row_wide<true>), dim3(b->wide_groups), dim3(kWideBlock), 0, s, bin_rows, bmeta,
-                       (int)P_WIDE, Ap, Ai, Ax, Bp, Bi, Bx, row_ub, row_off, scrd, sval, row_nnz,
-                       (int32_t*)P(BP_WKEY), (double*)P(BP_WVAL), b->wide_slots);
-  }
   dscan<int32_t, int32_t>(s, row_nnz, m_dev, (int32_t*)P(BP_SCAN), Cp);
   int64_t* req_nnz = (int64_t*)P(BP_REQNNZ);
   hipLaunchKernelGGL(k_batch_req_meta, dim3((unsigned)div_up(c.max_requests, 256)), dim3(256), 0, s, d_req, d_desc,
-                     Cp, req_nnz);
+                     Cp, req_nnz, req_nnz + c.max_requests);
   hipLaunchKernelGGL(k_batch_compact, dim3((unsigned)std::min<int64_t>(div_up(c.max_rows, 4), 16384)), dim3(256), 0,
-                     s, d_desc, row_off, Cp, scrd, sval, coloff, coloff + 2 * (size_t)c.max_rows, d_req, req_nnz, Ci,
-                     Cx, bits ? DirectRows{b->pp.wave2_ub, b->pp.block2_ub} : DirectRows{0, 0});
+                     s, d_desc, row_off, Cp, scrd, sval, coloff, coloff + 2 * (size_t)c.max_rows, d_req, req_nnz,
+                     Ci, Cx, bits ? DirectRows{b->pp.wave2_ub, b->pp.block2_ub} : DirectRows{0, 0});
   if (bits) {
     // the block bins' rows at their place (the long rows staged their
     // products in the pools: before this point only)
@@ -460,9 +462,7 @@ static void enqueue_batch(spws_batch* b) {
 #undef SPWS_BATCH_ROWS
 #undef SPWS_BATCH_ROWS_W
   }
-  hipLaunchKernelGGL(k_batch_total, dim3(1), dim3(64), 0, s, Cp, d_desc, (int64_t*)P(BP_TOTAL));
-  (void)hipMemcpyAsync(b->h_total, P(BP_TOTAL), 8, hipMemcpyDeviceToHost, s);
-  (void)hipMemcpyAsync(b->h_req_nnz, req_nnz, 8 * (size_t)c.max_requests, hipMemcpyDeviceToHost, s);
+  (void)hipMemcpyAsync(b->h_req_nnz, req_nnz, 8 * ((size_t)c.max_requests + 1), hipMemcpyDeviceToHost, s);
 }
 
 static void batch_release(spws_batch* b) {
@@ -470,9 +470,7 @@ static void batch_release(spws_batch* b) {
   if (b->graph) (void)hipGraphDestroy(b->graph);
   if (b->done) (void)hipEventDestroy(b->done);
   for (DevBuf& p : b->pool) p.release();
-  if (b->h_req) (void)hipHostFree(b->h_req);
-  if (b->h_desc) (void)hipHostFree(b->h_desc);
-  if (b->h_total) (void)hipHostFree(b->h_total);
+  if (b->h_desc) (void)hipHostFree(b->h_desc);  // h_req lies behind it, h_total behind h_req_nnz
   if (b->h_req_nnz) (void)hipHostFree(b->h_req_nnz);
   if (b->stream) (void)hipStreamDestroy(b->stream);
 }
@@ -485,19 +483,19 @@ static int batch_build(spws_batch* b) {
   b->wide_slots = std::max<int64_t>(64, next_pow2_u32((uint32_t)(2 * c.max_row_products)));
   b->wide_groups = 64;
   const size_t sizes[BP_COUNT] = {
-      sizeof(spws_batch_req) * (size_t)c.max_requests, sizeof(spws_batch_desc), (rows + 1) * 4, annz * 4, annz * 8,
+      kDescBytes + sizeof(spws_batch_req) * (size_t)c.max_requests, (rows + 1) * 4, annz * 4, annz * 8,
       (brows + 1) * 4, bnnz * 4, bnnz * 8, rows * 12, rows * 8, (rows + 1) * 8, rows * 4, rows * 4, 64 * 8, ub * 4,
       ub * 8, (rows + 1) * 4, ub * 4, ub * 8, (size_t)b->wide_groups * b->wide_slots * 4,
-      (size_t)b->wide_groups * b->wide_slots * 8, (kDScanBlocks + 1) * 8, 8, (size_t)c.max_requests * 8};
+      (size_t)b->wide_groups * b->wide_slots * 8, (kDScanBlocks + 1) * 8, ((size_t)c.max_requests + 1) * 8};
   int rc;
   for (int i = 0; i < BP_COUNT; ++i)
     if ((rc = b->pool[i].ensure(sizes[i] > 0 ? sizes[i] : 8))) return rc;
-  SPWS_HIP(hipHostMalloc((void**)&b->h_req, sizeof(spws_batch_req) * (size_t)c.max_requests, hipHostMallocDefault));
-  SPWS_HIP(hipHostMalloc((void**)&b->h_desc, sizeof(spws_batch_desc), hipHostMallocDefault));
-  SPWS_HIP(hipHostMalloc((void**)&b->h_total, 8, hipHostMallocDefault));
-  SPWS_HIP(hipHostMalloc((void**)&b->h_req_nnz, 8 * (size_t)c.max_requests, hipHostMallocDefault));
-  memset(b->h_req, 0, sizeof(spws_batch_req) * (size_t)c.max_requests);
-  memset(b->h_desc, 0, sizeof(spws_batch_desc));
+  const size_t table = kDescBytes + sizeof(spws_batch_req) * (size_t)c.max_requests;
+  SPWS_HIP(hipHostMalloc((void**)&b->h_desc, table, hipHostMallocDefault));
+  SPWS_HIP(hipHostMalloc((void**)&b->h_req_nnz, 8 * ((size_t)c.max_requests + 1), hipHostMallocDefault));
+  memset(b->h_desc, 0, table);
+  b->h_req = reinterpret_cast<spws_batch_req*>(reinterpret_cast<char*>(b->h_desc) + kDescBytes);
+  b->h_total = b->h_req_nnz + c.max_requests;
   SPWS_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
   SPWS_HIP(hipEventCreateWithFlags(&b->done, hipEventDisableTiming));
   // SPWS_BATCH_EAGER=1: no graph; every launch enqueues the same kernels

@@ -129,32 +129,16 @@ __global__ __launch_bounds__(kRsBlock) void k_rowstat(int32_t m_host, const int3
   }
 }
 
-// offsets of the paths' row lists (exclusive prefix of the counts)
-__global__ void k_bin_offsets(int32_t* __restrict__ bmeta) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    int32_t run = 0;
-    for (int p = 0; p < 8; ++p) {
-      bmeta[kMetaOff + p] = run;
-      if (p < P_EMPTY) run += bmeta[kMetaCount + p];
-    }
-  }
-}
-
 // ints of the metadata block: bmeta [0, kMetaInts), then 9 uint64 maxub
 // from int 32 on
 constexpr int kMetaBlockInts = 32 + 2 * 9;
 
-// zero the bin metadata (a kernel, so the sequence can be graph-captured)
-__global__ void k_meta_clear(int32_t* __restrict__ bmeta, unsigned long long* __restrict__ maxub) {
-  const int t = threadIdx.x;
-  if (t < kMetaInts) bmeta[t] = 0;
-  if (t < 9) maxub[t] = 0;  // [8]: sum of the upper bounds
-}
-
 // Row ids grouped by path, a tile of kRsBlock rows per workgroup: ranks
 // within each wavefront from ballots, wavefront offsets within the tile in
 // LDS, and one global cursor atomic per path and tile (issued by separate
-// threads, so a tile waits for one atomic latency).
+// threads, so a tile waits for one atomic latency).  The paths' offsets in the
+// list are the exclusive prefix of their counts, which every workgroup sums
+// for itself and the first one stores.
 __global__ __launch_bounds__(kRsBlock) void k_binscatter(int32_t m_host, const int32_t* __restrict__ m_dev,
                                                          int32_t ncols, const int64_t* __restrict__ row_ub,
                                                          int32_t* __restrict__ bmeta, int32_t* __restrict__ bin_rows,
@@ -164,6 +148,11 @@ __global__ __launch_bounds__(kRsBlock) void k_binscatter(int32_t m_host, const i
   __shared__ int32_t gbase[8];
   const int32_t m = dev_or(m_dev, m_host);
   const int t = threadIdx.x, lane = lane_id(), w = t / kWave;
+  int32_t list = 0;  // thread t < 8: where path t's rows start
+  if (t < 8) {
+    for (int p = 0; p < min(t, (int)P_EMPTY); ++p) list += bmeta[kMetaCount + p];
+    if (blockIdx.x == 0) bmeta[kMetaOff + t] = list;
+  }
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   for (int32_t base = blockIdx.x * kRsBlock; base < m; base += gridDim.x * kRsBlock) {
     const int32_t i = base + t;
@@ -184,7 +173,7 @@ __global__ __launch_bounds__(kRsBlock) void k_binscatter(int32_t m_host, const i
         woff[v][t] = run;
         run += c;
       }
-      gbase[t] = run ? bmeta[kMetaOff + t] + atomicAdd(&bmeta[kMetaCursor + t], run) : 0;
+      gbase[t] = run ? list + atomicAdd(&bmeta[kMetaCursor + t], run) : 0;
     }
     __syncthreads();
     if (path >= 0 && path < P_EMPTY) bin_rows[gbase[path] + woff[w][path] + rank] = i;
@@ -1407,8 +1396,10 @@ __global__ __launch_bounds__(BLOCK) void k_row_bitmap_staged(
 // wavefront), as were registers bounded below 120 (spills, each waited for).
 constexpr int kBits1Block = 256, kBits1Items = 4;  // threads and products per thread of the two bins
 constexpr int kBits2Block = 256, kBits2Items = 8;
-// rows of the second bin beyond those registers, in a launch of their own with
-// LDS for them (a workgroup's LDS for 4,096 entries leaves two on a CU)
+// Rows of the second bin beyond those registers, in a launch of their own: LDS
+// for 4,096 entries in the launch of the whole bin left two workgroups on a CU
+// (64 served products 2,217 us, 2,038 with two launches; 65,536 rows of 2..64
+// entries 775 and 767).
 constexpr int kBits3Block = 512, kBits3Items = 8;
 constexpr int32_t kBits2Products = kBits2Block * kBits2Items;
 constexpr int kBitsEntries = 256;

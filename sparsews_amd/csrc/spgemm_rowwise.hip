@@ -99,6 +99,13 @@ struct Fork {
   ~Fork() { (void)join(); }
 };
 
+// zero the bin metadata (a kernel, so the sequence can be graph-captured)
+__global__ void k_meta_clear(int32_t* __restrict__ bmeta, unsigned long long* __restrict__ maxub) {
+  const int t = threadIdx.x;
+  if (t < kMetaInts) bmeta[t] = 0;
+  if (t < 9) maxub[t] = 0;  // [8]: sum of the upper bounds
+}
+
 // The short-row product in two launches (k_short_rows, k_short_compact)
 // into the context's C arrays.  *ok is false when it does not apply (more
 // wavefronts than the compaction sums) or a row does not fit: the caller
@@ -307,7 +314,6 @@ static int rowwise_run(spws_ctx* ctx, int32_t m, int32_t kdim, int32_t n, const 
 
   rc = exclusive_scan<int64_t, int64_t>(ctx, ctx->row_ub.as<int64_t>(), ctx->row_off.as<int64_t>(), m);
   if (rc) return rc;
-  SPWS_LAUNCH(ctx, "bin_offsets", k_bin_offsets, dim3(1), dim3(64), 0, bmeta);
 
   const size_t slots = (size_t)(total_ub > 0 ? total_ub : 1);
   if (kValues) {
