@@ -3,11 +3,16 @@
 //
 // The key bits are split evenly over ceil(bits / 9) passes (34 bits: 9, 9,
 // 8, 8).  Per pass, three steps over tiles of kSortTile keys:
-//   1. k_radix_hist     per-tile digit histogram (LDS atomics), written
-//                       digit-major: hist[d * ntiles + t].
-//   2. exclusive scan   of the digit-major histogram -> global offset of
-//                       (digit d, tile t).
-//   3. k_radix_scatter  stable tile-local ranks by wavefront multisplit:
+//   1. k_radix_hist     per-tile digit histogram (LDS atomics), a row of
+//                       counts per tile: hist[t * digits + d].
+//   2. k_radix_chunks   the rows of a chunk of tiles become what the chunk's
+//                       earlier tiles hold of each digit, and the chunk's
+//                       total a row; k_radix_digits does the same to the
+//                       chunks' rows, with the digits' totals as last row.
+//                       (Few tiles: neither, the scatter sums the rows.)
+//   3. k_radix_scatter  adds the digits before (a scan of the totals), the
+//                       chunks before and the tiles before into the tile's
+//                       offset of each digit; stable tile-local ranks by wavefront multisplit:
 //                       each wave walks its contiguous quarter of the tile
 //                       64 keys at a time; one ballot per digit bit gives
 //                       the lanes holding the same digit, the group's rank
@@ -16,6 +21,11 @@
 //                       LDS in digit order (one buffer, two rounds) and
 //                       written out so that consecutive threads store
 //                       consecutive addresses of each digit's run.
+// Every row is read and written by consecutive threads.  (With the counts of a
+// digit side by side instead, one scan made every offset, but a tile stored
+// and loaded each of its 512 counts in a cache line of its own, shared with
+// tiles on other chiplets.  200,000 x 200,000 with 32 per row, two passes:
+// scatter 142 us, histogram 32, scans 28; rows: 131, 21, 25.)
 //
 // Where the pairs of the first pass come from and where those of the last go
 // is a template parameter each, so that keys made from a sparse structure are
@@ -42,7 +52,7 @@ constexpr int kSortDigitMax = 9;
 constexpr int kSortBucketsMax = 1 << kSortDigitMax;
 
 // int32 histogram entries one pass of radix_sort_pairs over n keys uses at
-// most (the scan of a pass covers as many).
+// most (the chunks' rows take at most as many).
 inline size_t radix_hist_entries(int64_t n) {
   return (size_t)div_up(n > 0 ? n : 1, kSortTile) * kSortBucketsMax;
 }
@@ -155,7 +165,7 @@ __device__ __forceinline__ int radix_digit(K key, int shift, uint32_t mask) {
 
 template <class K, class Source>
 __global__ __launch_bounds__(kSortBlock) void k_radix_hist(Source in, int64_t n, int shift, uint32_t mask,
-                                                           int32_t* __restrict__ hist, int64_t ntiles) {
+                                                           int32_t* __restrict__ hist) {
   __shared__ int32_t h[kSortBucketsMax];
   const int nb = (int)mask + 1;
   for (int d = threadIdx.x; d < nb; d += kSortBlock) h[d] = 0;
@@ -184,25 +194,99 @@ __global__ __launch_bounds__(kSortBlock) void k_radix_hist(Source in, int64_t n,
     }
   }
   __syncthreads();
-  for (int d = threadIdx.x; d < nb; d += kSortBlock) hist[(int64_t)d * ntiles + blockIdx.x] = h[d];
+  for (int d = threadIdx.x; d < nb; d += kSortBlock) hist[(int64_t)blockIdx.x * nb + d] = h[d];
+}
+
+// Tiles per chunk: 32 row reads are in flight at once; up to 128 tiles are one
+// chunk, which needs no second launch.
+constexpr int kSortChunk = 32;
+constexpr int kSortChunkOnly = 128;
+// Up to 64 tiles the scatter sums the rows itself, 16 reads in flight, and the
+// launch of one workgroup's width goes: 49 tiles, three passes, scatters 50 us
+// and 21 for the chunks' launches, 55 without them (whole call 180 -> 166 us);
+// four tiles, two passes, whole call 164 -> 149.  Reads grow with the square of
+// the tiles: at 128 tiles every tile would read 256 KB.
+constexpr int kSortDirect = 64;
+inline int64_t radix_chunk_tiles(int64_t ntiles) { return ntiles <= kSortChunkOnly ? ntiles : kSortChunk; }
+
+// hist's rows [c per, (c + 1) per) in place to their exclusive prefixes, their
+// sum to row c of chunk; a digit per thread.
+template <class Count>
+__global__ __launch_bounds__(kSortBlock) void k_radix_chunks(Count* __restrict__ hist, int64_t ntiles, int64_t per,
+                                                             int nb, Count* __restrict__ chunk) {
+  const int d = blockIdx.y * kSortBlock + threadIdx.x;
+  if (d >= nb) return;
+  const int64_t t0 = (int64_t)blockIdx.x * per;
+  const int64_t t1 = t0 + per < ntiles ? t0 + per : ntiles;
+  Count run = 0;
+  for (int64_t t = t0; t < t1; t += kSortChunk) {
+    Count c[kSortChunk];
+#pragma unroll
+    for (int q = 0; q < kSortChunk; ++q) c[q] = t + q < t1 ? hist[(t + q) * nb + d] : 0;
+#pragma unroll
+    for (int q = 0; q < kSortChunk; ++q) {
+      if (t + q < t1) hist[(t + q) * nb + d] = run;
+      run += c[q];
+    }
+  }
+  chunk[(int64_t)blockIdx.x * nb + d] = run;
+}
+
+// The chunks' rows to their exclusive prefixes, the digits' totals to row n:
+// 64 digits per workgroup, the rows split over its wavefronts.
+constexpr int kSortDigitsBlock = 1024;
+template <class Count>
+__global__ __launch_bounds__(kSortDigitsBlock) void k_radix_digits(Count* __restrict__ chunk, int64_t n, int nb) {
+  constexpr int kWaves = kSortDigitsBlock / kWave;
+  __shared__ Count part[kWaves][kWave];
+  const int lane = lane_id();
+  const int w = threadIdx.x / kWave;
+  const int d = blockIdx.x * kWave + lane;
+  const int64_t per = (n + kWaves - 1) / kWaves;
+  const int64_t c0 = w * per < n ? w * per : n;
+  const int64_t c1 = c0 + per < n ? c0 + per : n;
+  Count sum = 0;
+  if (d < nb) {
+#pragma unroll 8
+    for (int64_t c = c0; c < c1; ++c) sum += chunk[c * nb + d];
+  }
+  part[w][lane] = sum;
+  __syncthreads();
+  Count run = 0, all = 0;
+#pragma unroll
+  for (int q = 0; q < kWaves; ++q) {
+    const Count v = part[q][lane];
+    run += q < w ? v : 0;
+    all += v;
+  }
+  if (d >= nb) return;
+#pragma unroll 8
+  for (int64_t c = c0; c < c1; ++c) {
+    const Count v = chunk[c * nb + d];
+    chunk[c * nb + d] = run;
+    run += v;
+  }
+  if (w == 0) chunk[n * nb + d] = all;
 }
 
 template <class K, class Source, class Sink>
 __global__ __launch_bounds__(kSortBlock, 4) void k_radix_scatter(Source in, Sink out, int64_t n, int shift,
                                                                  uint32_t mask, int nbits,
-                                                                 const int32_t* __restrict__ offs, int64_t ntiles) {
+                                                                 const int32_t* __restrict__ hist,
+                                                                 const int32_t* __restrict__ chunk, int64_t chunks,
+                                                                 int64_t per) {
   constexpr int kWaves = kSortBlock / kWave;
   constexpr int kSub = kSortTile / kWaves;  // keys per wave
   static_assert(kSortBucketsMax == 2 * kSortBlock, "two digits per thread in the prefix step");
   static_assert(sizeof(K) <= sizeof(double), "one staging buffer for keys and values");
   __shared__ double stage[kSortTile];  // keys, then values, in digit order
-  // per (wavefront, digit): counts, then their prefixes over the wavefronts
-  // (at most kSortTile = 4096, so 16 bits: 38.9 KB of LDS in all, four
-  // workgroups per CU)
+  // per (wavefront, digit): counts, then where in the tile the wavefront's
+  // pairs of the digit start (at most kSortTile = 4096, so 16 bits: 39.0 KB of
+  // LDS in all, four workgroups per CU)
   __shared__ uint16_t wcnt[kWaves][kSortBucketsMax];
   static_assert(kSortTile < 65536, "per-wavefront digit prefixes fit 16 bits");
-  __shared__ int32_t dstart[kSortBucketsMax];
-  __shared__ int32_t scan_sh[kSortBlock / kWave + 1];
+  __shared__ int32_t goff[kSortBucketsMax];  // position of a digit's pairs, less their place in the tile
+  __shared__ int64_t scan_sh[kSortBlock / kWave + 1];
   K* sk = reinterpret_cast<K*>(stage);
 
   const int lane = lane_id();
@@ -223,6 +307,30 @@ __global__ __launch_bounds__(kSortBlock, 4) void k_radix_scatter(Source in, Sink
     if (idx < n) {
       raw[r] = in.raw(idx);
       val[r] = in.val(idx);
+    }
+  }
+  // digits 2t and 2t + 1 of thread t: their pairs in earlier tiles, and in all
+  int32_t before[2] = {}, all[2] = {};
+  if (chunks == 0) {  // few tiles: their rows summed here (nb is even)
+    if (2 * (int)threadIdx.x < nb) {
+#pragma unroll 16
+      for (int t = 0; t < (int)gridDim.x; ++t) {
+        const int2 c = *reinterpret_cast<const int2*>(hist + (int64_t)t * nb + 2 * threadIdx.x);
+        before[0] += t < (int)blockIdx.x ? c.x : 0;
+        before[1] += t < (int)blockIdx.x ? c.y : 0;
+        all[0] += c.x;
+        all[1] += c.y;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int d = 2 * threadIdx.x + e;
+      if (d < nb) {
+        before[e] = hist[(int64_t)blockIdx.x * nb + d];
+        all[e] = chunk[(chunks > 1 ? chunks * nb : 0) + d];  // a single chunk's row is the totals
+        if (chunks > 1) before[e] += chunk[((int64_t)blockIdx.x / per) * nb + d];
+      }
     }
   }
   int32_t owner[kSortItems] = {};
@@ -256,27 +364,39 @@ __global__ __launch_bounds__(kSortBlock, 4) void k_radix_scatter(Source in, Sink
   }
   __syncthreads();
   {
-    // thread t: digits 2t and 2t + 1: exclusive prefixes over the waves,
-    // then the tile-wide exclusive prefix of the digit totals
-    int32_t tot[2];
+    // thread t: digits 2t and 2t + 1: exclusive prefixes over the digits of
+    // the tile's counts and (from bit 16) of all, then over the waves
+    int32_t c[2][kWaves], tot[2];
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       const int d = 2 * threadIdx.x + e;
-      int32_t run = 0;
+      tot[e] = 0;
+#pragma unroll
+      for (int q = 0; q < kWaves; ++q) {
+        c[e][q] = d < nb ? wcnt[q][d] : 0;
+        tot[e] += c[e][q];
+      }
+    }
+    int64_t sum;
+    const int64_t st = block_excl_scan<int64_t, kSortBlock>(
+        (((int64_t)all[0] + all[1]) << 16) + tot[0] + tot[1], scan_sh, &sum);
+    int32_t in_tile = (int32_t)(st & 0xffff);  // the tile's counts sum to at most kSortTile
+    int32_t in_all = (int32_t)(st >> 16);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int d = 2 * threadIdx.x + e;
       if (d < nb) {
+        goff[d] = in_all + before[e] - in_tile;
+        int32_t run = in_tile;
 #pragma unroll
         for (int q = 0; q < kWaves; ++q) {
-          const int32_t c = wcnt[q][d];
           wcnt[q][d] = (uint16_t)run;
-          run += c;
+          run += c[e][q];
         }
       }
-      tot[e] = run;
+      in_tile += tot[e];
+      in_all += all[e];
     }
-    int32_t all;
-    const int32_t st = block_excl_scan<int32_t, kSortBlock>(tot[0] + tot[1], scan_sh, &all);
-    if (2 * (int)threadIdx.x < nb) dstart[2 * threadIdx.x] = st;
-    if (2 * (int)threadIdx.x + 1 < nb) dstart[2 * threadIdx.x + 1] = st + tot[0];
   }
   __syncthreads();
   const int64_t remain = n - base;
@@ -287,7 +407,8 @@ __global__ __launch_bounds__(kSortBlock, 4) void k_radix_scatter(Source in, Sink
     const int64_t idx = wbase + (int64_t)r * kWave + lane;
     if (idx < n) {
       const int d = radix_digit(key[r], shift, mask);
-      sk[dstart[d] + wcnt[w][d] + rank[r]] = key[r];
+      rank[r] += wcnt[w][d];
+      sk[rank[r]] = key[r];
     }
   }
   __syncthreads();
@@ -298,8 +419,7 @@ __global__ __launch_bounds__(kSortBlock, 4) void k_radix_scatter(Source in, Sink
     dst[it] = 0;
     if (i < tile_n) {
       const K k = sk[i];
-      const int d = radix_digit(k, shift, mask);
-      dst[it] = offs[(int64_t)d * ntiles + blockIdx.x] + (i - dstart[d]);
+      dst[it] = goff[radix_digit(k, shift, mask)] + i;
       out.key(dst[it], k);
     }
   }
@@ -308,10 +428,7 @@ __global__ __launch_bounds__(kSortBlock, 4) void k_radix_scatter(Source in, Sink
 #pragma unroll
   for (int r = 0; r < kSortItems; ++r) {
     const int64_t idx = wbase + (int64_t)r * kWave + lane;
-    if (idx < n) {
-      const int d = radix_digit(key[r], shift, mask);
-      stage[dstart[d] + wcnt[w][d] + rank[r]] = val[r];
-    }
+    if (idx < n) stage[rank[r]] = val[r];
   }
   __syncthreads();
 #pragma unroll
@@ -328,14 +445,20 @@ int radix_pass(spws_ctx* ctx, const Source& in, const Sink& out, int64_t n, int 
   int rc = ctx->radix_hist.ensure((2 * radix_hist_entries(n) + 1) * sizeof(int32_t));
   if (rc) return rc;
   int32_t* hist = ctx->radix_hist.as<int32_t>();
-  int32_t* offs = hist + radix_hist_entries(n);
+  int32_t* chunk = hist + radix_hist_entries(n);
   const uint32_t mask = (1u << nbits) - 1u;
+  const int nb = 1 << nbits;
+  const int64_t per = radix_chunk_tiles(ntiles), chunks = ntiles <= kSortDirect ? 0 : div_up(ntiles, per);
   SPWS_LAUNCH(ctx, "radix_hist", (k_radix_hist<K, Source>), dim3((unsigned)ntiles), dim3(kSortBlock), 0, in, n, shift,
-              mask, hist, ntiles);
-  rc = exclusive_scan<int32_t, int32_t>(ctx, hist, offs, ntiles << nbits);
-  if (rc) return rc;
+              mask, hist);
+  if (chunks > 0)
+    SPWS_LAUNCH(ctx, "radix_chunks", k_radix_chunks<int32_t>, dim3((unsigned)chunks, (unsigned)div_up(nb, kSortBlock)),
+                dim3(kSortBlock), 0, hist, ntiles, per, nb, chunk);
+  if (chunks > 1)
+    SPWS_LAUNCH(ctx, "radix_digits", k_radix_digits<int32_t>, dim3((unsigned)div_up(nb, kWave)), dim3(kSortDigitsBlock), 0,
+                chunk, chunks, nb);
   SPWS_LAUNCH(ctx, "radix_scatter", (k_radix_scatter<K, Source, Sink>), dim3((unsigned)ntiles), dim3(kSortBlock), 0,
-              in, out, n, shift, mask, nbits, (const int32_t*)offs, ntiles);
+              in, out, n, shift, mask, nbits, (const int32_t*)hist, (const int32_t*)chunk, chunks, per);
   return SPWS_OK;
 }
 

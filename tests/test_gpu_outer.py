@@ -492,6 +492,26 @@ def test_transpose_tiles_and_passes(ctx, n, pos64):
     np.testing.assert_array_equal(T.vals, A.vals[order])
 
 
+# the sort's tiles of 4,096 entries: 64 (the scatter sums their rows), 65 and
+# 128 (one chunk), 129 (five chunks, the last of one tile), 544 and 545 (more chunks than the 16 wavefronts that sum
+# them); one pass of fewer digits than a workgroup has threads, two passes
+@pytest.mark.parametrize("nnz", [64 * 4096, 64 * 4096 + 1, 128 * 4096, 128 * 4096 + 1, 544 * 4096, 544 * 4096 + 1])
+@pytest.mark.parametrize("n", [37, 70_000])
+def test_transpose_chunks_of_tiles(ctx, nnz, n):
+    print(f"case: transpose of {nnz} entries, {n} columns", flush=True)
+    from sparsews_amd.device import DeviceCSR, csr_transpose
+    rng = np.random.default_rng(n)
+    m = 1000
+    pos = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, m - 1)), [nnz]]).astype(np.int32)
+    crd = rng.integers(0, n, nnz).astype(np.int32)
+    A = CSR(m, n, pos, crd, rng.uniform(-1, 1, nnz))
+    T = csr_transpose(ctx, DeviceCSR.upload(ctx, A)).download()
+    order = np.argsort(crd, kind="stable")
+    np.testing.assert_array_equal(T.pos, np.concatenate([[0], np.cumsum(np.bincount(crd, minlength=n))]))
+    np.testing.assert_array_equal(T.crd, np.repeat(np.arange(m), np.diff(pos))[order])
+    np.testing.assert_array_equal(T.vals, A.vals[order])
+
+
 @pytest.mark.parametrize("n", [1, 3, 4, 4095, 4096, 4097, 8193, 16_384, 16_385, 20_483, 65_535, 65_536, 65_537, 200_001])
 def test_prefix_sum_lengths(ctx, n):
     """Row pointers (a prefix sum of n counts, most of them zero at the larger
