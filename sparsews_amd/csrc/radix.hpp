@@ -163,6 +163,18 @@ __device__ __forceinline__ int radix_digit(K key, int shift, uint32_t mask) {
   return (int)((key >> shift) & (K)mask);
 }
 
+// h[d] += 1 for every lane's digit d (d < 0: none); the first lane's digit is
+// added once for all the lanes that hold it.
+__device__ __forceinline__ void radix_count_common(int32_t* h, int d) {
+  uint64_t left = __ballot(d >= 0);
+  if (left == 0) return;  // uniform
+  const int lead = __builtin_ctzll(left);
+  const uint64_t same = __ballot(d == __builtin_amdgcn_readlane(d, lead));
+  if (lane_id() == lead) atomicAdd(&h[d], (int32_t)__popcll(same));
+  left &= ~same;
+  if (left >> lane_id() & 1) atomicAdd(&h[d], 1);
+}
+
 template <class K, class Source>
 __global__ __launch_bounds__(kSortBlock) void k_radix_hist(Source in, int64_t n, int shift, uint32_t mask,
                                                            int32_t* __restrict__ hist) {
@@ -187,10 +199,29 @@ __global__ __launch_bounds__(kSortBlock) void k_radix_hist(Source in, int64_t n,
       const int64_t idx = base + (int64_t)it * kSortBlock + threadIdx.x;
       if (idx < n) raw[it] = in.raw(idx);
     }
+    int dig[kSortItems];
 #pragma unroll
     for (int it = 0; it < kSortItems; ++it) {
       const int64_t idx = base + (int64_t)it * kSortBlock + threadIdx.x;
-      if (idx < n) atomicAdd(&h[radix_digit<K>(in.digit_bits(raw[it]), shift, mask)], 1);
+      dig[it] = idx < n ? radix_digit<K>(in.digit_bits(raw[it]), shift, mask) : -1;
+    }
+    // Adds to one counter follow one another: where digits are often equal,
+    // the first lane's is added once for all.  Neighbouring lanes show it: a
+    // digit of share p makes them equal p^2 of the time (6 of these 256 lanes:
+    // p = 0.15; 512 even digits: half a lane).  10M nonzeros of power-law
+    // coordinates, four passes: 134 us without, 74 with; 6.4M even columns, two
+    // passes: 22 either way (25 when every item looks for its own).
+    int equal = 0;
+#pragma unroll
+    for (int it = 0; it < kSortItems; it += kSortItems / 4)
+      equal += __popcll(__ballot(dig[it] >= 0 && dig[it] == __builtin_amdgcn_mov_dpp(dig[it], 0xB1, 0xF, 0xF, true)));
+    if (equal >= 6) {  // uniform
+#pragma unroll
+      for (int it = 0; it < kSortItems; ++it) radix_count_common(h, dig[it]);
+    } else {
+#pragma unroll
+      for (int it = 0; it < kSortItems; ++it)
+        if (dig[it] >= 0) atomicAdd(&h[dig[it]], 1);
     }
   }
   __syncthreads();

@@ -512,6 +512,24 @@ def test_transpose_chunks_of_tiles(ctx, nnz, n):
     np.testing.assert_array_equal(T.vals, A.vals[order])
 
 
+# one column's share of the entries: counted entry by entry, a common digit
+# counted once per wavefront, every entry the same; a last tile that is not full
+@pytest.mark.parametrize("share", [0.0, 0.3, 1.0])
+def test_transpose_common_columns(ctx, share):
+    print(f"case: transpose, one column with {share} of the entries", flush=True)
+    from sparsews_amd.device import DeviceCSR, csr_transpose
+    rng = np.random.default_rng(5)
+    m, n, nnz = 300, 5000, 3 * 4096 + 77
+    pos = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, m - 1)), [nnz]]).astype(np.int32)
+    crd = np.where(rng.random(nnz) < share, 4321, rng.integers(0, n, nnz)).astype(np.int32)
+    A = CSR(m, n, pos, crd, rng.uniform(-1, 1, nnz))
+    T = csr_transpose(ctx, DeviceCSR.upload(ctx, A)).download()
+    order = np.argsort(crd, kind="stable")
+    np.testing.assert_array_equal(T.pos, np.concatenate([[0], np.cumsum(np.bincount(crd, minlength=n))]))
+    np.testing.assert_array_equal(T.crd, np.repeat(np.arange(m), np.diff(pos))[order])
+    np.testing.assert_array_equal(T.vals, A.vals[order])
+
+
 @pytest.mark.parametrize("n", [1, 3, 4, 4095, 4096, 4097, 8193, 16_384, 16_385, 20_483, 65_535, 65_536, 65_537, 200_001])
 def test_prefix_sum_lengths(ctx, n):
     """Row pointers (a prefix sum of n counts, most of them zero at the larger
