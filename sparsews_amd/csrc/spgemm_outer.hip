@@ -2008,8 +2008,8 @@ static int outer_run(spws_ctx* ctx, const OuterArgs& a, int64_t* nnz_out) {
     method = (per_bucket >= 64.0 && W <= 4096 && max_pairs * W <= ((int64_t)1 << 28)) ? fused : 1;
     // Too few products per window: by rows, where the order of the sums may
     // change and the row kernels' column bitmap covers the output.  2,000
-    // rows of 8 squared (128k products): 276 us by the sort, 196 by rows;
-    // 30,000 rows of 2..32 (8.7M products): 2,770 and 370.
+    // rows of 8 squared (128k products): 231 us by the sort, 152 by rows;
+    // 30,000 rows of 2..32 (8.7M products): 663 and 357.
     if (method == 1 && !ctx->outer_auto_ordered && ctx->outer_max_products == 0 && ctx->outer_max_rows == 0 &&
         a.n <= kOuterRowsCols && products <= INT32_MAX && ctx->rw.force_path < 0 && m > 0 && a.a_ncols > 0 &&
         a.b_nrows > 0 && a.b_nrows < INT32_MAX - 1)
