@@ -7,6 +7,7 @@ increasing order, the order of the oracle's Gustavson restatement, so the
 values are compared bit-for-bit as well as against the 1e-12 bar.
 """
 import contextlib
+import time
 
 import numpy as np
 import pytest
@@ -14,7 +15,8 @@ import pytest
 import oracle
 from helpers import powerlaw_rows, random_csr, uniform_rows
 from sparsews_amd import formats, gen
-from sparsews_amd.device import DeviceArray, DeviceDCSR, set_outer_chunking, set_outer_method, spgemm_outer
+from sparsews_amd.device import (DeviceArray, DeviceCSR, DeviceCSR64, DeviceDCSR, csr64_transpose, csr_transpose,
+                                 set_outer_chunking, set_outer_method, spgemm_outer)
 from sparsews_amd.gen import CSR
 
 pytestmark = pytest.mark.gpu
@@ -466,6 +468,14 @@ def test_device_transpose(ctx, m, n, lo, hi, seed):
     np.testing.assert_array_equal(T.vals, O.vals)
 
 
+def transpose_csr(ctx, A, pos64):
+    """A's transpose on the device, from int32 or int64 row pointers."""
+    if not pos64:
+        return csr_transpose(ctx, DeviceCSR.upload(ctx, A))
+    return csr64_transpose(ctx, DeviceCSR64(A.nrows, A.ncols, A.nnz, DeviceArray.from_host(ctx, A.pos.astype(np.int64)),
+                                            DeviceArray.from_host(ctx, A.crd), DeviceArray.from_host(ctx, A.vals)))
+
+
 # one, two and three passes of the sort; rows longer than its tiles of 4,096,
 # tiles that start and end with runs of empty rows, rows that end on a tile
 @pytest.mark.parametrize("n", [1, 2, 512, 513, 262_145])
@@ -490,6 +500,55 @@ def test_transpose_tiles_and_passes(ctx, n, pos64):
     np.testing.assert_array_equal(T.pos, np.concatenate([[0], np.cumsum(np.bincount(crd, minlength=n))]))
     np.testing.assert_array_equal(T.crd, np.repeat(np.arange(A.nrows), lengths)[order])
     np.testing.assert_array_equal(T.vals, A.vals[order])
+
+
+# runs of empty rows inside a tile of 4,096 entries: up to eight rows an entry
+# in all (walked), one more (searched), and millions; before its first entry,
+# inside it, before its last
+@pytest.mark.parametrize("gap", [7 * 4096 - 1, 7 * 4096, 7 * 4096 + 1, 40_000, 3_000_000])
+@pytest.mark.parametrize("at", [0, 5000, 8191, 8192])
+@pytest.mark.parametrize("pos64", [False, True])
+def test_transpose_runs_of_empty_rows(ctx, gap, at, pos64):
+    print(f"case: transpose, {gap} empty rows before entry {at}, int64 positions {pos64}", flush=True)
+    rng = np.random.default_rng(gap + at)
+    lengths = np.concatenate([np.ones(at), np.zeros(gap), np.ones(9001 - at)]).astype(np.int64)
+    pos = np.concatenate([[0], np.cumsum(lengths)])
+    n, nnz = 700, 9001
+    crd = rng.integers(0, n, nnz).astype(np.int32)
+    A = CSR(len(lengths), n, pos.astype(np.int32), crd, rng.uniform(-1, 1, nnz))
+    T = transpose_csr(ctx, A, pos64).download()
+    order = np.argsort(crd, kind="stable")
+    np.testing.assert_array_equal(T.pos, np.concatenate([[0], np.cumsum(np.bincount(crd, minlength=n))]))
+    np.testing.assert_array_equal(T.crd, np.flatnonzero(lengths)[order])
+    np.testing.assert_array_equal(T.vals, A.vals[order])
+
+
+@pytest.mark.parametrize("spread", [False, True])
+def test_transpose_time_with_empty_rows(ctx, spread):
+    """Empty rows between the entries, in one run or everywhere, cost about
+    as much as the same rows behind the last entry: a tile's many rows are
+    not walked one after another.  (A search is at most 32 dependent reads on
+    top of a call of 60 us; one workgroup's walk over 6M rows takes 10 ms.)"""
+    print(f"case: transpose time with empty rows, spread {spread}", flush=True)
+    rng = np.random.default_rng(2)
+    m, n, nnz = 6_000_000, 5000, 100_000
+    crd = rng.integers(0, n, nnz).astype(np.int32)
+    vals = rng.uniform(-1, 1, nnz)
+    inside = np.sort(rng.choice(m, nnz, replace=False)) if spread else \
+        np.arange(nnz) + np.where(np.arange(nnz) < 50_000, 0, m - nnz)
+    times = []
+    for rows in (np.arange(nnz), inside):
+        pos = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=m))]).astype(np.int32)
+        A = DeviceCSR.upload(ctx, CSR(m, n, pos, crd, vals))
+        took = []
+        for _ in range(6):
+            ctx.sync()
+            t = time.perf_counter()
+            csr_transpose(ctx, A)
+            took.append(time.perf_counter() - t)
+        times.append(min(took[1:]))
+    print(f"behind {times[0] * 1e6:.0f} us, between {times[1] * 1e6:.0f} us", flush=True)
+    assert times[1] <= 5 * times[0]
 
 
 # the sort's tiles of 4,096 entries: 64 (the scatter sums their rows), 65 and
