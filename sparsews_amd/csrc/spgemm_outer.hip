@@ -95,29 +95,32 @@ __global__ __launch_bounds__(256) void k_outer_match(int32_t a_ncols, const int3
 
 // What the host decides the method on: sums and maxima over the rows' products
 // and matched A entries, and the operands' entry counts.
-enum OuterStat { kOsProducts, kOsBusyRows, kOsPairs, kOsMaxPairs, kOsNnzA, kOsNnzB, kOsCount };
+enum OuterStat { kOsProducts, kOsMaxProducts, kOsBusyRows, kOsPairs, kOsMaxPairs, kOsNnzA, kOsNnzB, kOsCount };
 
 __global__ __launch_bounds__(256) void k_outer_stats(int32_t m, const int64_t* __restrict__ row_ub,
                                                      const int32_t* __restrict__ row_pairs,
                                                      const int32_t* __restrict__ A_end,
                                                      const int32_t* __restrict__ B_end,
                                                      unsigned long long* __restrict__ out) {
-  int64_t products = 0, busy = 0, pairs = 0;
+  int64_t products = 0, most_products = 0, busy = 0, pairs = 0;
   int32_t most = 0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
     const int64_t u = row_ub[i];
     const int32_t p = row_pairs[i];
     products += u;
+    most_products = max(most_products, u);
     busy += u > 0;
     pairs += p;
     most = max(most, p);
   }
   products = wave_sum(products);
+  most_products = wave_max(most_products);
   busy = wave_sum(busy);
   pairs = wave_sum(pairs);
   most = wave_max(most);
   if (lane_id() == 0 && busy) {
     atomicAdd(&out[kOsProducts], (unsigned long long)products);
+    atomicMax(&out[kOsMaxProducts], (unsigned long long)most_products);
     atomicAdd(&out[kOsBusyRows], (unsigned long long)busy);
     atomicAdd(&out[kOsPairs], (unsigned long long)pairs);
     atomicMax(&out[kOsMaxPairs], (unsigned long long)most);
@@ -1910,6 +1913,14 @@ static int outer_fused(spws_ctx* ctx, const OuterArgs& a, int64_t En64, const in
 // product with B (whose int32 row pointers are widened to the outer product's).
 constexpr int32_t kOuterRowsCols = 1 << 17;  // columns at most (the row kernels' bitmap)
 
+// One row's products at most: a row beyond the block bins is one workgroup's
+// work (about 4 ns a product), while the sort shares all products out (0.055 ns
+// each and 225 us a call).  One row of L products among P, by rows and by the
+// sort: P = 0.15M, L = 16k 235 us and 254, P = 0.19M, L = 64k 417 and 343;
+// P = 8.7M, L = 34k 413 and 656, L = 136k 856 and 721; P = 48M, L = 320k 1,748
+// and 2,850, L = 1.28M 5,074 and 3,169.
+static int64_t outer_rows_longest(int64_t products) { return 16384 + products / 128; }
+
 static int outer_rows(spws_ctx* ctx, const OuterArgs& a, int64_t a_nnz, int64_t* nnz_out) {
   int rc;
   const size_t nn = (size_t)(a_nnz > 0 ? a_nnz : 1);
@@ -2007,12 +2018,13 @@ static int outer_run(spws_ctx* ctx, const OuterArgs& a, int64_t* nnz_out) {
     const int fused = ctx->outer_auto_ordered ? 3 : 4;
     method = (per_bucket >= 64.0 && W <= 4096 && max_pairs * W <= ((int64_t)1 << 28)) ? fused : 1;
     // Too few products per window: by rows, where the order of the sums may
-    // change and the row kernels' column bitmap covers the output.  2,000
-    // rows of 8 squared (128k products): 231 us by the sort, 152 by rows;
-    // 30,000 rows of 2..32 (8.7M products): 663 and 357.
+    // change, the row kernels' column bitmap covers the output and no row
+    // outweighs the others (outer_rows_longest).  2,000 rows of 8 squared
+    // (128k products): 231 us by the sort, 152 by rows; 30,000 rows of 2..32
+    // (8.7M products): 663 and 357; 100,000 of 60 (360M): 20,634 and 3,116.
     if (method == 1 && !ctx->outer_auto_ordered && ctx->outer_max_products == 0 && ctx->outer_max_rows == 0 &&
-        a.n <= kOuterRowsCols && products <= INT32_MAX && ctx->rw.force_path < 0 && m > 0 && a.a_ncols > 0 &&
-        a.b_nrows > 0 && a.b_nrows < INT32_MAX - 1)
+        a.n <= kOuterRowsCols && products <= INT32_MAX && hs[kOsMaxProducts] <= outer_rows_longest(products) &&
+        ctx->rw.force_path < 0 && m > 0 && a.a_ncols > 0 && a.b_nrows > 0 && a.b_nrows < INT32_MAX - 1)
       method = 5;
   }
   if (method == 5) {

@@ -291,6 +291,19 @@ def test_outer_by_rows(ctx, m, k, n, a, b, method, stored):
         check(C, A, B, exact_order=method == 1)
 
 
+@pytest.mark.parametrize("longest,method", [(16_516, 5), (16_517, 1)])
+def test_outer_by_rows_longest_row(ctx, longest, method):
+    """One row of at most 16,384 products and a 128th of all (16,516 of 17,016)
+    goes by rows, one product more keeps the balanced sort."""
+    print(f"case: outer by rows, longest row {longest}", flush=True)
+    k = 20_000
+    A = random_csr(51, k, np.concatenate([[longest], np.full(50, 10)]), 92, 0)
+    B = random_csr(k, 100_000, np.ones(k), 92, 1)
+    C = run_outer(ctx, A, B)
+    assert ctx.stats()["outer_method"] == method
+    check(C, A, B, exact_order=method == 1)
+
+
 def test_outer_wide_columns_64bit_keys(ctx):
     """ncols > 2^24 switches to 64-bit sort keys."""
     print("case: outer 64-bit keys", flush=True)
