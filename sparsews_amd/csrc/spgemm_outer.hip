@@ -1954,7 +1954,8 @@ static int outer_rows(spws_ctx* ctx, const OuterArgs& a, int64_t a_nnz, int64_t*
   return SPWS_OK;
 }
 
-static int outer_run(spws_ctx* ctx, const OuterArgs& a, int64_t* nnz_out) {
+// By the context's method, or `only` when not 0.
+static int outer_run(spws_ctx* ctx, const OuterArgs& a, int64_t* nnz_out, int only = 0) {
   int rc = ctx_activate(ctx);
   if (rc) return rc;
   SPWS_REQUIRE(a.m >= 0 && a.n >= 0 && a.kdim >= 0 && a.a_ncols >= 0 && a.b_nrows >= 0, SPWS_ERR_INVALID,
@@ -2003,7 +2004,7 @@ static int outer_run(spws_ctx* ctx, const OuterArgs& a, int64_t* nnz_out) {
   // workspace; on the 200k workload its step is about 7% shorter than the
   // bucket method's in order (3), and about 10% shorter again with the
   // unordered adds (within the 1e-12 bar; 3 keeps the sums reproducible).
-  int method = ctx->outer_method;
+  int method = only ? only : ctx->outer_method;
   int wlog = ctx->outer_window_log2;
   if (wlog == 0) {
     // about 1024 products per (row, window) bucket on average
@@ -2018,19 +2019,26 @@ static int outer_run(spws_ctx* ctx, const OuterArgs& a, int64_t* nnz_out) {
     const int fused = ctx->outer_auto_ordered ? 3 : 4;
     method = (per_bucket >= 64.0 && W <= 4096 && max_pairs * W <= ((int64_t)1 << 28)) ? fused : 1;
     // Too few products per window: by rows, where the order of the sums may
-    // change, the row kernels' column bitmap covers the output and no row
-    // outweighs the others (outer_rows_longest).  2,000 rows of 8 squared
+    // change, the row kernels' column bitmap covers the output, no row
+    // outweighs the others (outer_rows_longest) and the slots and the output,
+    // 24 bytes a product, take no more than the sort of one whole chunk.  2,000 rows of 8 squared
     // (128k products): 231 us by the sort, 152 by rows; 30,000 rows of 2..32
     // (8.7M products): 663 and 357; 100,000 of 60 (360M): 20,634 and 3,116.
     if (method == 1 && !ctx->outer_auto_ordered && ctx->outer_max_products == 0 && ctx->outer_max_rows == 0 &&
-        a.n <= kOuterRowsCols && products <= INT32_MAX && hs[kOsMaxProducts] <= outer_rows_longest(products) &&
+        a.n <= kOuterRowsCols && products <= max_products && hs[kOsMaxProducts] <= outer_rows_longest(products) &&
         ctx->rw.force_path < 0 && m > 0 && a.a_ncols > 0 && a.b_nrows > 0 && a.b_nrows < INT32_MAX - 1)
       method = 5;
   }
   if (method == 5) {
-    if ((rc = outer_rows(ctx, a, a_nnz, nnz_out))) return rc;
-    ctx->stats.nnz = *nnz_out;
-    return SPWS_OK;
+    rc = outer_rows(ctx, a, a_nnz, nnz_out);
+    ctx->stats.nnz = rc ? 0 : *nnz_out;
+    if (rc != SPWS_ERR_OOM) return rc;
+    // The sort may do with less: it cuts its chunks and grows its output.
+    // The row kernels' buffers make room for it.
+    for (DevBuf* b : {&ctx->slot_crd, &ctx->slot_val, &ctx->tr_keys, &ctx->tr_vals, &ctx->tr_out[0], &ctx->tr_out[1],
+                      &ctx->tr_out[2]})
+      b->release();
+    return outer_run(ctx, a, nnz_out, 1);
   }
   // the methods by chunks of output rows need every row's products and
   // matched entries on the host

@@ -7,6 +7,7 @@ increasing order, the order of the oracle's Gustavson restatement, so the
 values are compared bit-for-bit as well as against the 1e-12 bar.
 """
 import contextlib
+import ctypes
 import time
 
 import numpy as np
@@ -15,7 +16,8 @@ import pytest
 import oracle
 from helpers import powerlaw_rows, random_csr, uniform_rows
 from sparsews_amd import formats, gen
-from sparsews_amd.device import (DeviceArray, DeviceCSR, DeviceCSR64, DeviceDCSR, csr64_transpose, csr_transpose,
+from sparsews_amd._lib import lib
+from sparsews_amd.device import (Context, DeviceArray, DeviceCSR, DeviceCSR64, DeviceDCSR, csr64_transpose, csr_transpose,
                                  set_outer_chunking, set_outer_method, spgemm_outer)
 from sparsews_amd.gen import CSR
 
@@ -302,6 +304,44 @@ def test_outer_by_rows_longest_row(ctx, longest, method):
     C = run_outer(ctx, A, B)
     assert ctx.stats()["outer_method"] == method
     check(C, A, B, exact_order=method == 1)
+
+
+def test_outer_by_rows_falls_back_to_the_sort():
+    """By rows a product takes 24 bytes of slots and output per product at
+    once; beside a working set that leaves no room for them the automatic
+    choice still returns the product, by the sort in its chunks.  50M products
+    in two chunks, 1.2 GB by rows; 512 MiB are left after a product by the
+    sort, which needs nothing new."""
+    print("case: outer by rows without memory", flush=True)
+    m, k, n, r = 40_000, 3000, 131_072, 36
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    with Context(0) as ctx:
+        A = gen.uniform_csr(m, k, r, 93, 0)
+        dA = DeviceDCSR.from_csr(ctx, A.transpose())
+        dB = DeviceDCSR.from_csr(ctx, gen.uniform_csr(k, n, r, 93, 1))
+        with outer_method(ctx, 1):
+            S = spgemm_outer(ctx, dA, dB, m, k, n)
+            assert ctx.stats()["chunks"] == 2
+            want = [S.pos.to_host(), S.crd.to_host(), S.vals.to_host()]
+        hold = []
+        try:
+            while True:
+                assert lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+                room = free.value - (512 << 20)
+                if room < 64 << 20:
+                    break
+                hold.append(ctx.alloc(min(room, 32 << 30)))
+            C = spgemm_outer(ctx, dA, dB, m, k, n)
+            assert ctx.stats()["outer_method"] == 1
+            got = [C.pos.to_host(), C.crd.to_host(), C.vals.to_host()]
+        finally:
+            for p in hold:
+                ctx.free(p)
+        for g, w in zip(got, want):
+            np.testing.assert_array_equal(g, w)
+        C = spgemm_outer(ctx, dA, dB, m, k, n)
+        assert ctx.stats()["outer_method"] == 5
+        np.testing.assert_array_equal(C.crd.to_host(), want[1])
 
 
 def test_outer_wide_columns_64bit_keys(ctx):
