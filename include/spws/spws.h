@@ -173,8 +173,8 @@ int spws_ctx_set_outer_method(spws_ctx* ctx, int32_t method, int32_t window_log2
  * benchmark/CSC_CSR_T/nonfuse/CSC_CSR_T_hash.h:352: the m x n matrix
  * (pos[m+1], crd[nnz], vals[nnz]) becomes its n x m transpose in
  * out_pos[n+1], out_crd[nnz], out_vals[nnz] (device arrays the caller
- * provides), each output row's columns in increasing order.  Asynchronous
- * on the context's stream. */
+ * provides, which may be the input's own), each output row's columns in
+ * increasing order.  Asynchronous on the context's stream. */
 int spws_csr_transpose_dev(spws_ctx* ctx, int32_t m, int32_t n, int64_t nnz, const int32_t* pos,
                            const int32_t* crd, const double* vals, int32_t* out_pos, int32_t* out_crd,
                            double* out_vals);

@@ -16,6 +16,7 @@
 // apart by passes of their own and counted columns, 188 us now (two passes,
 // 2.9 TB/s in the scatters).
 #include <mutex>
+#include <utility>
 
 #include "radix.hpp"
 
@@ -74,8 +75,14 @@ __global__ __launch_bounds__(256) void k_tr_pos(int32_t n, int32_t nnz, const ui
   }
 }
 
+static bool overlap(const void* a, size_t an, const void* b, size_t bn) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return x < y + bn && y < x + an;
+}
+
 // The transpose on a context: its workspaces are the context's buffers
-// (tr_keys, tr_vals, and the radix and scan scratch).
+// (tr_keys, tr_vals, and the radix scratch).  Outputs may lie in the inputs'
+// memory.
 template <typename PosT>
 static int transpose_run(spws_ctx* ctx, int32_t m, int32_t n, int64_t nnz, const PosT* pos, const int32_t* crd,
                          const double* vals, int32_t* out_pos, int32_t* out_crd, double* out_vals) {
@@ -84,7 +91,17 @@ static int transpose_run(spws_ctx* ctx, int32_t m, int32_t n, int64_t nnz, const
   if ((rc = ctx->tr_keys.ensure(2 * nn * 8)) || (rc = ctx->tr_vals.ensure(2 * nn * 8))) return rc;
   uint64_t* const keys[2] = {ctx->tr_keys.as<uint64_t>(), ctx->tr_keys.as<uint64_t>() + nn};
   double* const kv[2] = {ctx->tr_vals.as<double>(), ctx->tr_vals.as<double>() + nn};
-  const int bits = column_bits(n);
+  int bits = column_bits(n);
+  // A single pass writes the outputs while other workgroups still read the
+  // inputs.  Where they share memory the columns are sorted on further bits,
+  // all zero, in two passes: only the first reads the inputs.
+  if (radix_passes(bits) == 1) {
+    bool shared = false;
+    for (const auto& [out, on] : {std::pair<const void*, size_t>{out_crd, nn * 4}, {out_vals, nn * 8}})
+      shared = shared || overlap(out, on, pos, ((size_t)m + 1) * sizeof(PosT)) || overlap(out, on, crd, nn * 4) ||
+               overlap(out, on, vals, nn * 8);
+    if (shared) bits = kSortDigitMax + 1;
+  }
   // the sorted columns take the key buffer that the last pass does not read
   uint32_t* const cols = reinterpret_cast<uint32_t*>(keys[(radix_passes(bits) - 1) & 1]);
   const bool any = m > 0 && nnz > 0;

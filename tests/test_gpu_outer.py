@@ -16,6 +16,7 @@ import pytest
 import oracle
 from helpers import powerlaw_rows, random_csr, uniform_rows
 from sparsews_amd import formats, gen
+from sparsews_amd._lib import check as capi_check
 from sparsews_amd._lib import lib
 from sparsews_amd.device import (Context, DeviceArray, DeviceCSR, DeviceCSR64, DeviceDCSR, csr64_transpose, csr_transpose,
                                  set_outer_chunking, set_outer_method, spgemm_outer)
@@ -602,6 +603,31 @@ def test_transpose_time_with_empty_rows(ctx, spread):
         times.append(min(took[1:]))
     print(f"behind {times[0] * 1e6:.0f} us, between {times[1] * 1e6:.0f} us", flush=True)
     assert times[1] <= 5 * times[0]
+
+
+@pytest.mark.parametrize("n", [1, 2, 300, 512, 513])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_transpose_in_place(ctx, n, noalloc):
+    """The outputs in the inputs' own arrays, in one pass of the sort and in
+    two: no tile's entries are overwritten before they are read."""
+    print(f"case: transpose in place n={n} no-alloc {noalloc}", flush=True)
+    rng = np.random.default_rng(n)
+    nnz = 200_000
+    pos = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, n - 1)), [nnz]]).astype(np.int32)
+    crd = rng.integers(0, n, nnz).astype(np.int32)
+    vals = rng.uniform(-1, 1, nnz)
+    order = np.argsort(crd, kind="stable")
+    for _ in range(3):
+        d = [DeviceArray.from_host(ctx, x) for x in (pos, crd, vals)]
+        p = [x.ptr for x in d]
+        if noalloc:
+            capi_check(lib().spws_csr_transpose_dev_noalloc(ctypes.c_void_p(ctx.stream), n, n, nnz, *p, *p))
+        else:
+            capi_check(lib().spws_csr_transpose_dev(ctx.h, n, n, nnz, *p, *p))
+        ctx.sync()
+        np.testing.assert_array_equal(d[0].to_host(), np.concatenate([[0], np.cumsum(np.bincount(crd, minlength=n))]))
+        np.testing.assert_array_equal(d[1].to_host(), np.repeat(np.arange(n), np.diff(pos))[order])
+        np.testing.assert_array_equal(d[2].to_host(), vals[order])
 
 
 # the sort's tiles of 4,096 entries: 64 (the scatter sums their rows), 65 and
