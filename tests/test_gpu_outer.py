@@ -669,14 +669,40 @@ def test_transpose_common_columns(ctx, share):
 
 
 @pytest.mark.parametrize("n", [1, 3, 4, 4095, 4096, 4097, 8193, 16_384, 16_385, 20_483, 65_535, 65_536, 65_537, 200_001])
-def test_prefix_sum_lengths(ctx, n):
-    """Row pointers (a prefix sum of n counts, most of them zero at the larger
-    n) of a transpose into n rows, at the edges of the scan's tiles."""
-    print(f"case: prefix sum of {n} counts", flush=True)
-    from sparsews_amd.device import DeviceCSR, csr_transpose
+def test_transpose_row_pointers(ctx, n):
+    """Row pointers of a transpose into n rows, most of them empty at the
+    larger n: each is the first sorted column that is not before it."""
+    print(f"case: row pointers of {n} rows", flush=True)
     A = uniform_rows(700, n, 0, min(n, 9), n, 0)
     T = csr_transpose(ctx, DeviceCSR.upload(ctx, A)).download()
     np.testing.assert_array_equal(T.pos, np.concatenate([[0], np.cumsum(np.bincount(A.crd, minlength=n))]))
+
+
+@pytest.mark.parametrize("m", [1, 4095, 4096, 4097, 16_384, 16_385, 65_535, 65_536, 65_537])
+def test_prefix_sum_of_fused_row_counts(ctx, m):
+    """The fused method's row pointers: the 64-bit prefix sum of m 32-bit row
+    counts, at the edges of the scan's tiles and of its one-launch form."""
+    print(f"case: outer prefix sum of {m} row counts", flush=True)
+    A, B = uniform_rows(m, 300, 0, 3, 94, 0), uniform_rows(300, 200, 0, 5, 94, 1)
+    with outer_method(ctx, 3):
+        check(run_outer(ctx, A, B), A, B)
+
+
+@pytest.mark.parametrize("rows", [4095, 16_383, 16_384, 16_385, 65_537])
+def test_prefix_sum_unaligned(ctx, rows):
+    """The bucket method's second chunk of output rows begins at an odd row:
+    the scan's input is not 16-byte aligned, below and above the lengths
+    that one workgroup takes alone."""
+    print(f"case: outer prefix sum of {rows} unaligned counts", flush=True)
+    first = rows | 1
+    A, B = uniform_rows(first + rows, 300, 0, 3, 95, 0), uniform_rows(300, 200, 0, 5, 95, 1)
+    try:
+        set_outer_chunking(ctx, 0, first)
+        with outer_method(ctx, 2):
+            check(run_outer(ctx, A, B), A, B)
+            assert ctx.stats()["chunks"] == 2
+    finally:
+        set_outer_chunking(ctx, 0, 0)
 
 
 @pytest.mark.parametrize("method", METHODS)

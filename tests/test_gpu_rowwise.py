@@ -296,6 +296,24 @@ def test_rows_of_many_a_entries(ctx, a_len, b_len, ncols, path):
     np.testing.assert_array_equal(spgemm_rowwise_symbolic(ctx, dA, dB), C.pos)
 
 
+@pytest.mark.parametrize("m", [1, 3, 4, 4095, 4096, 4097, 8193, 16_384, 16_385, 20_483, 65_535, 65_536, 65_537,
+                               200_001])
+def test_prefix_sum_lengths(ctx, m):
+    """Slot offsets (a 64-bit prefix sum of m upper bounds) and row pointers (a
+    32-bit one of m row lengths), at the edges of the scan's tiles and of its
+    one-launch form; a row of 300 products keeps the short-row path out."""
+    print(f"case: prefix sums of {m} rows", flush=True)
+    B = uniform_rows(400, 900, 1, 3, 96, 1)
+    lengths = np.random.default_rng(m).integers(0, 4, m)
+    lengths[m // 2] = 300
+    A = random_csr(m, 400, lengths, 96, 0)
+    C = run(ctx, A, B)
+    assert ctx.stats()["rows_per_path"][2] == 1
+    check(C, A, B)
+    dA, dB = DeviceCSR.upload(ctx, A), DeviceCSR.upload(ctx, B)
+    np.testing.assert_array_equal(spgemm_rowwise_symbolic(ctx, dA, dB), C.pos)
+
+
 # (B rows of 45 entries, B rows of 1) that a row of each kind takes
 ROW_KINDS = [
     (30, 0),    # 1,350 products, the bulk: second block bin, from registers
