@@ -938,7 +938,8 @@ def run_fusion(args):
         out["F"] = spgemm_outer(ctx, dB, dAc, n, k, m)
 
     names = ("radix_scatter", "radix_hist", "outer_expand", "outer_reduce", "bk_expand", "bk_count", "bk_reduce",
-             "fz_count", "fz_reduce")
+             "fz_count", "fz_reduce", "short_rows", "short_compact", "row_wave", "row_bitmap", "row_bitmap_long",
+             "row_count", "compact")
     sec, dom, dom_times, bd = timed_steps(ctx, step, 3, 1,
                                           lambda b: max((x for x in names if x in b), key=lambda x: b[x][0]))
     compulsory = 4 * (2 * k + 2) + 12 * nin + 8 * (n + 1) + 12 * nnz
