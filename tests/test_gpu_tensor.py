@@ -280,15 +280,17 @@ def test_ttm_segments_of_64(ctx):
     assert oracle.max_value_error(Y.ravel(), exact.ravel(), (np.abs(V) @ np.abs(U)).ravel()) <= TOL
 
 
+@pytest.mark.parametrize("method", [0, 1])
 @pytest.mark.parametrize("R", [16, 40])
-def test_ttm_long_fibers(ctx, R):
-    """Fibers of 139-200 nonzeros: two 128-nonzero work items per fiber
-    (partial sums combined in item order), items longer than one 16-lane
-    load, ranks in three 16-lane slices for R = 40."""
-    print(f"case: ttm long fibers R={R}", flush=True)
+def test_ttm_long_fibers(ctx, R, method):
+    """Fibers of 139-200 nonzeros, by roots and windows (the automatic choice
+    here) and by sorting: there most are longer than the group that starts
+    them follows (segments of 32 and 128 nonzeros beyond), so segments inside
+    them leave partial sums; ranks in three 16-lane slices for R = 40."""
+    print(f"case: ttm long fibers R={R} method {method}", flush=True)
     X = gen.zipf_coo3((20, 30, 400), 100000, (None, None, None), 21, 5, -1.0, 1.0)
     U = np.random.default_rng(30 + R).uniform(-1, 1, (400, R))
-    fi, fj, Y = run_ttm(ctx, X, U)
+    fi, fj, Y = run_ttm(ctx, X, U, method)
     csf = formats.csf3_from_coo(X, (0, 2, 1))
     ok, oj, ol, ov = oracle.ttm_hash_il(csf, formats.dense_as_dcsr(U), 20, 30, R)
     np.testing.assert_array_equal(np.repeat(fi, R), ok)
@@ -297,15 +299,16 @@ def test_ttm_long_fibers(ctx, R):
     assert oracle.max_value_error(Y.ravel(), ov, absY[fi, fj].ravel()) <= TOL
 
 
-def test_ttm_many_items_per_group(ctx):
-    """~400k short fibers: each 16-lane group of the accumulation grid walks
-    about two dozen items, with the next item's keys and record loaded
-    ahead."""
-    print("case: ttm many items per group", flush=True)
+@pytest.mark.parametrize("method", [0, 1])
+def test_ttm_many_short_fibers(ctx, method):
+    """~400k short fibers, by roots and windows (all of them light roots) and
+    by sorting: there each 16-lane group writes about thirty fibers of its
+    segment of 32 nonzeros."""
+    print(f"case: ttm many short fibers method {method}", flush=True)
     X = gen.zipf_coo3((3000, 3000, 50), 400000, (None, None, None), 22, 5, -1.0, 1.0)
     R = 16
     U = np.random.default_rng(40).uniform(-1, 1, (50, R))
-    fi, fj, Y = run_ttm(ctx, X, U)
+    fi, fj, Y = run_ttm(ctx, X, U, method)
     csf = formats.csf3_from_coo(X, (0, 2, 1))
     ok, oj, ol, ov = oracle.ttm_hash_il(csf, formats.dense_as_dcsr(U), 3000, 3000, R)
     np.testing.assert_array_equal(np.repeat(fi, R), ok)
