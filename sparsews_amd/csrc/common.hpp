@@ -167,8 +167,6 @@ struct StreamScope {
 // Tin/Tout in {int32_t, int64_t}.  Uses ctx->scan_tmp.
 template <class Tin, class Tout>
 int exclusive_scan(spws_ctx* ctx, const Tin* in, Tout* out, int64_t n);
-// Bytes of ctx->scan_tmp that exclusive_scan of n values of elem_bytes uses.
-size_t scan_scratch_bytes(int64_t n, size_t elem_bytes);
 
 // The m x n CSR's transpose in the given device arrays, and the row-wise
 // product C = A * B (in ctx->out_pos, out_crd, out_val), for other drivers.

@@ -347,11 +347,6 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_tile_fused(const Tin* __res
   }
 }
 
-size_t scan_scratch_bytes(int64_t n, size_t elem_bytes) {
-  if (n <= 4 * (int64_t)kScanTile) return 0;
-  return (size_t)(div_up(n, kScanTile) + 1) * 2 * elem_bytes;
-}
-
 template <class Tin, class Tout>
 int exclusive_scan(spws_ctx* ctx, const Tin* in, Tout* out, int64_t n) {
   if (n <= kScanSmall && reinterpret_cast<uintptr_t>(in) % 16 == 0) {

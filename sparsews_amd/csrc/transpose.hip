@@ -156,20 +156,15 @@ static int scratch_address(int device, unsigned char** out) {
 
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Bytes of each workspace the transpose of nnz entries into n rows uses
-// (keys, values, radix histograms, scan partials), and 4 more per output row:
-// the documented limit counts them.
+// Bytes of each workspace the transpose of nnz entries uses.
 struct TransposeScratch {
-  size_t keys, vals, counts, hist, scan, total;
-  TransposeScratch(int64_t nnz, int32_t n) {
+  size_t keys, vals, hist, total;
+  explicit TransposeScratch(int64_t nnz) {
     const size_t nn = (size_t)(nnz > 0 ? nnz : 1);
     keys = align256(2 * nn * 8);
     vals = align256(2 * nn * 8);
-    counts = align256((size_t)(n > 0 ? n : 1) * 4);
-    const size_t hn = radix_hist_entries((int64_t)nn);
-    hist = align256((2 * hn + 1) * 4);
-    scan = align256(std::max(scan_scratch_bytes((int64_t)hn, 4), scan_scratch_bytes((int64_t)n, 4)) + 4);
-    total = keys + vals + counts + hist + scan;
+    hist = align256((2 * radix_hist_entries((int64_t)nn) + 1) * 4);
+    total = keys + vals + hist;
   }
 };
 
@@ -212,11 +207,11 @@ extern "C" int spws_csr_transpose_dev_noalloc(void* stream, int32_t m, int32_t n
                                               int32_t* out_crd, double* out_vals) {
   int rc = check_args(m, n, nnz, pos, crd, vals, out_pos, out_crd, out_vals);
   if (rc) return rc;
-  const TransposeScratch need(nnz, n);
+  const TransposeScratch need(nnz);
   SPWS_REQUIRE(need.total <= kNoAllocScratchBytes, SPWS_ERR_UNSUPPORTED,
-               "the no-allocation transpose of %lld entries into %d rows needs %zu bytes of scratch; the fixed "
-               "scratch holds %zu (about 33 bytes per entry plus 4 per row)",
-               (long long)nnz, n, need.total, kNoAllocScratchBytes);
+               "the no-allocation transpose of %lld entries needs %zu bytes of scratch; the fixed scratch holds %zu "
+               "(about 33 bytes per entry)",
+               (long long)nnz, need.total, kNoAllocScratchBytes);
   int device = 0;
   SPWS_HIP(hipGetDevice(&device));
   unsigned char* base;
@@ -230,7 +225,5 @@ extern "C" int spws_csr_transpose_dev_noalloc(void* stream, int32_t m, int32_t n
   local.tr_vals.borrow(base + off, need.vals);
   off += need.vals;
   local.radix_hist.borrow(base + off, need.hist);
-  off += need.hist;
-  local.scan_tmp.borrow(base + off, need.scan);
   return transpose_run(&local, m, n, nnz, pos, crd, vals, out_pos, out_crd, out_vals);
 }

@@ -1,7 +1,7 @@
 """The no-allocation CSR transpose (spws_csr_transpose_dev_noalloc) on the
 GPU, through the C ABI: bit-identical to spws_csr_transpose_dev on two calls
 in a row, the second one smaller (the shared scratch keeps the first call's
-contents, so a stale column count or histogram would show), and inputs
+contents, so a stale histogram would show), and inputs
 beyond the fixed scratch refused before any launch.
 """
 import ctypes as C
@@ -44,6 +44,17 @@ def test_noalloc_transpose_matches_the_allocating_entry(ctx, sizes):
         np.testing.assert_array_equal(pos, S.indptr)
         np.testing.assert_array_equal(crd, S.indices)
         np.testing.assert_array_equal(val, S.data)
+
+
+def test_noalloc_transpose_of_the_most_entries(ctx):
+    """1.5M entries, into more rows than entries."""
+    print("case: no-alloc transpose of 1.5M entries", flush=True)
+    m, n = 15_000, 2_000_000
+    A = random_csr(m, n, np.full(m, 100), 42, 0)
+    dA = DeviceCSR.upload(ctx, A)
+    T = csr_transpose(ctx, dA).download()
+    for got, want in zip(noalloc_transpose(ctx, dA), (T.pos, T.crd, T.vals)):
+        np.testing.assert_array_equal(got, want)
 
 
 def test_noalloc_transpose_refuses_inputs_beyond_the_scratch(ctx):
