@@ -51,18 +51,24 @@ constexpr int kSortTile = kSortBlock * kSortItems;
 constexpr int kSortDigitMax = 9;
 constexpr int kSortBucketsMax = 1 << kSortDigitMax;
 
-// int32 histogram entries one pass of radix_sort_pairs over n keys uses at
-// most (the chunks' rows take at most as many).
+// Tiles per chunk: 32 row reads are in flight at once; up to 128 tiles are one
+// chunk, which needs no second launch.
+constexpr int kSortChunk = 32;
+constexpr int kSortChunkOnly = 128;
+
+// int32 entries of ctx->radix_hist that one pass over n keys uses at most: a
+// row of digits per tile, one per chunk of tiles, and the totals.
 inline size_t radix_hist_entries(int64_t n) {
-  return (size_t)div_up(n > 0 ? n : 1, kSortTile) * kSortBucketsMax;
+  const int64_t tiles = div_up(n > 0 ? n : 1, kSortTile);
+  return (size_t)(tiles + div_up(tiles, kSortChunk) + 1) * kSortBucketsMax;
 }
 
 // Sorts keys[0, n) by bits [begin_bit, end_bit) carrying vals along, using
 // keys_alt / vals_alt as the ping-pong buffers.  On return *in_alt says
 // whether the sorted data ended up in the _alt buffers.  K is uint32_t or
-// uint64_t.  Uses ctx->radix_hist and the scan scratch.  With vals_first,
-// the values are read from there instead of vals (which then needs no
-// copy of them; it is still filled when no pass runs).
+// uint64_t.  Uses ctx->radix_hist.  With vals_first, the values are read from
+// there instead of vals (which then needs no copy of them; it is still filled
+// when no pass runs).
 template <class K>
 int radix_sort_pairs(spws_ctx* ctx, K* keys, double* vals, K* keys_alt, double* vals_alt, int64_t n, int begin_bit,
                      int end_bit, bool* in_alt, const double* vals_first = nullptr);
@@ -257,10 +263,6 @@ __global__ __launch_bounds__(kSortBlock) void k_radix_hist(Source in, int64_t n,
   for (int d = threadIdx.x; d < nb; d += kSortBlock) hist[(int64_t)blockIdx.x * nb + d] = h[d];
 }
 
-// Tiles per chunk: 32 row reads are in flight at once; up to 128 tiles are one
-// chunk, which needs no second launch.
-constexpr int kSortChunk = 32;
-constexpr int kSortChunkOnly = 128;
 // Up to 64 tiles the scatter sums the rows itself, 16 reads in flight, and the
 // launch of one workgroup's width goes: 49 tiles, three passes, scatters 50 us
 // and 21 for the chunks' launches, 55 without them (whole call 180 -> 166 us);
@@ -502,10 +504,10 @@ __global__ __launch_bounds__(kSortBlock, 4) void k_radix_scatter(Source in, Sink
 template <class K, class Source, class Sink>
 int radix_pass(spws_ctx* ctx, const Source& in, const Sink& out, int64_t n, int shift, int nbits) {
   const int64_t ntiles = div_up(n, kSortTile);
-  int rc = ctx->radix_hist.ensure((2 * radix_hist_entries(n) + 1) * sizeof(int32_t));
+  int rc = ctx->radix_hist.ensure(radix_hist_entries(n) * sizeof(int32_t));
   if (rc) return rc;
   int32_t* hist = ctx->radix_hist.as<int32_t>();
-  int32_t* chunk = hist + radix_hist_entries(n);
+  int32_t* chunk = hist + ntiles * kSortBucketsMax;
   const uint32_t mask = (1u << nbits) - 1u;
   const int nb = 1 << nbits;
   const int64_t per = radix_chunk_tiles(ntiles), chunks = ntiles <= kSortDirect ? 0 : div_up(ntiles, per);

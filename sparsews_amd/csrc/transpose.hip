@@ -163,7 +163,7 @@ struct TransposeScratch {
     const size_t nn = (size_t)(nnz > 0 ? nnz : 1);
     keys = align256(2 * nn * 8);
     vals = align256(2 * nn * 8);
-    hist = align256((2 * radix_hist_entries((int64_t)nn) + 1) * 4);
+    hist = align256(radix_hist_entries((int64_t)nn) * 4);
     total = keys + vals + hist;
   }
 };
