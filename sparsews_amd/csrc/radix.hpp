@@ -273,16 +273,15 @@ inline int64_t radix_chunk_tiles(int64_t ntiles) { return ntiles <= kSortChunkOn
 
 // hist's rows [c per, (c + 1) per) in place to their exclusive prefixes, their
 // sum to row c of chunk; a digit per thread.
-template <class Count>
-__global__ __launch_bounds__(kSortBlock) void k_radix_chunks(Count* __restrict__ hist, int64_t ntiles, int64_t per,
-                                                             int nb, Count* __restrict__ chunk) {
+[[maybe_unused]] static __global__ __launch_bounds__(kSortBlock) void k_radix_chunks(
+    int32_t* __restrict__ hist, int64_t ntiles, int64_t per, int nb, int32_t* __restrict__ chunk) {
   const int d = blockIdx.y * kSortBlock + threadIdx.x;
   if (d >= nb) return;
   const int64_t t0 = (int64_t)blockIdx.x * per;
   const int64_t t1 = t0 + per < ntiles ? t0 + per : ntiles;
-  Count run = 0;
+  int32_t run = 0;
   for (int64_t t = t0; t < t1; t += kSortChunk) {
-    Count c[kSortChunk];
+    int32_t c[kSortChunk];
 #pragma unroll
     for (int q = 0; q < kSortChunk; ++q) c[q] = t + q < t1 ? hist[(t + q) * nb + d] : 0;
 #pragma unroll
@@ -297,34 +296,34 @@ __global__ __launch_bounds__(kSortBlock) void k_radix_chunks(Count* __restrict__
 // The chunks' rows to their exclusive prefixes, the digits' totals to row n:
 // 64 digits per workgroup, the rows split over its wavefronts.
 constexpr int kSortDigitsBlock = 1024;
-template <class Count>
-__global__ __launch_bounds__(kSortDigitsBlock) void k_radix_digits(Count* __restrict__ chunk, int64_t n, int nb) {
+[[maybe_unused]] static __global__ __launch_bounds__(kSortDigitsBlock) void k_radix_digits(
+    int32_t* __restrict__ chunk, int64_t n, int nb) {
   constexpr int kWaves = kSortDigitsBlock / kWave;
-  __shared__ Count part[kWaves][kWave];
+  __shared__ int32_t part[kWaves][kWave];
   const int lane = lane_id();
   const int w = threadIdx.x / kWave;
   const int d = blockIdx.x * kWave + lane;
   const int64_t per = (n + kWaves - 1) / kWaves;
   const int64_t c0 = w * per < n ? w * per : n;
   const int64_t c1 = c0 + per < n ? c0 + per : n;
-  Count sum = 0;
+  int32_t sum = 0;
   if (d < nb) {
 #pragma unroll 8
     for (int64_t c = c0; c < c1; ++c) sum += chunk[c * nb + d];
   }
   part[w][lane] = sum;
   __syncthreads();
-  Count run = 0, all = 0;
+  int32_t run = 0, all = 0;
 #pragma unroll
   for (int q = 0; q < kWaves; ++q) {
-    const Count v = part[q][lane];
+    const int32_t v = part[q][lane];
     run += q < w ? v : 0;
     all += v;
   }
   if (d >= nb) return;
 #pragma unroll 8
   for (int64_t c = c0; c < c1; ++c) {
-    const Count v = chunk[c * nb + d];
+    const int32_t v = chunk[c * nb + d];
     chunk[c * nb + d] = run;
     run += v;
   }
@@ -514,10 +513,10 @@ int radix_pass(spws_ctx* ctx, const Source& in, const Sink& out, int64_t n, int 
   SPWS_LAUNCH(ctx, "radix_hist", (k_radix_hist<K, Source>), dim3((unsigned)ntiles), dim3(kSortBlock), 0, in, n, shift,
               mask, hist);
   if (chunks > 0)
-    SPWS_LAUNCH(ctx, "radix_chunks", k_radix_chunks<int32_t>, dim3((unsigned)chunks, (unsigned)div_up(nb, kSortBlock)),
+    SPWS_LAUNCH(ctx, "radix_chunks", k_radix_chunks, dim3((unsigned)chunks, (unsigned)div_up(nb, kSortBlock)),
                 dim3(kSortBlock), 0, hist, ntiles, per, nb, chunk);
   if (chunks > 1)
-    SPWS_LAUNCH(ctx, "radix_digits", k_radix_digits<int32_t>, dim3((unsigned)div_up(nb, kWave)), dim3(kSortDigitsBlock), 0,
+    SPWS_LAUNCH(ctx, "radix_digits", k_radix_digits, dim3((unsigned)div_up(nb, kWave)), dim3(kSortDigitsBlock), 0,
                 chunk, chunks, nb);
   SPWS_LAUNCH(ctx, "radix_scatter", (k_radix_scatter<K, Source, Sink>), dim3((unsigned)ntiles), dim3(kSortBlock), 0,
               in, out, n, shift, mask, nbits, (const int32_t*)hist, (const int32_t*)chunk, chunks, per);

@@ -142,7 +142,6 @@ static int bits_of(int64_t v) {  // bits for values in [0, v)
 // nonzero whose two rows share no stored column takes no part (the
 // reference's co-iteration never reaches it): it gets the row key `drop_i`,
 // past every output row, so the sort moves it to the end, and is counted.
-template <bool kMask>
 __global__ __launch_bounds__(256) void k_mttkrp_keys(int64_t nnz, const int32_t* __restrict__ leaf_fiber,
                                                      const int32_t* __restrict__ fiber_root,
                                                      const int32_t* __restrict__ l1_crd,
@@ -157,16 +156,14 @@ __global__ __launch_bounds__(256) void k_mttkrp_keys(int64_t nnz, const int32_t*
     const uint64_t j = (uint32_t)l1_crd[fiber_root[f]];
     const uint64_t k = (uint32_t)l2_crd[f];
     uint64_t i = (uint32_t)l3_crd[e];
-    if (kMask && (mB[j] & mC[k]) == 0) {
+    if ((mB[j] & mC[k]) == 0) {
       i = drop_i;
       ++nd;
     }
     keys[e] = (i << (bj + bk)) | (j << bk) | k;
   }
-  if (kMask) {
-    nd = wave_sum(nd);
-    if (lane_id() == 0 && nd) atomicAdd(dropped, nd);
-  }
+  nd = wave_sum(nd);
+  if (lane_id() == 0 && nd) atomicAdd(dropped, nd);
 }
 
 // The bucketed nonzeros in tiles of one workgroup, `seg` consecutive ones per
@@ -712,7 +709,6 @@ __global__ __launch_bounds__(kTtmBlock) void k_ttm_fixup(int segl, int64_t nseg,
 // nothing takes no part (the reference's co-iteration of the contracted
 // level with U's rows skips it): it gets the fiber key of row `drop_i`, past
 // every root, so the sort moves it to the end, and is counted.
-template <bool kMask>
 __global__ __launch_bounds__(256) void k_ttm_direct_keys(int64_t nnz, const int32_t* __restrict__ leaf_fiber,
                                                          const int32_t* __restrict__ fiber_root,
                                                          const int32_t* __restrict__ l1_crd,
@@ -727,16 +723,14 @@ __global__ __launch_bounds__(256) void k_ttm_direct_keys(int64_t nnz, const int3
     uint64_t i = (uint32_t)l1_crd[fiber_root[f]];
     const uint64_t k = (uint32_t)l2_crd[f];
     const uint64_t j = (uint32_t)l3_crd[e];
-    if (kMask && umask[k] == 0) {
+    if (umask[k] == 0) {
       i = drop_i;
       ++nd;
     }
     keys[e] = (i << (bj + bk)) | (j << bk) | k;
   }
-  if (kMask) {
-    nd = wave_sum(nd);
-    if (lane_id() == 0 && nd) atomicAdd(dropped, nd);
-  }
+  nd = wave_sum(nd);
+  if (lane_id() == 0 && nd) atomicAdd(dropped, nd);
 }
 
 static int csf_owners(spws_ctx* ctx, const Csf3& x, int32_t** leaf_fiber, int32_t** fiber_root) {
@@ -816,7 +810,7 @@ static int mttkrp_run(spws_ctx* ctx, const Csf3& x, int32_t I, int32_t J, int32_
       int32_t *leaf_fiber, *fiber_root;
       if ((rc = csf_owners(ctx, x, &leaf_fiber, &fiber_root))) return rc;
       const unsigned g = (unsigned)std::min<int64_t>(div_up(x.nnz, 256), 65536);
-      SPWS_LAUNCH(ctx, "mttkrp_keys", k_mttkrp_keys<true>, dim3(g), dim3(256), 0, x.nnz, leaf_fiber, fiber_root,
+      SPWS_LAUNCH(ctx, "mttkrp_keys", k_mttkrp_keys, dim3(g), dim3(256), 0, x.nnz, leaf_fiber, fiber_root,
                   x.l1_crd, x.l2_crd, x.l3_crd, bj, bk, ctx->keys[0].as<uint64_t>(), mB, mC, (uint64_t)I, dropped);
       bool in_alt = false;
       if ((rc = radix_sort_pairs<uint64_t>(ctx, ctx->keys[0].as<uint64_t>(), ctx->vals[0].as<double>(),
@@ -998,7 +992,7 @@ static int ttm_run(spws_ctx* ctx, const Csf3& x, int32_t I, int32_t J, int32_t K
       if ((rc = ctx->obuf[6].ensure(256))) return rc;
       dropped = ctx->obuf[6].as<unsigned long long>();
       SPWS_HIP(hipMemsetAsync(dropped, 0, 8, s));
-      SPWS_LAUNCH(ctx, "ttm_keys", k_ttm_direct_keys<true>, dim3(g), dim3(256), 0, x.nnz, leaf_fiber, fiber_root,
+      SPWS_LAUNCH(ctx, "ttm_keys", k_ttm_direct_keys, dim3(g), dim3(256), 0, x.nnz, leaf_fiber, fiber_root,
                   x.l1_crd, x.l2_crd, x.l3_crd, bj, bk, ctx->keys[0].as<uint64_t>(), umask, (uint64_t)I, dropped);
       bool alt = false;
       if ((rc = radix_sort_pairs<uint64_t>(ctx, ctx->keys[0].as<uint64_t>(), ctx->vals[0].as<double>(),
