@@ -131,7 +131,8 @@ int spws_spgemm_rowwise_symbolic(spws_ctx* ctx, int32_t m, int32_t k, int32_t n,
  * A_vals hold them; B1_crd[b_nrows] / B2_pos / B2_crd / B_vals likewise for
  * B's stored rows (NULL = CSR).  A's columns and B's rows are co-iterated on
  * j.  Output: sorted CSR with int64 row pointers (nnz may exceed 2^31),
- * context-owned.  Each entry is summed over j in increasing order.
+ * context-owned.  Each entry is summed over j, in increasing order except by
+ * the methods that spws_ctx_set_outer_method says add in any order.
  * Replaces compute() of benchmark/DCSC_DCSR/DCSC_DCSR_coord_index_chase.h:194. */
 int spws_spgemm_outer(spws_ctx* ctx, int32_t m, int32_t k, int32_t n,
                       int32_t a_ncols, const int32_t* A1_crd, const int32_t* A2_pos, const int32_t* A2_crd,

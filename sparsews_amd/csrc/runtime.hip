@@ -148,7 +148,9 @@ void prof_collect(spws_ctx* ctx) {
 // and a rescan of each tile with its offset.
 //
 // Inputs of at most kScanSmall values take one launch: every workgroup sums
-// all the values before its tile itself.  PERF_SCAN
+// all the values before its tile itself.  65,536 32-bit values take 9.5 us so,
+// 65,537 in two launches 14.9 (events around each launch, some 4 us of each);
+// at the limit the last workgroup reads 240 KB before its own tile.
 
 constexpr int kScanBlock = 256;
 constexpr int kScanItems = 16;

@@ -1787,7 +1787,8 @@ constexpr int kFzNumWavesPerCu = 8;   // k_fz_rows<true>: bounded by the LDS win
 // within a row), one record per entry, the symbolic pass and its prefix
 // (exact row pointers, and an output allocated to the exact size), then the
 // numeric pass writing every entry in place.
-static int outer_fused(spws_ctx* ctx, const OuterArgs& a, int64_t En64, const int32_t* row_pairs, int s, bool ordered, bool off32, int64_t* nnz_out) {
+static int outer_fused(spws_ctx* ctx, const OuterArgs& a, int64_t En64, const int32_t* row_pairs, int s, bool ordered,
+                       bool off32, int64_t* nnz_out) {
   hipStream_t st = ctx->stream;
   int rc;
   const int32_t m = a.m;

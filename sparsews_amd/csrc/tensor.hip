@@ -192,14 +192,11 @@ constexpr int kAccSegMin = 32;
 // kMask: per row, the OR of its nonzeros' shared stored factor columns
 // (mB[j] & mC[k]) is or-ed into rmask[i], the row's stored output columns.
 template <int G, int S, bool kMask, bool kOff32>
-__global__ __launch_bounds__(kAccBlock, S == 1 && !kMask ? 8 : 4) void k_mttkrp_accum(int64_t nnz, int seg, const uint64_t* __restrict__ keys,
-                                                            const double* __restrict__ vals, int bj, int bk, int R,
-                                                            const double* __restrict__ Bf,
-                                                            const double* __restrict__ Cf, double* __restrict__ M,
-                                                            int32_t* __restrict__ present,
-                                                            const uint64_t* __restrict__ mB,
-                                                            const uint64_t* __restrict__ mC,
-                                                            unsigned long long* __restrict__ rmask) {
+__global__ __launch_bounds__(kAccBlock, S == 1 && !kMask ? 8 : 4) void k_mttkrp_accum(
+    int64_t nnz, int seg, const uint64_t* __restrict__ keys, const double* __restrict__ vals, int bj, int bk, int R,
+    const double* __restrict__ Bf, const double* __restrict__ Cf, double* __restrict__ M,
+    int32_t* __restrict__ present, const uint64_t* __restrict__ mB, const uint64_t* __restrict__ mC,
+    unsigned long long* __restrict__ rmask) {
   constexpr int NG = kAccBlock / G;
   // a nonzero as the walk reads it: its factor rows' byte offsets (kOff32:
   // both factors below 4 GiB) or its j and k, its value, and its row with

@@ -18,8 +18,8 @@ from helpers import powerlaw_rows, random_csr, uniform_rows
 from sparsews_amd import formats, gen
 from sparsews_amd._lib import check as capi_check
 from sparsews_amd._lib import lib
-from sparsews_amd.device import (Context, DeviceArray, DeviceCSR, DeviceCSR64, DeviceDCSR, csr64_transpose, csr_transpose,
-                                 set_outer_chunking, set_outer_method, spgemm_outer)
+from sparsews_amd.device import (Context, DeviceArray, DeviceCSR, DeviceCSR64, DeviceDCSR, csr64_transpose,
+                                 csr_transpose, set_outer_chunking, set_outer_method, spgemm_outer)
 from sparsews_amd.gen import CSR
 
 pytestmark = pytest.mark.gpu
@@ -668,7 +668,8 @@ def test_transpose_common_columns(ctx, share):
     np.testing.assert_array_equal(T.vals, A.vals[order])
 
 
-@pytest.mark.parametrize("n", [1, 3, 4, 4095, 4096, 4097, 8193, 16_384, 16_385, 20_483, 65_535, 65_536, 65_537, 200_001])
+@pytest.mark.parametrize("n", [1, 3, 4, 4095, 4096, 4097, 8193, 16_384, 16_385, 20_483, 65_535, 65_536, 65_537,
+                               200_001])
 def test_transpose_row_pointers(ctx, n):
     """Row pointers of a transpose into n rows, most of them empty at the
     larger n: each is the first sorted column that is not before it."""
