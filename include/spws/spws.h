@@ -163,8 +163,9 @@ int spws_ctx_set_outer_chunking(spws_ctx* ctx, int64_t max_products, int32_t max
  *   0  automatic: 4 unless the windows would be too sparse or too many; then
  *      by rows (A's columns transposed into rows, then the row-wise product;
  *      outputs of at most 2^17 columns and 2^30 products, no row of more
- *      than 16,384 products and a 128th of all, memory permitting; reported
- *      as method 5, sums in any order as 4), else 1.
+ *      than 16,384 products and a 128th of all, an A whose entries mostly
+ *      meet a row of B, memory permitting; reported as method 5, sums in any
+ *      order as 4), else 1.
  * window_log2 sets the column window of methods 2-4 (6..11; 0 = chosen
  * from the average products per row).  Methods 1-3 sum each entry in
  * increasing j and give identical results. */

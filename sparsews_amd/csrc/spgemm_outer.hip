@@ -1922,6 +1922,15 @@ constexpr int32_t kOuterRowsCols = 1 << 17;  // columns at most (the row kernels
 // and 2,850, L = 1.28M 5,074 and 3,169.
 static int64_t outer_rows_longest(int64_t products) { return 16384 + products / 128; }
 
+// A's entries at most: by rows all of them are transposed and looked at (40 to
+// 90 ns a thousand), the sort sees only those that meet a row of B but brings
+// the rows' products to the host (3 ns a row).  Rows m, entries of A and
+// products, by rows and by the sort: 2,000, 0.1M and 3k 194 us and 208, with
+// 1M and 30k 266 and 230, with 10M and 0.3M 1,057 and 230; 100,000, 4M and
+// 0.12M 369 and 501, with 10M and 0.3M 610 and 500, with 10M and 5M 1,068 and
+// 1,129, with 20M and 6M 1,251 and 893.
+static int64_t outer_rows_entries(int64_t products, int32_t m) { return products + (1 << 19) + 50 * (int64_t)m; }
+
 static int outer_rows(spws_ctx* ctx, const OuterArgs& a, int64_t a_nnz, int64_t* nnz_out) {
   int rc;
   const size_t nn = (size_t)(a_nnz > 0 ? a_nnz : 1);
@@ -2021,13 +2030,14 @@ static int outer_run(spws_ctx* ctx, const OuterArgs& a, int64_t* nnz_out, int on
     method = (per_bucket >= 64.0 && W <= 4096 && max_pairs * W <= ((int64_t)1 << 28)) ? fused : 1;
     // Too few products per window: by rows, where the order of the sums may
     // change, the row kernels' column bitmap covers the output, no row
-    // outweighs the others (outer_rows_longest) and the slots and the output,
-    // 24 bytes a product, take no more than the sort of one whole chunk.  2,000 rows of 8 squared
+    // outweighs the others (outer_rows_longest), A is not mostly without a
+    // match in B (outer_rows_entries) and the slots and the output, 24 bytes a
+    // product, take no more than the sort of one whole chunk.  2,000 rows of 8 squared
     // (128k products): 231 us by the sort, 152 by rows; 30,000 rows of 2..32
     // (8.7M products): 663 and 357; 100,000 of 60 (360M): 20,634 and 3,116.
     if (method == 1 && !ctx->outer_auto_ordered && ctx->outer_max_products == 0 && ctx->outer_max_rows == 0 &&
         a.n <= kOuterRowsCols && products <= max_products && hs[kOsMaxProducts] <= outer_rows_longest(products) &&
-        ctx->rw.force_path < 0 && m > 0 && a.a_ncols > 0 && a.b_nrows > 0 && a.b_nrows < INT32_MAX - 1)
+        a_nnz <= outer_rows_entries(products, m) && ctx->rw.force_path < 0 && m > 0 && a.a_ncols > 0 && a.b_nrows > 0 && a.b_nrows < INT32_MAX - 1)
       method = 5;
   }
   if (method == 5) {

@@ -307,6 +307,23 @@ def test_outer_by_rows_longest_row(ctx, longest, method):
     check(C, A, B, exact_order=method == 1)
 
 
+@pytest.mark.parametrize("entries,method", [(525_388, 5), (525_389, 1)])
+def test_outer_by_rows_unmatched_entries(ctx, entries, method):
+    """A of as many entries as products (600), rows times 50 (500) and 2^19
+    goes by rows; one more that meets no row of B and the sort takes it."""
+    print(f"case: outer by rows, {entries} entries of A", flush=True)
+    m, k, n = 10, 60_000, 50_000
+    lengths = np.full(m, entries // m)
+    lengths[-1] += entries % m
+    pos = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    crd = np.concatenate([np.arange(c) for c in lengths]).astype(np.int32)
+    A = CSR(m, k, pos, crd, np.random.default_rng(97).uniform(-1, 1, entries))
+    B = random_csr(k, n, np.where(np.arange(k) % 2000 == 7, 3, 0) * (np.arange(k) < 40_000), 97, 1)
+    C = run_outer(ctx, A, B)
+    assert ctx.stats()["products"] == 600 and ctx.stats()["outer_method"] == method
+    check(C, A, B, exact_order=method == 1)
+
+
 def test_outer_by_rows_falls_back_to_the_sort():
     """By rows a product takes 24 bytes of slots and output per product at
     once; beside a working set that leaves no room for them the automatic
