@@ -3,6 +3,8 @@
 Structure (output rows / fibers) must be bit-exact; values within
 |x - y| <= 1e-12 * max(|y|, sum|terms|).
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -278,6 +280,36 @@ def test_ttm_segments_of_64(ctx):
     V = X.vals.reshape(-1, 300)
     exact = (V.astype(np.longdouble) @ U.astype(np.longdouble)).astype(np.float64)
     assert oracle.max_value_error(Y.ravel(), exact.ravel(), (np.abs(V) @ np.abs(U)).ravel()) <= TOL
+
+
+def test_ttm_time_of_a_long_fiber(ctx):
+    """One fiber of 300,000 nonzeros by sorting: its parts are added one after
+    another, but not one slice of 16 ranks after another (four slices then
+    take 3.2 times as long as one)."""
+    print("case: ttm time of a long fiber", flush=True)
+    K = 300_000
+    X = gen.COO3((1, 1, K), np.stack([np.zeros(K), np.zeros(K), np.arange(K)], axis=1).astype(np.int32),
+                 np.random.default_rng(9).uniform(-1, 1, K))
+    dX = DeviceCSF.upload(ctx, formats.csf3_from_coo(X, (0, 2, 1)))
+    times = []
+    try:
+        set_ttm_method(ctx, 1)
+        for R in (16, 64):
+            U = np.random.default_rng(R).uniform(-1, 1, (K, R))
+            dU = DeviceArray.from_host(ctx, U.ravel())
+            took = []
+            for _ in range(6):
+                ctx.sync()
+                t = time.perf_counter()
+                Y = ttm(ctx, dX, 1, 1, K, R, dU)[2]
+                ctx.sync()
+                took.append(time.perf_counter() - t)
+            times.append(min(took[1:]))
+            assert oracle.max_value_error(Y.to_host(), X.vals @ U, np.abs(X.vals) @ np.abs(U)) <= TOL
+    finally:
+        set_ttm_method(ctx, 0)
+    print(f"R = 16 {times[0] * 1e6:.0f} us, R = 64 {times[1] * 1e6:.0f} us", flush=True)
+    assert times[1] <= 2 * times[0]
 
 
 @pytest.mark.parametrize("method", [0, 1])
