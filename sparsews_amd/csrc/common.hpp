@@ -277,6 +277,10 @@ __device__ __forceinline__ T wave_sum(T v) {
   return wave_last(wave_incl_scan(v));
 }
 
+__device__ __forceinline__ uint64_t wave_or(uint64_t v) {
+  return wave_last(wave_incl_scan_op(v, (uint64_t)0, [](uint64_t a, uint64_t b) { return a | b; }));
+}
+
 // v of lane (lane ^ D) without LDS: DPP quad permutes, half-row and row
 // mirrors and the row rotate by 8, and gfx950's 16- and 32-lane swaps
 // (each swap returns both halves exchanged; the lane keeps the half that

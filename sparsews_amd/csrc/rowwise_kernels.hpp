@@ -1235,14 +1235,18 @@ __global__ __launch_bounds__(BLOCK) void k_row_bitmap(const int32_t* __restrict_
 //
 // Pass 1 lists the non-empty A entries in LDS (up to ecap at a time, in the
 // accumulators' place) with their products' prefix, and deals the products out
-// evenly over the threads, each finding its entry by a binary search: with
-// the entries dealt out instead, the wavefront that gets a B row of 4,096
-// entries works alone while fifteen wait.  20k power-law rows, 108 of them
-// long: 117 -> 102 us, as long as the longest row takes.  (All workgroups on all
+// evenly over the threads: with the entries dealt out instead, the wavefront
+// that gets a B row of 4,096 entries works alone while fifteen wait.  20k
+// power-law rows, 108 of them long: 117 -> 102 us, as long as the longest row
+// takes.  A wavefront finds the entries of 64 neighbouring products together,
+// with four LDS reads; a binary search by every thread took 12 one after
+// another: 102 -> 75 us, and the first pass of one row of 9M products 11.5 ms
+// (7.2 with the entries dealt out, as much now).  (All workgroups on all
 // rows, with FP64 atomics into dense rows in HBM: 135 us, about 20 G scattered
 // atomics a second.)
 constexpr int kLongItems = 8;      // products per thread in flight
 constexpr int kLongEntries = 4096; // A entries listed at a time at most
+static_assert(kLongEntries <= kWave * kWave, "64 probes twice find an entry");
 // accumulators the kernel's LDS holds at least (16 bytes per listed entry)
 constexpr int32_t kLongAccMin = 2 * kBitmapLongBlock;
 
@@ -1259,6 +1263,7 @@ __global__ __launch_bounds__(BLOCK) void k_row_bitmap_staged(
   __shared__ int64_t sh64[BLOCK / kWave + 1];
   BitmapLds L;
   L.init<BLOCK>(bml_d, ncols);  // ends with a barrier
+  const int lane = lane_id();
   const int32_t count = bmeta[kMetaCount + path];
   const int32_t* rows = bin_rows + bmeta[kMetaOff + path];
   // listed entries: values, then first products, then B row start - first
@@ -1311,21 +1316,24 @@ __global__ __launch_bounds__(BLOCK) void k_row_bitmap_staged(
               }
             __syncthreads();
             const int32_t listed = (int32_t)(all >> 40), total = (int32_t)(all & (((int64_t)1 << 40) - 1));
-            int top = 1;  // a power of two, at least `listed`
-            while (top < listed) top <<= 1;
+            const int32_t coarse = lane * kWave < listed ? efirst[lane * kWave] : INT_MAX;
             for (int32_t q0 = 0; q0 < total; q0 += BLOCK * kLongItems) {
               int32_t col[kLongItems], own[kLongItems];
               double bv[kLongItems];
+              // the last entry whose first product is at most the product: of
+              // the wavefront's first product by 64 probes twice, of the others
+              // by the entries that start after it
 #pragma unroll
-              for (int u = 0; u < kLongItems; ++u) own[u] = 0;
-              // the last entry whose first product is at most the product
-              for (int d = top >> 1; d > 0; d >>= 1) {
-#pragma unroll
-                for (int u = 0; u < kLongItems; ++u) {
-                  const int32_t q = q0 + u * BLOCK + (int32_t)threadIdx.x;
-                  const int32_t mid = own[u] + d;
-                  if (mid < listed && efirst[mid] <= q) own[u] = mid;
-                }
+              for (int u = 0; u < kLongItems; ++u) {
+                const int32_t p0 = __builtin_amdgcn_readfirstlane(q0 + u * BLOCK + (int32_t)threadIdx.x - lane);
+                const int32_t block = (kWave - 1 - __builtin_clzll(__ballot(coarse <= p0))) * kWave;
+                const int32_t f = block + lane < listed ? efirst[block + lane] : INT_MAX;
+                const int32_t first_own = block + (int32_t)__popcll(__ballot(f <= p0)) - 1;
+                const int32_t next = first_own + 1 + lane;
+                const uint32_t d = (uint32_t)((next < listed ? efirst[next] : INT_MAX) - p0);  // at least 1
+                const uint64_t starts = wave_or(d < (uint32_t)kWave ? 1ull << d : 0ull) >> 1;
+                own[u] = first_own + (int32_t)__builtin_amdgcn_mbcnt_hi(
+                                         (uint32_t)(starts >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)starts, 0));
               }
 #pragma unroll
               for (int u = 0; u < kLongItems; ++u) {
