@@ -38,9 +38,11 @@ __host__ __device__ __forceinline__ int classify_row(int64_t ub, int32_t ncols, 
 
 // Bin metadata on the device (int32 bmeta): [0, 8) rows per path, [8, 16)
 // offset of each path's rows in bin_rows, [16, 24) scatter cursors; maxub
-// (uint64): [0, 8) largest row upper bound per path, [8] sum of all upper
-// bounds.
+// (uint64): [0, 7) largest row upper bound per path, [kMetaEntries] A's
+// entries, [8] sum of all upper bounds.
 constexpr int kMetaCount = 0, kMetaOff = 8, kMetaCursor = 16, kMetaInts = 24;
+constexpr int kMetaEntries = 7;
+static_assert(kMetaEntries >= kPaths, "not a path's");
 
 __device__ __forceinline__ int32_t dev_or(const int32_t* p, int32_t v) { return p ? *p : v; }
 
@@ -122,6 +124,7 @@ __global__ __launch_bounds__(kRsBlock) void k_rowstat(int32_t m_host, const int3
   }
   tot = wave_sum(tot);
   if (lane_id() == 0 && tot) atomicAdd(&maxub[8], tot);
+  if (blockIdx.x == 0 && t == 0 && m > 0) maxub[kMetaEntries] = (unsigned long long)(Ap[m] - Ap[0]);
   __syncthreads();
   if (t < kPaths && cnt[t]) {
     atomicAdd(&bmeta[kMetaCount + t], cnt[t]);
@@ -187,13 +190,13 @@ __global__ __launch_bounds__(kRsBlock) void k_binscatter(int32_t m_host, const i
 // loads one A entry (j, a) and len(B_j); an inclusive wave scan gives the
 // product offsets, and each lane then finds, for its product index q, the
 // owning A entry by a binary search over the lanes' offsets (six
-// ds_bpermute rounds).  Rows with fewer than two chunks of A entries per
+// ds_bpermute rounds).  Rows with fewer than kOwn chunks of A entries per
 // wavefront: every wavefront scans the same chunk and takes its own strides
 // of the chunk's products, so rows with few A entries but long B rows still
 // use all wavefronts.  Longer rows: each wavefront takes whole chunks.  Loop
 // bounds are wave-uniform, so the shuffles see every lane.
 
-template <bool kValues, int kU = 4, class F>
+template <bool kValues, int kU = 4, int kOwn = 2, class F>
 __device__ __forceinline__ void expand_products(int32_t a_beg, int32_t a_end, int32_t widx, int32_t nwaves,
                                                 const int32_t* __restrict__ Ai, const double* __restrict__ Ax,
                                                 const int32_t* __restrict__ Bp, const int32_t* __restrict__ Bi,
@@ -201,10 +204,10 @@ __device__ __forceinline__ void expand_products(int32_t a_beg, int32_t a_end, in
   // kU strides of products are located and loaded before any is inserted,
   // so their B loads are in flight together
   const int lane = lane_id();
-  // rows of at least two chunks per wavefront: each wavefront takes whole
+  // rows of at least kOwn chunks per wavefront: each wavefront takes whole
   // chunks of its own (chunk widx, widx + nwaves, ...), so the chunks' load
   // chains run side by side instead of one after another
-  const bool own_chunks = a_end - a_beg >= 2 * kWave * nwaves;
+  const bool own_chunks = a_end - a_beg >= kOwn * kWave * nwaves;
   const int32_t c_first = own_chunks ? a_beg + widx * kWave : a_beg;
   const int32_t c_step = own_chunks ? nwaves * kWave : kWave;
   if (own_chunks) {
@@ -1388,9 +1391,12 @@ __global__ __launch_bounds__(BLOCK) void k_row_bitmap_staged(
 // While a row is worked on, the loads of the next ones are in flight, each
 // level of the chain row list -> row pointers -> A entries -> B row bounds ->
 // B entries one row further ahead, so a row costs its own work and not five
-// memory latencies.  A row of more than kBitsEntries A entries or
+// memory latencies.  A row of more than bits_entries A entries or
 // BLOCK * ITEMS products takes the plain expansion instead, one product per
-// lane at a time (more in flight there would cost every row its registers).
+// lane at a time (more in flight there would cost every row its registers, or
+// leave wavefronts without products) and, from one chunk of A entries per
+// wavefront on, every wavefront its own chunks: 5,000 rows of 1,000 entries, 3
+// products each, 730 us with all wavefronts on the same chunk, 420 so.
 //
 // A wavefront finds the A entry of each of its products with a max-scan over
 // marks at the entries' first products (12 instructions per 64 products; a
@@ -1410,7 +1416,14 @@ constexpr int kBits2Block = 256, kBits2Items = 8;
 // entries 775 and 767).
 constexpr int kBits3Block = 512, kBits3Items = 8;
 constexpr int32_t kBits2Products = kBits2Block * kBits2Items;
-constexpr int kBitsEntries = 256;
+// A row's A entries at most, 64 of them at a time: 20,000 rows of 300 entries
+// and 3,600 products take 1,105 us in the plain expansion and 567 from
+// registers.  The count goes through its products once, not twice: of 300
+// entries with one product each 61 us and 76, with twelve each 210 and 192.  In
+// the first bin positions of 16 bits take the sixth wavefront per SIMD (65,536
+// rows of 2..64 entries 748 us, 793 with them).
+constexpr int bits_entries(bool values, int items) { return values && items > 4 ? 512 : 256; }
+constexpr int bits_pos_per_word(int items) { return items > 4 ? 2 : 4; }  // positions of A entries in 32 bits
 constexpr int32_t kBitsNarrow = 1 << 16;  // row widths whose columns are staged in 16 bits
 
 // LDS of a row: its bitmap in vectors of 128 columns, then (values) vcap
@@ -1431,7 +1444,7 @@ struct RowAhead {
 
 // Items of the row in `r` (bounds of its first 64 entries loaded) for this
 // wavefront: columns (-1: none), B values and the positions of their A entries
-// in the row (a byte each), the loads left in flight.  `marks` is the
+// in the row (8 or 16 bits each), the loads left in flight.  `marks` is the
 // wavefront's own area of 64 * ITEMS bytes, zero on entry and on return.
 // Returns the row's products, or -1 when the row does not fit.
 template <int BLOCK, int ITEMS, bool kValues>
@@ -1439,17 +1452,18 @@ __device__ __forceinline__ int32_t gather_marked(const RowAhead& r, uint8_t* __r
                                                  const int32_t* __restrict__ Ai, const int32_t* __restrict__ Bp,
                                                  const int32_t* __restrict__ Bi, const double* __restrict__ Bx,
                                                  int32_t (&col)[ITEMS], double (&bv)[ITEMS],
-                                                 uint32_t (&own)[(ITEMS + 3) / 4]) {
+                                                 uint32_t (&own)[ITEMS / bits_pos_per_word(ITEMS)]) {
   constexpr int kWaves = BLOCK / kWave;
-  static_assert(kBitsEntries <= 256, "positions of A entries in a byte");
+  constexpr int kPos = bits_pos_per_word(ITEMS);
+  static_assert(bits_entries(kValues, ITEMS) <= 1 << (32 / kPos), "positions of A entries");
   const int lane = lane_id();
   const int w = threadIdx.x / kWave;
 #pragma unroll
   for (int u = 0; u < ITEMS; ++u) col[u] = -1;
 #pragma unroll
-  for (int u = 0; u < (ITEMS + 3) / 4; ++u) own[u] = 0;
+  for (int u = 0; u < ITEMS / kPos; ++u) own[u] = 0;
   const int32_t na = r.a_end - r.a_beg;
-  if (na > kBitsEntries) return -1;
+  if (na > bits_entries(kValues, ITEMS)) return -1;
   int32_t bstart = r.bstart, blen = r.blen, base = 0;
   for (int32_t c = 0; c < na; c += kWave) {
     if (c > 0) {
@@ -1482,7 +1496,7 @@ __device__ __forceinline__ int32_t gather_marked(const RowAhead& r, uint8_t* __r
         col[u] = Bi[kb];
         if (kValues) {
           bv[u] = Bx[kb];
-          own[u / 4] |= (uint32_t)(c + at) << (8 * (u % 4));
+          own[u / kPos] |= (uint32_t)(c + at) << (32 / kPos * (u % kPos));
         }
       }
     }
@@ -1600,7 +1614,8 @@ __global__ __launch_bounds__(BLOCK, !kValues ? 7 : ITEMS <= 4 ? 5 : 4) void k_ro
   entries(x1);
   int32_t col[ITEMS];
   double bv[ITEMS];
-  uint32_t own[(ITEMS + 3) / 4];
+  constexpr int kPos = bits_pos_per_word(ITEMS);
+  uint32_t own[ITEMS / kPos];
   int32_t total = gather_marked<BLOCK, ITEMS, kValues>(x0, s_marks[w], Ai, Bp, Bi, Bx, col, bv, own);
   int parity = 0;
   for (; x0.i >= 0; parity ^= 1) {
@@ -1624,7 +1639,7 @@ __global__ __launch_bounds__(BLOCK, !kValues ? 7 : ITEMS <= 4 ? 5 : 4) void k_ro
         for (int u = 0; u < ITEMS; ++u)
           if (col[u] >= 0) fresh += set(col[u]) ? 1 : 0;
       } else {
-        expand_products<false, 1>(a_beg, a_end, w, kWaves, Ai, Ax, Bp, Bi, Bx,
+        expand_products<false, 1, 1>(a_beg, a_end, w, kWaves, Ai, Ax, Bp, Bi, Bx,
                                   [&](int32_t c, double) { fresh += set(c) ? 1 : 0; });
       }
       fresh = wave_sum(fresh);
@@ -1656,7 +1671,7 @@ __global__ __launch_bounds__(BLOCK, !kValues ? 7 : ITEMS <= 4 ? 5 : 4) void k_ro
             atomicOr(&bm[cc >> 5], 1u << (cc & 31));
           }
       } else {
-        expand_products<false, 1>(a_beg, a_end, w, kWaves, Ai, Ax, Bp, Bi, Bx, [&](int32_t c, double) {
+        expand_products<false, 1, 1>(a_beg, a_end, w, kWaves, Ai, Ax, Bp, Bi, Bx, [&](int32_t c, double) {
           const uint32_t cc = (uint32_t)(c - cb);
           atomicOr(&bm[cc >> 5], 1u << (cc & 31));
         });
@@ -1700,12 +1715,12 @@ __global__ __launch_bounds__(BLOCK, !kValues ? 7 : ITEMS <= 4 ? 5 : 4) void k_ro
         double av[ITEMS];
 #pragma unroll
         for (int u = 0; u < ITEMS; ++u)
-          if (col[u] >= 0) av[u] = Ax[a_beg + (int32_t)((own[u / 4] >> (8 * (u % 4))) & 0xFFu)];
+          if (col[u] >= 0) av[u] = Ax[a_beg + (int32_t)((own[u / kPos] >> (32 / kPos * (u % kPos))) & (0xFFFFFFFFu >> (32 - 32 / kPos)))];
 #pragma unroll
         for (int u = 0; u < ITEMS; ++u)
           if (col[u] >= 0) add(col[u], av[u] * bv[u]);
       } else {
-        expand_products<true, 1>(a_beg, a_end, w, kWaves, Ai, Ax, Bp, Bi, Bx, add);
+        expand_products<true, 1, 1>(a_beg, a_end, w, kWaves, Ai, Ax, Bp, Bi, Bx, add);
       }
       if (t == 0) row_nnz[i] = nnz;
       total = gather_marked<BLOCK, ITEMS, kValues>(x1, s_marks[w], Ai, Bp, Bi, Bx, col, bv, own);

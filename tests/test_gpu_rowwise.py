@@ -318,7 +318,9 @@ def test_prefix_sum_lengths(ctx, m):
 ROW_KINDS = [
     (30, 0),    # 1,350 products, the bulk: second block bin, from registers
     (20, 236),  # 256 A entries: four chunks, from registers
-    (20, 256),  # 276 A entries: plain expansion
+    (20, 256),  # 276 A entries: from registers, counted by the plain expansion
+    (20, 492), (10, 503), (0, 512),  # 512 A entries: from registers
+    (20, 493), (10, 504), (0, 513),  # 513: plain expansion, a chunk per wavefront
     (45, 0),    # 2,025 products: the registers' edge
     (50, 0),    # 2,250 products: plain expansion
     (10, 0), (1, 255), (0, 257), (1, 256),  # first block bin, both ways
