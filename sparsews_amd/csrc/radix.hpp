@@ -77,19 +77,32 @@ inline int radix_passes(int bits) { return (bits + kSortDigitMax - 1) / kSortDig
 
 // ------------------------------------------------------------ segment owners
 
-// The last s in [0, n) with pos[s] <= x (pos[0] <= x, pos nondecreasing), by
-// the whole wavefront: 64 probes a round.
+// s[e] = the last s in [0, n) with pos[s] <= x[e] (pos[0] <= x[e], pos
+// nondecreasing), by the whole wavefront: 64 probes a round for each, the same
+// ones as long as both lie between the same two.
 template <class PosT>
-__device__ __forceinline__ int32_t last_at_or_before(const PosT* __restrict__ pos, int32_t n, int64_t x) {
-  int32_t lo = 0, hi = n;
-  while (hi - lo > 1) {
-    const int32_t step = (hi - lo + kWave - 1) / kWave;
-    const int64_t at = lo + (int64_t)lane_id() * step;
-    const uint64_t ok = __ballot(at < hi && (int64_t)pos[at] <= x);
-    lo += (kWave - 1 - __builtin_clzll(ok)) * step;  // lane 0 always holds
-    hi = min(hi, lo + step);
+__device__ __forceinline__ void last_at_or_before(const PosT* __restrict__ pos, int32_t n, const int64_t (&x)[2],
+                                                  int32_t (&s)[2]) {
+  int32_t lo[2] = {0, 0}, hi[2] = {n, n};
+  while (max(hi[0] - lo[0], hi[1] - lo[1]) > 1) {
+    PosT v[2];
+    int32_t step[2];
+    const bool same = lo[0] == lo[1] && hi[0] == hi[1];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      step[e] = (hi[e] - lo[e] + kWave - 1) / kWave;
+      const int64_t at = lo[e] + (int64_t)lane_id() * step[e];
+      v[e] = v[0];
+      if (e == 0 || !same) v[e] = at < hi[e] ? pos[at] : std::numeric_limits<PosT>::max();
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      lo[e] += (kWave - 1 - __builtin_clzll(__ballot((int64_t)v[e] <= x[e]))) * step[e];  // lane 0 always holds
+      hi[e] = min(hi[e], lo[e] + step[e]);
+    }
   }
-  return lo;
+  s[0] = lo[0];
+  s[1] = lo[1];
 }
 
 // owner[r] = the segment s with pos[s] <= e < pos[s + 1] of item
@@ -102,9 +115,11 @@ __device__ __forceinline__ int32_t last_at_or_before(const PosT* __restrict__ po
 // The marks cost the tile a look at every segment that starts in it, empty
 // ones too, BLOCK at a time, about 0.2 us each time.  A tile of more than
 // eight times as many segments as items searches each item's segment instead:
-// 100k entries transposed with 6M empty rows between two of them take 90 us so
+// 100k entries transposed with 6M empty rows between two of them take 89 us so
 // and 9,660 walked; with 900k rows spread between them (ten segments an item)
-// 94 searched and 95 walked, with 300k 97 and 71.
+// 88 searched and 95 walked, with 300k 97 and 67.  The search for the first
+// item's segment finds the last one's with it: looked up after it, the number
+// of segments cost a call 2 to 6 us.
 constexpr int kOwnerWalk = 8;    // segments walked per item of a tile at most
 constexpr int kOwnerSearch = 8;  // items searched together
 template <int BLOCK, int ITEMS, class PosT>
@@ -115,11 +130,13 @@ __device__ __forceinline__ void tile_owners(const PosT* __restrict__ pos, int32_
   __shared__ uint32_t top[kWaves];
   const int lane = lane_id();
   const int w = threadIdx.x / kWave;
-  const int32_t s0 = last_at_or_before(pos, nseg, base);
-  constexpr int32_t kMost = kOwnerWalk * BLOCK * ITEMS;
-  if (nseg - s0 > kMost && (int64_t)pos[s0 + kMost] < end) {  // uniform
+  int32_t edge[2];  // the first and the last item's segments
+  last_at_or_before(pos, nseg, {base, end - 1}, edge);
+  const int32_t s0 = edge[0];
+  const uint32_t span = (uint32_t)(edge[1] - s0);
+  if (span >= (uint32_t)(kOwnerWalk * BLOCK * ITEMS)) {  // uniform
     uint32_t top_step = 1;
-    while (top_step < (uint32_t)(nseg - s0)) top_step <<= 1;
+    while (top_step <= span >> 1) top_step <<= 1;
 #pragma unroll
     for (int q = 0; q < ITEMS; q += kOwnerSearch) {
 #pragma unroll
@@ -129,7 +146,7 @@ __device__ __forceinline__ void tile_owners(const PosT* __restrict__ pos, int32_
         for (int r = q; r < q + kOwnerSearch; ++r) {
           const int64_t e = min(base + (w * ITEMS + r) * kWave + lane, end - 1);
           const uint32_t s = (uint32_t)owner[r] + step;
-          if (s < (uint32_t)nseg && (int64_t)pos[s] <= e) owner[r] = (int32_t)s;
+          if (s <= (uint32_t)edge[1] && (int64_t)pos[s] <= e) owner[r] = (int32_t)s;
         }
       }
     }
@@ -137,10 +154,9 @@ __device__ __forceinline__ void tile_owners(const PosT* __restrict__ pos, int32_
   }
   for (int e = threadIdx.x; e < BLOCK * ITEMS; e += BLOCK) marks[e] = 0;
   __syncthreads();
-  for (int32_t s = s0 + (int32_t)threadIdx.x; s < nseg; s += BLOCK) {
-    const int64_t p = (int64_t)pos[s];
-    if (p >= end) break;
-    if ((int64_t)pos[s + 1] > p) marks[p > base ? p - base : 0] = (uint32_t)(s - s0) + 1;
+  for (uint32_t s = threadIdx.x; s <= span; s += BLOCK) {
+    const int64_t p = (int64_t)pos[s0 + s];
+    if ((int64_t)pos[s0 + s + 1] > p) marks[p > base ? p - base : 0] = s + 1;
   }
   __syncthreads();
   uint32_t m[ITEMS];
