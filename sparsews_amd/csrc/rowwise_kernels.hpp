@@ -1715,7 +1715,10 @@ __global__ __launch_bounds__(BLOCK, !kValues ? 7 : ITEMS <= 4 ? 5 : 4) void k_ro
         double av[ITEMS];
 #pragma unroll
         for (int u = 0; u < ITEMS; ++u)
-          if (col[u] >= 0) av[u] = Ax[a_beg + (int32_t)((own[u / kPos] >> (32 / kPos * (u % kPos))) & (0xFFFFFFFFu >> (32 - 32 / kPos)))];
+          if (col[u] >= 0) {
+            constexpr uint32_t kPosMask = 0xFFFFFFFFu >> (32 - 32 / kPos);
+            av[u] = Ax[a_beg + (int32_t)((own[u / kPos] >> (32 / kPos * (u % kPos))) & kPosMask)];
+          }
 #pragma unroll
         for (int u = 0; u < ITEMS; ++u)
           if (col[u] >= 0) add(col[u], av[u] * bv[u]);
