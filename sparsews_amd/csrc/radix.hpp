@@ -119,7 +119,7 @@ __device__ __forceinline__ void last_at_or_before(const PosT* __restrict__ pos, 
 // and 9,660 walked; with 900k rows spread between them (ten segments an item)
 // 88 searched and 95 walked, with 300k 97 and 67.  The search for the first
 // item's segment finds the last one's with it: looked up after it, the number
-// of segments cost a call 2 to 6 us.
+// of segments cost small calls up to 6 us.
 constexpr int kOwnerWalk = 8;    // segments walked per item of a tile at most
 constexpr int kOwnerSearch = 8;  // items searched together
 template <int BLOCK, int ITEMS, class PosT>
@@ -287,64 +287,10 @@ __global__ __launch_bounds__(kSortBlock) void k_radix_hist(Source in, int64_t n,
 constexpr int kSortDirect = 64;
 inline int64_t radix_chunk_tiles(int64_t ntiles) { return ntiles <= kSortChunkOnly ? ntiles : kSortChunk; }
 
-// hist's rows [c per, (c + 1) per) in place to their exclusive prefixes, their
-// sum to row c of chunk; a digit per thread.
-[[maybe_unused]] static __global__ __launch_bounds__(kSortBlock) void k_radix_chunks(
-    int32_t* __restrict__ hist, int64_t ntiles, int64_t per, int nb, int32_t* __restrict__ chunk) {
-  const int d = blockIdx.y * kSortBlock + threadIdx.x;
-  if (d >= nb) return;
-  const int64_t t0 = (int64_t)blockIdx.x * per;
-  const int64_t t1 = t0 + per < ntiles ? t0 + per : ntiles;
-  int32_t run = 0;
-  for (int64_t t = t0; t < t1; t += kSortChunk) {
-    int32_t c[kSortChunk];
-#pragma unroll
-    for (int q = 0; q < kSortChunk; ++q) c[q] = t + q < t1 ? hist[(t + q) * nb + d] : 0;
-#pragma unroll
-    for (int q = 0; q < kSortChunk; ++q) {
-      if (t + q < t1) hist[(t + q) * nb + d] = run;
-      run += c[q];
-    }
-  }
-  chunk[(int64_t)blockIdx.x * nb + d] = run;
-}
-
-// The chunks' rows to their exclusive prefixes, the digits' totals to row n:
-// 64 digits per workgroup, the rows split over its wavefronts.
-constexpr int kSortDigitsBlock = 1024;
-[[maybe_unused]] static __global__ __launch_bounds__(kSortDigitsBlock) void k_radix_digits(
-    int32_t* __restrict__ chunk, int64_t n, int nb) {
-  constexpr int kWaves = kSortDigitsBlock / kWave;
-  __shared__ int32_t part[kWaves][kWave];
-  const int lane = lane_id();
-  const int w = threadIdx.x / kWave;
-  const int d = blockIdx.x * kWave + lane;
-  const int64_t per = (n + kWaves - 1) / kWaves;
-  const int64_t c0 = w * per < n ? w * per : n;
-  const int64_t c1 = c0 + per < n ? c0 + per : n;
-  int32_t sum = 0;
-  if (d < nb) {
-#pragma unroll 8
-    for (int64_t c = c0; c < c1; ++c) sum += chunk[c * nb + d];
-  }
-  part[w][lane] = sum;
-  __syncthreads();
-  int32_t run = 0, all = 0;
-#pragma unroll
-  for (int q = 0; q < kWaves; ++q) {
-    const int32_t v = part[q][lane];
-    run += q < w ? v : 0;
-    all += v;
-  }
-  if (d >= nb) return;
-#pragma unroll 8
-  for (int64_t c = c0; c < c1; ++c) {
-    const int32_t v = chunk[c * nb + d];
-    chunk[c * nb + d] = run;
-    run += v;
-  }
-  if (w == 0) chunk[n * nb + d] = all;
-}
+// hist's rows of nb counts, one per tile, in place to what the earlier tiles of
+// their chunk hold, and the chunks' rows in chunk likewise, with the totals
+// behind them (a single chunk's row is the totals).
+int radix_offsets(spws_ctx* ctx, int32_t* hist, int64_t ntiles, int nb, int32_t* chunk);
 
 template <class K, class Source, class Sink>
 __global__ __launch_bounds__(kSortBlock, 4) void k_radix_scatter(Source in, Sink out, int64_t n, int shift,
@@ -528,12 +474,7 @@ int radix_pass(spws_ctx* ctx, const Source& in, const Sink& out, int64_t n, int 
   const int64_t per = radix_chunk_tiles(ntiles), chunks = ntiles <= kSortDirect ? 0 : div_up(ntiles, per);
   SPWS_LAUNCH(ctx, "radix_hist", (k_radix_hist<K, Source>), dim3((unsigned)ntiles), dim3(kSortBlock), 0, in, n, shift,
               mask, hist);
-  if (chunks > 0)
-    SPWS_LAUNCH(ctx, "radix_chunks", k_radix_chunks, dim3((unsigned)chunks, (unsigned)div_up(nb, kSortBlock)),
-                dim3(kSortBlock), 0, hist, ntiles, per, nb, chunk);
-  if (chunks > 1)
-    SPWS_LAUNCH(ctx, "radix_digits", k_radix_digits, dim3((unsigned)div_up(nb, kWave)), dim3(kSortDigitsBlock), 0,
-                chunk, chunks, nb);
+  if (chunks > 0 && (rc = radix_offsets(ctx, hist, ntiles, nb, chunk))) return rc;
   SPWS_LAUNCH(ctx, "radix_scatter", (k_radix_scatter<K, Source, Sink>), dim3((unsigned)ntiles), dim3(kSortBlock), 0,
               in, out, n, shift, mask, nbits, (const int32_t*)hist, (const int32_t*)chunk, chunks, per);
   return SPWS_OK;
